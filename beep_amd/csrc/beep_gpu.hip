@@ -1797,37 +1797,55 @@ int beep_abcsmc_weights(int device, int nvar, int n_prev, const double* prev, co
     return BEEP_EINVAL;
   if (n_new == 0) return BEEP_OK;
   if (hipSetDevice(device) != hipSuccess) return BEEP_EHIP;
-  const size_t b_prev = (size_t)n_prev * nvar * 8, b_w = (size_t)n_prev * 8, b_th = (size_t)n_new * nvar * 8,
-               b_M = (size_t)nvar * nvar * 8, b_lp = (size_t)n_new * 8, b_out = (size_t)n_new * 8;
-  char* d = nullptr;
-  if (hipMalloc((void**)&d, b_prev + b_w + b_th + b_M + b_lp + b_out) != hipSuccess) return BEEP_ENOMEM;
-  double* d_prev = (double*)d;
-  double* d_w = (double*)(d + b_prev);
-  double* d_th = (double*)(d + b_prev + b_w);
-  double* d_M = (double*)(d + b_prev + b_w + b_th);
-  double* d_lp = (double*)(d + b_prev + b_w + b_th + b_M);
-  double* d_out = (double*)(d + b_prev + b_w + b_th + b_M + b_lp);
+  // One upload: the previous particles and the proposals in rows of NV, the
+  // weights, the triangle U of the quadratic form (k_abcsmc_partial), the
+  // log priors.
+  const int NV = (nvar + 1) / 2 * 2;
+  const size_t o_th = (size_t)n_prev * NV, o_w = o_th + (size_t)n_new * NV, o_U = o_w + n_prev,
+               o_lp = o_U + (size_t)8 * beepdev::abc_blocks(NV), n_in = o_lp + n_new;
+  std::vector<double> h(n_in, 0.0);
+  auto rows = [&](double* d, const double* src, int n) {
+    if (NV == nvar) std::copy(src, src + (size_t)n * nvar, d);
+    else
+      for (int i = 0; i < n; i++) std::copy(src + (size_t)i * nvar, src + (size_t)(i + 1) * nvar, d + (size_t)i * NV);
+  };
+  rows(h.data(), prev, n_prev);
+  rows(h.data() + o_th, theta, n_new);
+  std::copy(w_prev, w_prev + n_prev, h.begin() + o_w);
+  for (int v = 0, e = 0; v < NV; v++)
+    for (int x = v; x < NV; x++, e++)
+      if (x < nvar) h[o_U + e] =
+          (x == v ? inv_M[(size_t)v * nvar + v] : inv_M[(size_t)v * nvar + x] + inv_M[(size_t)x * nvar + v]) / size / size;
+  std::copy(logprior, logprior + n_new, h.begin() + o_lp);
+  // Splits of the previous generation: enough workgroups to fill the device,
+  // each of at least 16 previous particles.
+  const int nb = (n_new + BEEP_ABC_BLOCK - 1) / BEEP_ABC_BLOCK;
+  const int want = std::max(1, BEEP_ABC_WGS / nb);
+  const int jper = std::max(16, ((n_prev + want - 1) / want + BEEP_ABC_J - 1) / BEEP_ABC_J * BEEP_ABC_J);
+  const int nsplit = (n_prev + jper - 1) / jper;
+  double* d = nullptr;
+  if (hipMalloc((void**)&d, (n_in + (size_t)n_new * (nsplit + 1)) * 8) != hipSuccess) return BEEP_ENOMEM;
+  double* d_part = d + n_in;
+  double* d_out = d_part + (size_t)n_new * nsplit;
   int rc = BEEP_OK;
-  if (hipMemcpy(d_prev, prev, b_prev, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(d_w, w_prev, b_w, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(d_th, theta, b_th, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(d_M, inv_M, b_M, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(d_lp, logprior, b_lp, hipMemcpyHostToDevice) != hipSuccess)
-    rc = BEEP_EHIP;
+  if (hipMemcpy(d, h.data(), n_in * 8, hipMemcpyHostToDevice) != hipSuccess) rc = BEEP_EHIP;
   if (!rc) {
-    const size_t lds = 8 * ((size_t)nvar * nvar + (size_t)nvar * BEEP_ABC_BLOCK + (size_t)BEEP_ABC_TILE * nvar +
-                            BEEP_ABC_TILE);
-    if (lds > 65536 &&
-        hipFuncSetAttribute((const void*)beepdev::k_abcsmc_weights, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds) != hipSuccess)
+    using K = decltype(&beepdev::k_abcsmc_partial<2>);
+    static const K ks[16] = {
+        beepdev::k_abcsmc_partial<2>,  beepdev::k_abcsmc_partial<4>,  beepdev::k_abcsmc_partial<6>,
+        beepdev::k_abcsmc_partial<8>,  beepdev::k_abcsmc_partial<10>, beepdev::k_abcsmc_partial<12>,
+        beepdev::k_abcsmc_partial<14>, beepdev::k_abcsmc_partial<16>, beepdev::k_abcsmc_partial<18>,
+        beepdev::k_abcsmc_partial<20>, beepdev::k_abcsmc_partial<22>, beepdev::k_abcsmc_partial<24>,
+        beepdev::k_abcsmc_partial<26>, beepdev::k_abcsmc_partial<28>, beepdev::k_abcsmc_partial<30>,
+        beepdev::k_abcsmc_partial<32>};
+    hipLaunchKernelGGL(ks[NV / 2 - 1], dim3((unsigned)nb, (unsigned)nsplit), dim3(BEEP_ABC_BLOCK), 0, 0, n_prev, jper,
+                       (const double*)d, (const double*)(d + o_w), n_new, (const double*)(d + o_th),
+                       (const double*)(d + o_U), d_part);
+    hipLaunchKernelGGL(beepdev::k_abcsmc_finish, dim3((unsigned)nb), dim3(BEEP_ABC_BLOCK), 0, 0, n_new, nsplit,
+                       (const double*)d_part, (const double*)(d + o_lp), d_out);
+    if (hipGetLastError() != hipSuccess || hipMemcpy(w_out, d_out, (size_t)n_new * 8, hipMemcpyDeviceToHost) != hipSuccess)
       rc = BEEP_EHIP;
-    if (!rc) {
-      hipLaunchKernelGGL(beepdev::k_abcsmc_weights, dim3((n_new + BEEP_ABC_BLOCK - 1) / BEEP_ABC_BLOCK),
-                         dim3(BEEP_ABC_BLOCK), lds, 0, nvar, n_prev, d_prev, d_w, n_new, d_th, d_M, size, d_lp, d_out);
-      if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) rc = BEEP_EHIP;
-    }
   }
-  if (!rc && hipMemcpy(w_out, d_out, b_out, hipMemcpyDeviceToHost) != hipSuccess) rc = BEEP_EHIP;
   (void)hipFree(d);
   return rc;
 }

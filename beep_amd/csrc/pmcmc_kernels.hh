@@ -212,8 +212,11 @@ __global__ void k_particle_sample(int n, int nsec, const int* __restrict__ sec_t
 
 namespace beepdev {
 
-#define BEEP_ABC_BLOCK 128
-#define BEEP_ABC_TILE 64
+#define BEEP_ABC_BLOCK 256
+#define BEEP_ABC_J 2                // previous particles a thread works on at a time (4: 253 registers, two wavefronts per SIMD)
+#define BEEP_ABC_WGS 2048           // workgroups aimed at: eight per CU
+
+typedef const __attribute__((address_space(4))) double cdouble;
 
 // ABCSMC::calculate_particle_weight (src/abcsmc.cc:260-271) for n_new
 // proposals at once, FP64:
@@ -221,43 +224,115 @@ namespace beepdev {
 //   MVN::probability(a, b) = -0.5 sum_{v1} sum_{v2} ((a-b)_v1 / size) invM[v1][v2] ((a-b)_v2 / size)
 //                                                         (src/mvn.cc:185-195)
 //   out[i] = exp(logprior[i]) / den[i].
-// One thread per proposal; the previous generation passes through LDS in
-// tiles.  LDS: invM [nvar][nvar], this block's scaled differences e[v][t]
-// = (theta_i - prev_j)_v / size, and a tile of prev and w.
-__global__ void __launch_bounds__(BEEP_ABC_BLOCK) k_abcsmc_weights(int nvar, int n_prev, const double* __restrict__ prev,
-                                                                 const double* __restrict__ w, int n_new,
-                                                                 const double* __restrict__ theta,
-                                                                 const double* __restrict__ invM, double size,
-                                                                 const double* __restrict__ logprior,
-                                                                 double* __restrict__ out) {
-  extern __shared__ double sh[];
-  double* sM = sh;                                   // [nvar][nvar]
-  double* se = sM + nvar * nvar;                     // [nvar][BEEP_ABC_BLOCK]
-  double* sp = se + nvar * BEEP_ABC_BLOCK;           // [BEEP_ABC_TILE][nvar]
-  double* sw = sp + BEEP_ABC_TILE * nvar;            // [BEEP_ABC_TILE]
-  const int t = threadIdx.x;
-  const int i = blockIdx.x * BEEP_ABC_BLOCK + t;
-  for (int k = t; k < nvar * nvar; k += BEEP_ABC_BLOCK) sM[k] = invM[k];
-  double den = 0.0;
-  for (int j0 = 0; j0 < n_prev; j0 += BEEP_ABC_TILE) {
-    const int nj = min(BEEP_ABC_TILE, n_prev - j0);
-    __syncthreads();
-    for (int k = t; k < nj * nvar; k += BEEP_ABC_BLOCK) sp[k] = prev[(size_t)j0 * nvar + k];
-    for (int k = t; k < nj; k += BEEP_ABC_BLOCK) sw[k] = w[j0 + k];
-    __syncthreads();
-    if (i < n_new) {
-      for (int jj = 0; jj < nj; jj++) {
-        for (int v = 0; v < nvar; v++) se[v * BEEP_ABC_BLOCK + t] = (theta[(size_t)i * nvar + v] - sp[jj * nvar + v]) / size;
-        double sum = 0.0;
-        for (int v1 = 0; v1 < nvar; v1++) {
-          const double e1 = se[v1 * BEEP_ABC_BLOCK + t];
-          for (int v2 = 0; v2 < nvar; v2++) sum += e1 * sM[v1 * nvar + v2] * se[v2 * BEEP_ABC_BLOCK + t];
-        }
-        den += sw[jj] * exp(-0.5 * sum);
+// The quadratic form of any matrix is that of its upper triangle with the
+// mirrored entries added, so a pair costs NV (NV + 1) / 2 + NV FMAs: U holds
+// that triangle over size^2, row after row, NV being nvar rounded up to an
+// even number and the padding zero.  The differences
+// are formed per pair, so nothing cancels that did not before.
+//
+// Bound: FP64 FMA issue (253 + 22 per pair at 22 variables, plus the exp).  A
+// thread keeps its proposal and the differences of BEEP_ABC_J previous
+// particles in registers; U and the previous particles are the same for the
+// whole wavefront and come as scalar operands, each entry of U feeding
+// BEEP_ABC_J FMAs, so the loop has no LDS and no vector loads.  The previous
+// generation is split over workgroups (grid: blocks of proposals x splits of
+// jper previous particles), one partial sum per (split, proposal).
+// 4096 x 4096 x 22: 0.20 ms, 5.0 G FMAs at 0.69 of the FP64 product rate; one
+// thread per proposal with the matrix and the differences in LDS, on 32
+// workgroups, took 92 ms.
+// Blocks of eight entries of the triangle of NV variables (at least two).
+__host__ __device__ constexpr int abc_blocks(int NV) {
+  const int n = (NV * (NV + 1) / 2 + 7) / 8;
+  return n < 2 ? 2 : n;
+}
+
+// Rows V and up of the triangle (compile-time recursion over rows, the row
+// unrolled: every index below is a constant): q = the form so far, for J pairs.
+template <int NV, int J, int V>
+__device__ inline __attribute__((always_inline)) void abc_rows(cdouble*& Up, double (&u)[3][8], const double (&d)[J][NV],
+                                                               double (&q)[J]) {
+  if constexpr (V < NV) {
+    constexpr int E0 = V * NV - V * (V - 1) / 2;       // the row's first entry
+    double a[J];
+#pragma unroll
+    for (int k = 0; k < J; k++) a[k] = 0.0;
+#pragma unroll
+    for (int x = V; x < NV; x++) {
+      const int E = E0 + x - V, c = E / 8;
+      if (E % 8 == 0 && c + 2 < abc_blocks(NV)) {
+        if (c > 0) asm volatile("" : "+s"(Up), "+v"(a[0]));
+#pragma unroll
+        for (int e = 0; e < 8; e++) u[(c + 2) % 3][e] = Up[(c + 2) * 8 + e];
       }
+#pragma unroll
+      for (int k = 0; k < J; k++)
+        a[k] = x == V ? u[c % 3][E % 8] * d[k][x] : __builtin_fma(u[c % 3][E % 8], d[k][x], a[k]);
     }
+#pragma unroll
+    for (int k = 0; k < J; k++) q[k] = __builtin_fma(a[k], d[k][V], q[k]);
+    abc_rows<NV, J, V + 1>(Up, u, d, q);
   }
-  if (i < n_new) out[i] = exp(logprior[i]) / den;
+}
+
+template <int NV>
+__global__ void __launch_bounds__(BEEP_ABC_BLOCK, 2)
+    k_abcsmc_partial(int n_prev, int jper, const double* prev_, const double* w_, int n_new,
+                     const double* __restrict__ theta, const double* U_, double* __restrict__ partial) {
+  constexpr int J = BEEP_ABC_J;
+  cdouble* prev = (cdouble*)prev_;
+  cdouble* w = (cdouble*)w_;
+  cdouble* U = (cdouble*)U_;
+  const int i = blockIdx.x * BEEP_ABC_BLOCK + threadIdx.x;
+  const int ic = min(i, n_new - 1);
+  double th[NV];
+#pragma unroll
+  for (int v = 0; v < NV; v++) th[v] = theta[(size_t)ic * NV + v];
+  const int j0 = blockIdx.y * jper, j1 = min(n_prev, j0 + jper);
+  double den = 0.0;
+  for (int j = j0; j < j1; j += J) {
+    double d[J][NV], q[J];
+#pragma unroll
+    for (int k = 0; k < J; k++) {
+      cdouble* pj = prev + (size_t)min(j + k, n_prev - 1) * NV;
+      if (k > 0) asm volatile("" : "+s"(pj), "+v"(d[k - 1][NV - 1]));
+      q[k] = 0.0;
+#pragma unroll
+      for (int v = 0; v < NV; v++) d[k][v] = th[v] - pj[v];
+    }
+    // The triangle in order, eight entries (one 64-byte scalar load) at a
+    // time, two loads ahead.  The empty asm ties each load's address to a
+    // value of the block before: hoisted to the top or out of the loop, the
+    // loads would spill the whole triangle.
+    cdouble* Up = U;
+    asm volatile("" : "+s"(Up), "+v"(d[J - 1][NV - 1]));
+    double u[3][8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) u[0][e] = Up[e];
+#pragma unroll
+    for (int e = 0; e < 8; e++) u[1][e] = Up[8 + e];
+    abc_rows<NV, J, 0>(Up, u, d, q);
+    // All J forms are done here: sunk into the conditions below, the FMAs of
+    // the later pairs would keep the whole triangle alive.
+#pragma unroll
+    for (int k = 0; k < J; k++) asm volatile("" : "+v"(q[k]));
+#pragma unroll
+    for (int k = 0; k < J; k++)
+      if (j + k < j1) den += w[j + k] * exp(-0.5 * q[k]);
+  }
+  if (i < n_new) partial[(size_t)blockIdx.y * n_new + i] = den;
+}
+
+// The splits' sums in order, and the weight.
+__global__ void __launch_bounds__(BEEP_ABC_BLOCK) k_abcsmc_finish(int n_new, int nsplit,
+                                                                const double* __restrict__ partial,
+                                                                const double* __restrict__ logprior,
+                                                                double* __restrict__ out) {
+  const int i = blockIdx.x * BEEP_ABC_BLOCK + threadIdx.x;
+  if (i >= n_new) return;
+  double den = 0.0;
+#pragma unroll 8
+  for (int s = 0; s < nsplit; s++) den += partial[(size_t)s * n_new + i];
+  out[i] = exp(logprior[i]) / den;
 }
 
 // MC3::swap_states (src/mc3.cc:153-215) for the chains of one launch, each
