@@ -164,50 +164,81 @@ __device__ inline float log_pois_f(float k, float lam) {
   return -0.5f * __logf(6.2831853071795865f * k) - stirlerr_f(k) - bd0_f(k, lam);
 }
 
-// Four terms k0+1 .. k0+4 of the inversion search with 1/k as constants:
-// p_k = p_{k-1} * lam / k, F_k = F_{k-1} + p_k; r = the first k whose F_k
-// reaches u (or stops growing), 0 if none.
-#define BEEP_INV_BLOCK(K0)                                                              \
-  {                                                                                     \
-    float p1 = p * (lam * (1.0f / (K0 + 1))), F1 = F + p1;                             \
-    float p2 = p1 * (lam * (1.0f / (K0 + 2))), F2 = F1 + p2;                           \
-    float p3 = p2 * (lam * (1.0f / (K0 + 3))), F3 = F2 + p3;                           \
-    float p4 = p3 * (lam * (1.0f / (K0 + 4))), F4 = F3 + p4;                           \
-    int r = (u <= F4 || F4 == F3) ? K0 + 4 : 0;                                         \
-    r = (u <= F3 || F3 == F2) ? K0 + 3 : r;                                             \
-    r = (u <= F2 || F2 == F1) ? K0 + 2 : r;                                             \
-    r = (u <= F1 || F1 == F) ? K0 + 1 : r;                                              \
-    if (r) return r;                                                                    \
-    p = p4;                                                                             \
-    F = F4;                                                                             \
-  }
+// Whether any active lane of the wavefront holds c.
+__device__ inline bool wave_any(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
 
-// Poisson(lam) with first uniform u (FP32 path for small means): sequential
-// inversion, the CDF summed until it passes u.  When FP32 rounding leaves u
-// above the largest representable CDF value, the search stops where further
-// terms no longer change the sum (a tail event of probability ~1e-7).  The
-// first 16 terms are evaluated four at a time with constant reciprocals (one
-// branch per four terms, which matters where the lanes of a wavefront need
-// different numbers of terms); later terms, rare below mean 10, one at a time.
-__device__ inline int poisson_inversion(float lam, float u) {
-  float p = __expf(-lam);
-  if (u <= p) return 0;
+// Where the running sum of the inversion search first stops growing (or 64):
+// the search's result when FP32 rounding leaves u above that sum, a tail event
+// of probability ~1e-7, hence one compact loop.  1 / k up to 16 is the
+// correctly rounded reciprocal: a Newton step from any value within one ulp
+// of 1 / k gives it for these k.
+__device__ inline int poisson_stall(float lam, float p) {
   float F = p;
-  BEEP_INV_BLOCK(0)
-  BEEP_INV_BLOCK(4)
-  BEEP_INV_BLOCK(8)
-  BEEP_INV_BLOCK(12)
-  int k = 16;
+  int k = 0;
+#pragma unroll 1
   while (k < 64) {
     k++;
-    p *= lam * __builtin_amdgcn_rcpf((float)k);
-    float Fn = F + p;
-    if (u <= Fn || Fn == F) return k;
+    float r = __builtin_amdgcn_rcpf((float)k);
+    if (k <= 16) r = __builtin_fmaf(__builtin_fmaf(-(float)k, r, 1.f), r, r);
+    const float l = lam * r, Fn = __builtin_fmaf(l, p, F);
+    p *= l;
+    if (Fn == F) return k;
     F = Fn;
   }
   return k;
 }
+
+// One term of the search: F_k = F_{k-1} + p_k with p_k = p_{k-1} lam / k.
+#define BEEP_INV_TERM(K)                           \
+  {                                                \
+    const float l = lam * (1.0f / (K));            \
+    F = __builtin_fmaf(l, p, F);                   \
+    p = l * p;                                     \
+    k += u > F;                                    \
+  }
+#define BEEP_INV_BLOCK(K0) BEEP_INV_TERM(K0 + 1) BEEP_INV_TERM(K0 + 2) BEEP_INV_TERM(K0 + 3) BEEP_INV_TERM(K0 + 4)
+
+// Poisson(lam) with first uniform u (FP32, lam < 10): sequential inversion,
+// the first k at which the CDF F_k reaches u or stops growing.
+//
+// The F_k of a lane never fall, so k is the number of them below u: a compare
+// and an add with carry per term, with no lane masked off, and the wavefront
+// goes on, four terms at a time, while any lane's u is above its sum (a lane
+// that is done counts nothing more).  Below mean 10 a sum that has stopped
+// growing never grows again, so u at or below the last sum was reached before
+// any stop; a lane still above its sum at the end has stopped
+// (poisson_stall).  Terms 1-16 have their reciprocals as constants.
+// The search with its first-of-four selection and masked exits cost 32
+// instructions per block of four terms and lane-mask work between blocks, this
+// one 20: spatial simulation of 4096 x 400 cells x 200 steps 15.8 -> 14.35 ms.
+__device__ inline int poisson_inversion(float lam, float u) {
+  const float p0 = __expf(-lam);
+  float p = p0, F = p0;
+  int k = u > F;
+  if (!wave_any(u > F)) return k;
+  BEEP_INV_BLOCK(0)
+  if (wave_any(u > F)) {
+    BEEP_INV_BLOCK(4)
+    if (wave_any(u > F)) {
+      BEEP_INV_BLOCK(8)
+      if (wave_any(u > F)) {
+        BEEP_INV_BLOCK(12)
+        float Fp = -1.f;
+        for (int t = 17; t <= 64 && wave_any(u > F && F != Fp); t++) {
+          const float l = lam * __builtin_amdgcn_rcpf((float)t);
+          Fp = F;
+          F = __builtin_fmaf(l, p, F);
+          p *= l;
+          k += u > F;
+        }
+        if (u > F) k = poisson_stall(lam, p0);
+      }
+    }
+  }
+  return k;
+}
 #undef BEEP_INV_BLOCK
+#undef BEEP_INV_TERM
 
 // PTRS (Hormann 1993) for 10 <= lam < 2^23: the squeeze accepts most
 // candidates; the exact test compares with the saddle-point log-pmf.
