@@ -109,11 +109,11 @@ struct beep_ctx {
   // structure-specialised fused kernel (null: generic kernel or step-wise path)
   SpecKernels* spec = nullptr;
   size_t spec_lds = 0;
-  // Streams over which a mixed batch launched from this context spreads its
-  // size classes (created on first use), and the event they start from.
-  hipStream_t bstream[4] = {};
+  // The events a mixed batch launched from this context starts the device's
+  // batch streams from and joins them with (created on first use).
   hipEvent_t bstart = nullptr;
-  hipEvent_t bend[4] = {};         // end of each batch stream's work
+  std::vector<hipEvent_t> bend;    // end of each batch stream's work
+  bool counted = false;            // holds a share of the device's batch streams
   bool obs_general = false;        // observations other than plain normal ones
   bool obs_pop = false;            // observations counting population elements
   // Observation splines: their values per slot, [nslot][nospl][S] (FP64), and
@@ -142,6 +142,25 @@ static __device__ __align__(256) unsigned char scratch[BEEP_NOALLOC_BYTES];
 namespace {
 
 constexpr int kMaxDevices = 64;
+
+// Streams over which mixed batches spread their size classes, one set per
+// device, made by the first batch and destroyed with the device's last
+// context.  A launch of a batch is rarely wide enough to fill the device and
+// lasts as long as its longest instance, so what counts is how many launches
+// run at once: ordinary streams share a handful of hardware queues, whose
+// launches run one after the other, while a stream made with a compute-unit
+// mask (here of every unit) has a queue of its own (16 launches of 16
+// workgroups each: 22.8 ms on 16 ordinary streams, 5.7 ms on 16 masked ones,
+// 6.1 ms for one launch).  Batches of several host threads share the streams:
+// each joins on events of its own.
+constexpr int kBatchStreams = 12;
+struct BatchStreams {
+  std::vector<hipStream_t> st;
+  int users = 0;                   // contexts of the device
+};
+std::mutex g_bstream_mu;
+BatchStreams g_bstream[kMaxDevices];
+
 std::mutex g_noalloc_mu;
 void* g_noalloc_ptr[kMaxDevices] = {};
 
@@ -674,6 +693,11 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
   HIPCHK(c, hipSetDevice(device));
   int rc0 = noalloc_setup(c);
   if (rc0) return rc0;
+  {
+    std::lock_guard<std::mutex> lk(g_bstream_mu);
+    g_bstream[device].users++;
+    c->counted = true;
+  }
   HIPCHK(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   for (auto& e : c->ev) HIPCHK(c, hipEventCreate(&e));
   const auto& m = c->m;
@@ -939,11 +963,17 @@ int beep_destroy(beep_ctx* c) {
   for (auto& e : c->ev)
     if (e) (void)hipEventDestroy(e);
   for (auto& g : c->graphs) (void)hipGraphExecDestroy(g.exec);
-  for (auto& st : c->bstream)
-    if (st) {
-      (void)hipStreamSynchronize(st);
-      (void)hipStreamDestroy(st);
+  if (c->counted) {
+    std::lock_guard<std::mutex> lk(g_bstream_mu);
+    BatchStreams& b = g_bstream[c->device];
+    if (--b.users == 0) {
+      for (auto& st : b.st) {
+        (void)hipStreamSynchronize(st);
+        (void)hipStreamDestroy(st);
+      }
+      b.st.clear();
     }
+  }
   if (c->bstart) (void)hipEventDestroy(c->bstart);
   for (auto& e : c->bend)
     if (e) (void)hipEventDestroy(e);
@@ -1965,12 +1995,34 @@ int pow2_ceil(int x) {
   return p;
 }
 
-// The streams a batch launched from c0 spreads its work over (made once).
-int ensure_bstreams(beep_ctx* c0) {
-  if (c0->bstart) return BEEP_OK;
-  HIPCHK(c0, hipEventCreateWithFlags(&c0->bstart, hipEventDisableTiming));
-  for (auto& e : c0->bend) HIPCHK(c0, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  for (auto& st : c0->bstream) HIPCHK(c0, hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+// The device's batch streams (made by the first batch) and c0's events.
+int ensure_bstreams(beep_ctx* c0, std::vector<hipStream_t>& out) {
+  {
+    std::lock_guard<std::mutex> lk(g_bstream_mu);
+    BatchStreams& b = g_bstream[c0->device];
+    if (b.st.empty()) {
+      hipDeviceProp_t prop;
+      HIPCHK(c0, hipGetDeviceProperties(&prop, c0->device));
+      const int ncu = prop.multiProcessorCount;
+      std::vector<uint32_t> mask((ncu + 31) / 32, 0u);
+      for (int i = 0; i < ncu; i++) mask[i / 32] |= 1u << (i % 32);
+      for (int k = 0; k < kBatchStreams; k++) {
+        hipStream_t st = nullptr;
+        if (hipExtStreamCreateWithCUMask(&st, (uint32_t)mask.size(), mask.data()) != hipSuccess) {
+          (void)hipGetLastError();
+          HIPCHK(c0, hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+        }
+        b.st.push_back(st);
+      }
+    }
+    out = b.st;
+  }
+  if (!c0->bstart) HIPCHK(c0, hipEventCreateWithFlags(&c0->bstart, hipEventDisableTiming));
+  while (c0->bend.size() < out.size()) {
+    hipEvent_t e = nullptr;
+    HIPCHK(c0, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    c0->bend.push_back(e);
+  }
   return BEEP_OK;
 }
 
@@ -2239,9 +2291,9 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
       launches.emplace_back(kv.first.first, all.size(), v.size(), lds, maxAG, kv.first.second, rerunnable, lead);
       for (auto& it : v) all.push_back(it.job);
     }
-    // Launches in order of their longest job, longest first, dealt round-robin
-    // over the batch streams: the classes whose workgroups run longest start
-    // first, and the short ones fill the device as those drain.
+    // Launches in order of their longest job, longest first, each to the batch
+    // stream with the least work so far (a launch lasting about as long as its
+    // longest job).
     std::stable_sort(launches.begin(), launches.end(),
                      [](const auto& a, const auto& b) { return std::get<7>(a) > std::get<7>(b); });
     if (all.size() > c0->bjobs_cap) {
@@ -2262,14 +2314,15 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
     // instances of one launch overlap the next launch instead of leaving the
     // device idle; each stream starts after the job upload.  (Autotuning
     // launches run alone on the context stream to be timed.)
-    const int nbs = (int)(sizeof c0->bstream / sizeof c0->bstream[0]);
-    if ((rc = ensure_bstreams(c0))) return rc;
+    std::vector<hipStream_t> bst;
+    if ((rc = ensure_bstreams(c0, bst))) return rc;
+    const int nbs = (int)std::min(bst.size(), launches.size());
+    std::vector<double> load(nbs, 0.0);
     // The fused phase is timed on the context stream from before the batch
     // streams start to after they have all ended (timing[0]).
     record(c0, 0);
     HIPCHK(c0, hipEventRecord(c0->bstart, c0->stream));
-    for (auto& st : c0->bstream) HIPCHK(c0, hipStreamWaitEvent(st, c0->bstart, 0));
-    int next_stream = 0;
+    for (int k = 0; k < nbs; k++) HIPCHK(c0, hipStreamWaitEvent(bst[k], c0->bstart, 0));
     std::lock_guard<std::mutex> lk(g_tune_mu);
     tune_load();
     bool tuned_any = false;
@@ -2325,7 +2378,12 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
       }
       // An autotuning call keeps every launch on the context stream, so that
       // the timed candidates run alone.
-      hipStream_t st = (flags & BEEP_BATCH_AUTOTUNE) ? nullptr : c0->bstream[next_stream++ % nbs];
+      hipStream_t st = nullptr;
+      if (!(flags & BEEP_BATCH_AUTOTUNE)) {
+        const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+        load[k] += std::get<7>(L);
+        st = bst[k];
+      }
       if ((rc = launch_any(block, st))) return rc;
       nlaunch++;
     }
@@ -2333,7 +2391,7 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
     // Join: the context stream waits for every batch stream, then records the
     // end of the fused phase.
     for (int k = 0; k < nbs; k++) {
-      HIPCHK(c0, hipEventRecord(c0->bend[k], c0->bstream[k]));
+      HIPCHK(c0, hipEventRecord(c0->bend[k], bst[k]));
       HIPCHK(c0, hipStreamWaitEvent(c0->stream, c0->bend[k], 0));
     }
     record(c0, 1);
