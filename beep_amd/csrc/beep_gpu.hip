@@ -39,7 +39,7 @@ using beepdev::TopoDev;
 // of the process.
 struct SpecKernels {
   hipModule_t mod = nullptr;
-  hipFunction_t fn[4] = {};        // fused kernel, indexed by MODE_SIM / MBP / REPLAY / ANY
+  hipFunction_t fn[3] = {};        // fused kernel, indexed by MODE_SIM / MBP / REPLAY
   hipFunction_t step[3] = {};      // step-wise transition kernel, MODE_SIM / MBP / REPLAY
   int max_dyn_lds = 65536;         // dynamic LDS the fused kernels accept (the device's, less static use)
 };
@@ -403,8 +403,8 @@ int spec_kernels(beep_ctx* c, SpecKernels** out) {
   hiprtcDestroyProgram(&prog);
   auto* k = new SpecKernels();
   hipError_t e = hipModuleLoadData(&k->mod, code.data());
-  const char* fn[4] = {"beep_fused_spec_sim", "beep_fused_spec_mbp", "beep_fused_spec_replay", "beep_fused_spec_any"};
-  for (int i = 0; e == hipSuccess && i < 4; i++) e = hipModuleGetFunction(&k->fn[i], k->mod, fn[i]);
+  const char* fn[3] = {"beep_fused_spec_sim", "beep_fused_spec_mbp", "beep_fused_spec_replay"};
+  for (int i = 0; e == hipSuccess && i < 3; i++) e = hipModuleGetFunction(&k->fn[i], k->mod, fn[i]);
   const char* sn[3] = {"beep_step_spec_sim", "beep_step_spec_mbp", "beep_step_spec_replay"};
   for (int i = 0; e == hipSuccess && i < 3; i++) e = hipModuleGetFunction(&k->step[i], k->mod, sn[i]);
   if (e != hipSuccess) {
@@ -412,7 +412,7 @@ int spec_kernels(beep_ctx* c, SpecKernels** out) {
     return fail(c, BEEP_EHIP, "loading the specialised kernel: %s", hipGetErrorString(e));
   }
   int lim = 0;
-  for (int i = 0; i < 4; i++) {
+  for (int i = 0; i < 3; i++) {
     int v = 0;
     if (hipFuncGetAttribute(&v, HIP_FUNC_ATTRIBUTE_MAX_DYNAMIC_SHARED_SIZE_BYTES, k->fn[i]) == hipSuccess && v > 0)
       lim = i == 0 ? v : std::min(lim, v);
@@ -538,7 +538,6 @@ int launch_fused(beep_ctx* c, int mode, const Job* djobs, int njobs, uint64_t se
   size_t lds = beepdev::fused_lds_bytes(m.A, m.G, m.C, m.T, c->h_topo.nnz, c->h_topo.stage_mix);
   if (lds > 160 * 1024) return fail(c, BEEP_EINVAL, "instance needs %zu bytes of LDS (max 163840)", lds);
   int block = fused_block(m.AG);
-  if (mode == beepdev::MODE_ANY) return launch_fused_t<beepdev::MODE_ANY>(c, djobs, njobs, lds, block, seed, stream);
   if (mode == beepdev::MODE_SIM) return launch_fused_t<beepdev::MODE_SIM>(c, djobs, njobs, lds, block, seed, stream);
   if (mode == beepdev::MODE_MBP) return launch_fused_t<beepdev::MODE_MBP>(c, djobs, njobs, lds, block, seed, stream);
   return launch_fused_t<beepdev::MODE_REPLAY>(c, djobs, njobs, lds, block, seed, stream);
@@ -772,13 +771,17 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
   }
   tp.off_af = -1;
   tp.af = nullptr;
+  tp.af_static = 0;
   if (m.af_param) {
     tp.off_af = off;
     off += m.period * m.A;
   } else {
     float* d_af = nullptr;
-    if ((rc = upload(c, &d_af, to_f32(m.af_const)))) return rc;
+    const std::vector<float> af = to_f32(m.af_const);
+    if ((rc = upload(c, &d_af, af))) return rc;
     tp.af = d_af;
+    tp.af_static = 1;
+    for (size_t k = m.A; k < af.size() && tp.af_static; k++) tp.af_static = af[k] == af[k - m.A];
   }
   c->slot_stride = ((size_t)off + 63) / 64 * 64;
   tp.from = d_from; tp.to = d_to; tp.diag = d_diag; tp.fac = d_fac;

@@ -32,6 +32,7 @@ struct TopoDev {
   // on the parameters (off_af >= 0), else this context-wide table.
   const float* af;
   int off_af;
+  int af_static;         // 1: the area factor's rows are all the same
   const float* agedist;  // [nE][G] age weights of the external force of each group (efoi[S][nE] per slot)
   // Prediction-mode modifications, null when absent: multipliers of beta and
   // of the external force per step and cell, [S][AG], and of every transition
@@ -62,10 +63,10 @@ struct Job {
   uint32_t key;
   int t0, t1;
   int from_init;              // 1: start from topo->pop_init
-  int mode;                   // MODE_SIM / MODE_MBP / MODE_REPLAY (read by MODE_ANY launches)
+  int mode;                   // MODE_SIM / MODE_MBP / MODE_REPLAY
 };
 
-enum { MODE_SIM = 0, MODE_MBP = 1, MODE_REPLAY = 2, MODE_ANY = 3 };
+enum { MODE_SIM = 0, MODE_MBP = 1, MODE_REPLAY = 2 };
 
 // Trajectory outputs are written once and read by later kernels: global
 // address space, non-temporal (streaming) stores.
@@ -76,6 +77,16 @@ typedef __attribute__((address_space(1))) float gfloat;
 // 32-bit per-lane offset, with no 64-bit address arithmetic per lane.
 __device__ inline void st_nt(int* p, uint32_t i, int v) { __builtin_nontemporal_store(v, (gint*)p + i); }
 __device__ inline void st_nt(float* p, uint32_t i, float v) { __builtin_nontemporal_store(v, (gfloat*)p + i); }
+
+// One step's slab of an instance's trajectory as a buffer: a store's address is
+// the slab's base, a scalar offset (the row of a transition or compartment)
+// and the lane's byte offset, and the hardware drops a store whose lane offset
+// lies past the slab, so a lane opts out without a branch.
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ inline rsrc_t slab(void* p, uint32_t bytes) { return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00020000); }
+__device__ inline void st_slab(rsrc_t r, int v, uint32_t lane_off, uint32_t row_off) {
+  __builtin_amdgcn_raw_buffer_store_b32(v, r, (int)lane_off, (int)row_off, 2);       // 2: non-temporal
+}
 
 // Pointers typed by address space.  A plain pointer read out of a job
 // descriptor is generic, and a generic (flat) load counts against both the
@@ -232,6 +243,16 @@ __device__ inline __attribute__((always_inline)) int draw_item_body(int kind, fl
 __device__ inline int draw_item(int kind, float val, int ni, uint32_t k0, uint32_t k1, uint32_t c0, uint32_t cell,
                                 uint32_t tr, uint32_t key) {
   return draw_item_body(kind, val, ni, k0, k1, c0, cell, tr, key);
+}
+// The same for the simulation kernels, whose queued draws are all Poisson of
+// mean BEEP_POIS_INLINE and above.
+__device__ inline __attribute__((always_inline)) int draw_large_poisson(float lam, uint32_t k0, uint32_t k1, uint32_t c0,
+                                                                        uint32_t cell, uint32_t tr, uint32_t key) {
+  ExtraUniforms xr;
+  xr.init(k0, k1, c0, cell, key);
+  xr.block = 0x80000000u | (tr << 22);
+  const float u = xr.next();
+  return lam < BEEP_SPLIT ? poisson_ptrs(lam, u, xr) : poisson_draw(lam, u, xr);
 }
 __device__ inline __attribute__((always_inline)) int draw_item_inline(int kind, float val, int ni, uint32_t k0,
                                                                       uint32_t k1, uint32_t c0, uint32_t cell,

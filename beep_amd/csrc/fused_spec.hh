@@ -19,8 +19,26 @@
 // four compartments so one cell's compartments load and store as vectors.
 //
 // Per step: (B) area mixing, (C) means, small draws, updates of the cell's own
-// populations, large draws queued, (D) the queued draws by all lanes, applied
-// with LDS atomics, (E) the infectivity of each cell for the next step.
+// populations and its infectivity for the next step, large draws queued; where
+// some draw was queued, (D) the queued draws by all lanes, applied with LDS
+// atomics, (E) the infectivities again.
+//
+// Few instances leave a compute unit with one or two wavefronts per SIMD, and
+// a step is then a serial chain of latencies.  What keeps it short:
+//  - loads and stores share one counter, so a load issued after a step's
+//    trajectory stores waits for them too.  The step's scalars (beta, external
+//    force, m) are held 64 steps to a register, one lane each; the area factor
+//    is staged once when it does not vary; a cell's means are all formed before
+//    its first store;
+//  - a taken branch refetches instructions: stores go through slabs whose range
+//    check drops a lane's store (st_slab), a cell's queued draws take one LDS
+//    atomic together, errors are tested once per cell;
+//  - steps that queue nothing have neither (D) nor (E): two barriers.
+// Replaced: a branch per transition for each null check, error check, queue
+// push and masked store, and four global loads per step behind the stores
+// (92 branches per step of a single-cell instance, half of a wavefront's time in
+// waits).  Proposals of 256 x 400 cells x 200 steps: 2.87 -> 1.96 ms; one
+// single-cell instance, 100 steps: 0.395 -> 0.32 ms.
 #pragma once
 
 namespace beepdev {
@@ -31,6 +49,29 @@ static_assert(beepspec::CP % 4 == 0 && beepspec::CP >= beepspec::C, "CP");
 // cell; chunk k of all cells is contiguous, so one wavefront's 16-byte
 // accesses to its cells' chunk are consecutive in LDS.
 __device__ inline int pidx(int c, int cell, int AG) { return ((c >> 2) * AG + cell) * 4 + (c & 3); }
+
+// Infectivity of a cell, dinf = sum_c inf_c * pop_c (State::set_I_from_pop),
+// from its populations in registers or in LDS.
+__device__ inline float infectivity(const int (&p)[beepspec::CP], const float* sinf) {
+  float d = 0.f;
+#pragma unroll
+  for (int c = 0; c < beepspec::C; c++)
+    if (beepspec::INFC[c]) {
+      const float w = sinf[c];
+      if (w != 0.f) d += w * (float)p[c];
+    }
+  return d;
+}
+__device__ inline float cell_infectivity(const int* pop, int cell, int AG, const float* sinf) {
+  const int4* pv = (const int4*)pop;
+  int p[beepspec::CP];
+#pragma unroll
+  for (int c4 = 0; c4 < beepspec::CP / 4; c4++) {
+    const int4 v = pv[c4 * AG + cell];
+    p[4 * c4] = v.x; p[4 * c4 + 1] = v.y; p[4 * c4 + 2] = v.z; p[4 * c4 + 3] = v.w;
+  }
+  return infectivity(p, sinf);
+}
 
 // Strains: for each strain-0 cell, the susceptibles of its dp summed over
 // the strains (reads pop only; the caller's barrier publishes spool).
@@ -53,7 +94,7 @@ template <int MODE>
 __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t seed, uint32_t stream) {
   using namespace beepspec;
   const Job jb = jobs[blockIdx.x];
-  const int mode = MODE == MODE_ANY ? jb.mode : MODE;
+  constexpr int mode = MODE;
   ctopo* __restrict__ tpp = (ctopo*)jb.topo;
   const int A = tpp->A, S = tpp->S, AG = tpp->AG;
   const int nt = blockDim.x, tid = threadIdx.x;
@@ -125,40 +166,45 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
       for (int i = tid; i < NSTRAIN * A; i += nt) segrp[i] = tpp->nE > 1 ? gptr(tpp->egrp)[i] : 0;
     if (tid == 0) qcount[0] = 0;
   }
+  const bool af_static = tpp->af_static != 0;
+  if (af_static) {
+    gcfloat* af0 = af_row(tpp, tab, 0);
+    for (int i = tid; i < A; i += nt) saf[i] = af0[i];
+  }
   __syncthreads();
 
-  // (E) for the first step: dinf = sum_c inf_c * pop_c (State::set_I_from_pop).
-  for (int cell = tid; cell < AG; cell += nt) {
-    const int4* pv = (const int4*)pop;
-    float d = 0.f;
-#pragma unroll
-    for (int c4 = 0; c4 < CP / 4; c4++) {
-      int4 v = pv[c4 * AG + cell];
-      int pc[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const int c = 4 * c4 + k;
-        if (c < C && INFC[c]) {
-          float w = sinf[c];
-          if (w != 0.f) d += w * (float)pc[k];
-        }
-      }
-    }
-    sdinf[cell] = d;
-  }
+  // (E) for the first step.
+  for (int cell = tid; cell < AG; cell += nt) sdinf[cell] = cell_infectivity(pop, cell, AG, sinf);
   pool_susceptibles(pop, spool, AG, tid, nt);
   __syncthreads();
 
   const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
-  const size_t TAG = (size_t)T * AG, CAG = (size_t)C * AG;
+  const uint32_t TAG = (uint32_t)(T * AG), CAG = (uint32_t)(C * AG);
 
-  for (int s = jb.t0; s < jb.t1; s++) {
-    const float beta_s = tab[tpp->off_beta + s];
-    gcfloat* af_s = af_row(tpp, tab, s);
-    const float efoi_s = tab[tpp->off_efoi + s];
-    // Read in (C) after the barrier that ends (B); step s-1's reads ended at
-    // the barriers of (C), (D) and (E).
-    for (int i = tid; i < A; i += nt) saf[i] = af_s[i];
+  const int lane64 = tid & 63;
+  float vbeta = 0.f, vefoi = 0.f, vgeo = 0.f;          // this lane's step of the current 64
+  gcfloat* tbeta = tab + tpp->off_beta;
+  gcfloat* tefoi = tab + tpp->off_efoi;
+  gcfloat* tgeo = tab + tpp->off_geo;
+  const int t0 = jb.t0, spd = tpp->spd;
+
+  for (int s = t0; s < jb.t1; s++) {
+    const int s64 = (s - t0) & 63;
+    if (s64 == 0) {
+      const int sl = min(s + lane64, S - 1);
+      vbeta = tbeta[sl];
+      vefoi = tefoi[sl];
+      vgeo = tgeo[sl];
+    }
+    auto of_step = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), s64)); };
+    const float beta_s = of_step(vbeta), efoi_s = of_step(vefoi), m = of_step(vgeo);
+    // The area factor's row where it varies: loaded here, written to LDS after
+    // the mixing.  Read in (C) after the barrier that ends (B); step s-1's
+    // reads ended at the barrier of (C).
+    gcfloat* af_s = af_static ? nullptr : af_row(tpp, tab, s);
+    const bool newrow = !af_static && (s == t0 || s % spd == 0);
+    float afr = 0.f;
+    if (newrow && tid < A) afr = af_s[tid];
     if (grouped) {
       const int nR = tpp->nR;
       for (int i = tid; i < A; i += nt) sbeta[i] = tab[tpp->off_beta + (size_t)s * nR + (nR > 1 ? gptr(tpp->rgrp)[i] : 0)];
@@ -169,15 +215,6 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
     if (tpp->N_tv) {
       for (int i = tid; i < G * G; i += nt) sN[i] = tab[tpp->off_N + (size_t)s * G * G + i];
     }
-    // (B) area mixing, from LDS when the CSR is staged there.
-    const float m = tab[tpp->off_geo + s];
-    if (staged)
-      mix_cells((lcfloat*)sdiag, (lcfloat*)sfac, (lcint*)sptr, (lcint*)ssrc, (lcfloat*)sw, (lcint*)sord, sdinf, sI, m,
-                G, AG, tid, nt);
-    else
-      mix_cells(diag, fac, in_ptr, in_src, in_w, order, sdinf, sI, m, G, AG, tid, nt);
-    __syncthreads();
-    // (C) means, small draws, own-cell updates; large draws queued.
     int* tn_s = jb.tn ? jb.tn + (size_t)s * TAG : nullptr;
     float* tm_s = jb.tm ? jb.tm + (size_t)s * TAG : nullptr;
     int* pt_s = jb.pt ? jb.pt + (size_t)s * CAG : nullptr;
@@ -185,26 +222,44 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
     gcfloat* itm = mode == MODE_MBP ? gptr(jb.init_tm) + (size_t)s * TAG : nullptr;
     gcint* tn_r = mode == MODE_REPLAY ? gptr(jb.tn) + (size_t)s * TAG : nullptr;
     gcbyte* simu_s = mode == MODE_MBP && jb.simu ? gptr(jb.simu) + (size_t)s * A : nullptr;
-    const bool update = s < S - 1;           // the last step is not applied (src/state.cc:634)
-    const uint32_t c0 = (uint32_t)s | (stream << 16);
-    for (int cell = tid; cell < AG; cell += nt) {
-      const int j = cell / G, g = cell - j * G;
-      // The cell's global reads are issued before its first store: a load
-      // issued after a store waits for that store too.
-      const bool simu = mode == MODE_MBP ? (simu_s ? simu_s[j] != 0 : false) : true;
-      int nrep[T], nini[T];
-      float lini[T];
+    // A cell's global reads, issued before its first store.
+    bool simu = mode != MODE_MBP;
+    int nrep[T], nini[T];
+    float lini[T];
+    auto read_cell = [&](int cell) {
       if (mode == MODE_REPLAY) {
 #pragma unroll
         for (int tr = 0; tr < T; tr++) nrep[tr] = tn_r[tr * AG + cell];
       }
-      if (mode == MODE_MBP && !simu) {
+      if (mode == MODE_MBP) {
+        simu = simu_s ? simu_s[cell / G] != 0 : false;
 #pragma unroll
         for (int tr = 0; tr < T; tr++) {
           nini[tr] = itn[tr * AG + cell];
           lini[tr] = itm[tr * AG + cell];
         }
       }
+    };
+    // (B) area mixing, from LDS when the CSR is staged there.
+    if (staged)
+      mix_cells((lcfloat*)sdiag, (lcfloat*)sfac, (lcint*)sptr, (lcint*)ssrc, (lcfloat*)sw, (lcint*)sord, sdinf, sI, m,
+                G, AG, tid, nt);
+    else
+      mix_cells(diag, fac, in_ptr, in_src, in_w, order, sdinf, sI, m, G, AG, tid, nt);
+    if (newrow) {
+      if (tid < A) saf[tid] = afr;
+      for (int i = tid + nt; i < A; i += nt) saf[i] = af_s[i];
+    }
+    __syncthreads();
+    // (C) means, small draws, own-cell updates; large draws queued.
+    const bool update = s < S - 1;           // the last step is not applied (src/state.cc:634)
+    const int upd = update ? -1 : 0;
+    const uint32_t c0 = (uint32_t)s | (stream << 16);
+    const rsrc_t tn_b = slab(tn_s, TAG * 4), tm_b = slab(tm_s, TAG * 4), pt_b = slab(pt_s, CAG * 4);
+    for (int cell = tid; cell < AG; cell += nt) {
+      const int j = cell / G, g = cell - j * G;
+      const uint32_t off = 4u * (uint32_t)cell;
+      read_cell(cell);
       int p[CP];
       {
         const int4* pv = (const int4*)pop;
@@ -222,13 +277,6 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
         pool = spool[j * G + (g - st * DPM)];
         p[FROM[INF_TR]] = st == 0 ? pool : 0;
       }
-      if (pt_s) {
-#pragma unroll
-        for (int c = 0; c < C; c++) st_nt(pt_s, c * AG + cell, p[c]);
-      }
-      int q[CP];
-#pragma unroll
-      for (int c = 0; c < CP; c++) q[c] = p[c];
       float nmi = 0.f;
 #pragma unroll
       for (int gg = 0; gg < G; gg++) nmi += sN[g * G + gg] * sI[j * G + gg];
@@ -244,73 +292,118 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
       }
       mod_foi_factors(tpp, s, cell, afc, agc);
       const float foi = foi_mean(bet, afc, nmi, ef, agc);
-      CellRng rng;
-      rng.init(k0, k1, c0, (uint32_t)cell, jb.key);
-      if (mode != MODE_REPLAY) rng.prime();
+      // All means first, without a branch.
+      float lp[T];
+      int bad = 0;
 #pragma unroll
       for (int tr = 0; tr < T; tr++) {
-        const int fr = FROM[tr], to = TO[tr];
-        float popu = (float)p[fr];
+        float popu = (float)p[FROM[tr]];
         if constexpr (NSTRAIN > 1) {
           if (tr == INF_TR) popu = (float)pool;
         }
-        float lp = 0.f;
-        if (popu > 0.f) lp = tr == INF_TR ? dt * popu * ssus[g] * foi : dt * popu * srate[tr * G + g];
-        lp = mod_mean(tpp, s, tr, cell, lp);
-        // src/state.cc:429 (NaN mean) and src/utils.cc:150 (mean > 1e9) stop the reference.
-        if (lp != lp) { atomicOr(jb.err, 1); lp = 0.f; }
-        else if (lp > 1e9f) { atomicOr(jb.err, 2); lp = 0.f; }
-        if (tm_s) st_nt(tm_s, tr * AG + cell, lp);
-        int n = 0;
-        int kind = -1;
-        float val = 0.f;
-        if (mode == MODE_REPLAY) {
-          n = nrep[tr];
-        } else if (lp > 0.f) {
-          if (mode == MODE_SIM || simu) {
-            if (lp < BEEP_POIS_INLINE) n = poisson_inversion(lp, rng.next());
-            else { kind = ITEM_POIS; val = lp; }
-          } else {
+        const float mean = tr == INF_TR ? dt * popu * ssus[g] * foi : dt * popu * srate[tr * G + g];
+        lp[tr] = popu > 0.f ? mean : 0.f;
+      }
+      if (tpp->mod_trans) {
+#pragma unroll
+        for (int tr = 0; tr < T; tr++) lp[tr] = mod_mean(tpp, s, tr, cell, lp[tr]);
+      }
+      // src/state.cc:429 (NaN mean) and src/utils.cc:150 (mean > 1e9) stop the reference.
+#pragma unroll
+      for (int tr = 0; tr < T; tr++) {
+        bad |= lp[tr] != lp[tr] ? 1 : lp[tr] > 1e9f ? 2 : 0;
+        lp[tr] = lp[tr] <= 1e9f ? lp[tr] : 0.f;
+      }
+      if (wave_any(bad != 0)) {
+        if (bad) atomicOr(jb.err, bad);
+      }
+      if (pt_s) {
+#pragma unroll
+        for (int c = 0; c < C; c++) st_slab(pt_b, p[c], off, (uint32_t)(4 * c * AG));
+      }
+      if (tm_s) {
+#pragma unroll
+        for (int tr = 0; tr < T; tr++) st_slab(tm_b, __float_as_int(lp[tr]), off, (uint32_t)(4 * tr * AG));
+      }
+      // Draws in transition order: n[tr] events now, or qv[tr] != 0 queued for
+      // (D): a Poisson mean (>= 10), minus the mean of a proposal's additional
+      // events (<= -10), or a binomial probability in (0, 1).
+      int q[CP];
+#pragma unroll
+      for (int c = 0; c < CP; c++) q[c] = p[c];
+      float qv[T];
+      if constexpr (MODE == MODE_REPLAY) {
+#pragma unroll
+        for (int tr = 0; tr < T; tr++) {
+          q[FROM[tr]] -= nrep[tr] & upd;
+          q[TO[tr]] += nrep[tr] & upd;
+        }
+      } else {
+        CellRng rng;
+        rng.init(k0, k1, c0, (uint32_t)cell, jb.key);
+        rng.prime();
+#pragma unroll
+        for (int tr = 0; tr < T; tr++) {
+          float lam = lp[tr];                // mean of the Poisson part
+          int base = 0;                      // events carried over from the current trajectory
+          bool bino = false;
+          float pr = 0.f;
+          qv[tr] = lam >= BEEP_POIS_INLINE ? lam : 0.f;
+          if constexpr (MODE == MODE_MBP) {
             // Coupled proposal (src/mbp.cc:286-311).
             const int ni = nini[tr];
             const float li = lini[tr];
-            if (lp > li) {
-              float dl = lp - li;
-              if (dl < BEEP_POIS_INLINE) n = ni + poisson_inversion(dl, rng.next());
-              else { kind = ITEM_POIS_ADD; val = dl; }
-            } else if (lp == li) {
-              n = ni;
-            } else {
-              float pr = lp / li;
-              float pp = pr > 0.5f ? 1.f - pr : pr;
-              if ((float)ni * pp < 10.f) n = binomial_draw_small(ni, pr, rng.next(), rng);
-              else { kind = ITEM_BINOM; val = pr; }
+            const bool coupled = !simu && lam > 0.f;
+            const bool down = coupled && !(lam > li) && !(lam == li);
+            const float dl = lam > li ? lam - li : 0.f;
+            if (coupled) {
+              base = ni;
+              qv[tr] = dl >= BEEP_POIS_INLINE ? -dl : 0.f;
+              lam = dl;
+            }
+            if (down) {
+              pr = lp[tr] / li;
+              const float pp = pr > 0.5f ? 1.f - pr : pr;
+              bino = (float)ni * pp < 10.f;
+              qv[tr] = bino ? 0.f : pr;
             }
           }
-        }
-        // Draws queued for (D): the wavefront's lanes that queue this
-        // transition take consecutive slots from one LDS atomic (the draws are
-        // keyed by cell and transition, so the slots' order is immaterial).
-        const unsigned long long qm = __ballot(kind >= 0);
-        if (qm) {
-          const int lane = (int)__lane_id();
-          const int leader = __ffsll((long long)qm) - 1;
-          int base = 0;
-          if (lane == leader) base = atomicAdd(qcount, __popcll(qm));
-          base = __shfl(base, leader);
-          if (kind >= 0) {
-            const int slot = base + __popcll(qm & ((1ull << lane) - 1ull));
-            const uint32_t idx = (uint32_t)cell * T + tr;
-            if (q16) qidx16[slot] = (uint16_t)idx;
-            else qidx32[slot] = idx;
-            qval[slot] = kind == ITEM_POIS_ADD ? -val : val;
+          const bool pois = lam > 0.f && qv[tr] == 0.f && !bino;
+          int n = base;
+          if (pois || bino) {
+            const float u = rng.next();
+            if (!bino) n = base + poisson_inversion(lam, u);
+            else n = binomial_draw_small(nini[tr], pr, u, rng);
           }
+          n = qv[tr] != 0.f ? 0 : n;
+          // Lanes that queue have the store dropped by the slab's range check.
+          if (tn_s) st_slab(tn_b, n, qv[tr] != 0.f ? 0x80000000u : off, (uint32_t)(4 * tr * AG));
+          q[FROM[tr]] -= n & upd;
+          q[TO[tr]] += n & upd;
         }
-        if (kind < 0) {
-          if (tn_s && mode != MODE_REPLAY) st_nt(tn_s, tr * AG + cell, n);
-          if (update) {
-            q[fr] -= n;
-            q[to] += n;
+        // The wavefront's queued draws take consecutive slots from one LDS
+        // atomic (they are keyed by cell and transition, so the slots' order
+        // is immaterial).
+        int total = 0;
+#pragma unroll
+        for (int tr = 0; tr < T; tr++) total += __popcll(__builtin_amdgcn_ballot_w64(qv[tr] != 0.f));
+        if (total) {
+          const int lane = (int)__lane_id();
+          const int leader = __ffsll((long long)__builtin_amdgcn_ballot_w64(true)) - 1;
+          int base = 0;
+          if (lane == leader) base = atomicAdd(qcount, total);
+          base = __builtin_amdgcn_readlane(base, leader);
+#pragma unroll
+          for (int tr = 0; tr < T; tr++) {
+            const unsigned long long qm = __builtin_amdgcn_ballot_w64(qv[tr] != 0.f);
+            if (qv[tr] != 0.f) {
+              const int slot = base + __popcll(qm & ((1ull << lane) - 1ull));
+              const uint32_t idx = (uint32_t)cell * T + tr;
+              if (q16) qidx16[slot] = (uint16_t)idx;
+              else qidx32[slot] = idx;
+              qval[slot] = qv[tr];
+            }
+            base += __popcll(qm);
           }
         }
       }
@@ -320,23 +413,26 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
         for (int c4 = 0; c4 < CP / 4; c4++)
           pv[c4 * AG + cell] = make_int4(q[4 * c4], q[4 * c4 + 1], q[4 * c4 + 2], q[4 * c4 + 3]);
       }
+      if constexpr (NSTRAIN == 1) sdinf[cell] = infectivity(q, sinf);
     }
     __syncthreads();
     // (D) the queued large draws (PTRS / BTRD), every lane busy.
-    if (mode != MODE_REPLAY) {
-      const int nq = qcount[0];
+    int nq = 0;
+    if constexpr (MODE != MODE_REPLAY) {
+      nq = qcount[0];
       if (nq > 0) {
         for (int i = tid; i < nq; i += nt) {
           const uint32_t idx = q16 ? (uint32_t)qidx16[i] : qidx32[i];
           const int cell = (int)(idx / T), tr = (int)(idx - (uint32_t)cell * T);
-          // The kind from the value: Poisson means queued are >= the inline
-          // limit, binomial probabilities lie in (0, 1), coupled Poisson
-          // increments are stored negated.
           const float v = qval[i];
-          const int kind = v < 0.f ? ITEM_POIS_ADD : (v < 1.f ? ITEM_BINOM : ITEM_POIS);
-          int ni = mode == MODE_MBP ? itn[tr * AG + cell] : 0;
-          int n = draw_item_inline(kind, fabsf(v), ni, k0, k1, c0, (uint32_t)cell, (uint32_t)tr, jb.key);
-          if (tn_s) st_nt(tn_s, tr * AG + cell, n);
+          int n;
+          if constexpr (MODE == MODE_SIM) {
+            n = draw_large_poisson(v, k0, k1, c0, (uint32_t)cell, (uint32_t)tr, jb.key);
+          } else {
+            const int kind = v < 0.f ? ITEM_POIS_ADD : (v < 1.f ? ITEM_BINOM : ITEM_POIS);
+            n = draw_item_inline(kind, fabsf(v), itn[tr * AG + cell], k0, k1, c0, (uint32_t)cell, (uint32_t)tr, jb.key);
+          }
+          if (tn_s) st_slab(tn_b, n, 4u * (uint32_t)(tr * AG + cell), 0);
           if (update && n != 0) {
             int fr = 0, to = 0;
 #pragma unroll
@@ -350,27 +446,13 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
         if (tid == 0) qcount[0] = 0;
       }
     }
-    // (E) infectivity for the next step.
-    for (int cell = tid; cell < AG; cell += nt) {
-      const int4* pv = (const int4*)pop;
-      float d = 0.f;
-#pragma unroll
-      for (int c4 = 0; c4 < CP / 4; c4++) {
-        int4 v = pv[c4 * AG + cell];
-        int pc[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-          const int c = 4 * c4 + k;
-          if (c < C && INFC[c]) {
-            float w = sinf[c];
-            if (w != 0.f) d += w * (float)pc[k];
-          }
-        }
-      }
-      sdinf[cell] = d;
+    // (E) infectivity for the next step, where (D) or the pooling over strains
+    // changed what (C) wrote.
+    if (NSTRAIN > 1 || nq > 0) {
+      for (int cell = tid; cell < AG; cell += nt) sdinf[cell] = cell_infectivity(pop, cell, AG, sinf);
+      pool_susceptibles(pop, spool, AG, tid, nt);
+      __syncthreads();
     }
-    pool_susceptibles(pop, spool, AG, tid, nt);
-    __syncthreads();
   }
   for (int cell = tid; cell < AG; cell += nt) {
 #pragma unroll
@@ -393,8 +475,4 @@ extern "C" __global__ void __launch_bounds__(BEEP_SPEC_MAX_BLOCK, beepspec::MIN_
 extern "C" __global__ void __launch_bounds__(BEEP_SPEC_MAX_BLOCK, beepspec::MIN_WAVES)
     beep_fused_spec_replay(const beepdev::Job* jobs, uint64_t seed, uint32_t stream) {
   beepdev::fused_spec_body<beepdev::MODE_REPLAY>(jobs, seed, stream);
-}
-extern "C" __global__ void __launch_bounds__(BEEP_SPEC_MAX_BLOCK, beepspec::MIN_WAVES)
-    beep_fused_spec_any(const beepdev::Job* jobs, uint64_t seed, uint32_t stream) {
-  beepdev::fused_spec_body<beepdev::MODE_ANY>(jobs, seed, stream);
 }

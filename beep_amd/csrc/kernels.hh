@@ -27,8 +27,7 @@ template <int MODE>
 __global__ void __launch_bounds__(BEEP_FUSED_MAX_BLOCK, 4)
     k_fused(const Job* __restrict__ jobs, uint64_t seed, uint32_t stream) {
   const Job jb = jobs[blockIdx.x];
-  // MODE_ANY launches mix simulations and proposals: the job says which.
-  const int mode = MODE == MODE_ANY ? jb.mode : MODE;
+  constexpr int mode = MODE;
   ctopo* __restrict__ tpp = (ctopo*)jb.topo;
   const int A = tpp->A, G = tpp->G, C = tpp->C, T = tpp->T, S = tpp->S, AG = tpp->AG, inf_tr = tpp->inf_tr;
   const int nt = blockDim.x, tid = threadIdx.x;
