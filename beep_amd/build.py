@@ -21,13 +21,17 @@ JIT_INC = os.path.join(CSRC, "jit_sources.inc")
 # Compartment structures the run-time compiled kernel is checked with at build
 # time: SEIR (S->E, E->I, I->R, I infectious) with one strain, and the same
 # with two strains (which compiles the pooling of susceptibles).
-CHECK_PRELUDES = ["""namespace beepspec {
+CHECK_PRELUDES = ["""#define BEEP_SPEC_FUSED
+#define BEEP_SPEC_STEP
+namespace beepspec {
 constexpr int C = 4, T = 3, G = %d, CP = 4, INF_TR = 0, MIN_WAVES = 4, STEP_WAVES = 4, NSTRAIN = %d, DPM = 1;
+constexpr bool GROUPED = %s, N_TV = false, MODS = false, AF_STATIC = true, STAGED = true, Q16 = true;
+constexpr bool KEEP_TN = true, KEEP_TM = true, KEEP_PT = true;
 constexpr int FROM[3] = {0, 1, 2};
 constexpr int TO[3] = {1, 2, 3};
 constexpr bool INFC[4] = {false, false, true, false};
 }  // namespace beepspec
-""" % (g, g) for g in (1, 2)]
+""" % (g, g, "true" if g == 2 else "false") for g in (1, 2)]
 CHECK_SRC = os.path.join(CSRC, "host", "gpu_state_check.cc")
 CHECK_BIN = os.path.join(HERE, "bin", "gpu_state_check")
 

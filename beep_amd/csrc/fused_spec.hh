@@ -8,6 +8,10 @@
 //   constexpr int FROM[T], TO[T];     transition source / destination
 //   constexpr bool INFC[C];           compartments with an infectivity weight
 //   constexpr int NSTRAIN, DPM;       strains, and groups per strain (G = NSTRAIN * DPM)
+//   constexpr bool GROUPED, N_TV, MODS, AF_STATIC;   R or external-force groups, a time-varying age matrix,
+//                                     prediction-mode modifications, an area factor that does not vary
+//   constexpr bool STAGED, Q16;       the mixing CSR staged in LDS, 16-bit queue indices
+//   constexpr bool KEEP_TN, KEEP_TM, KEEP_PT;   the trajectories kept
 //
 // It computes exactly what k_fused (kernels.hh) computes -- the same FP32
 // expressions in the same order and the same uniforms consumed in the same
@@ -100,7 +104,7 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
   const int nt = blockDim.x, tid = threadIdx.x;
   const float dt = tpp->dt;
   const int qcap = T * AG;                             // every (cell, transition): never full
-  const bool q16 = spec_queue16(T, AG);
+  constexpr bool q16 = Q16;
 
   extern __shared__ int smem[];
   int* pop = smem;                                     // [CP/4][AG] chunks of 4 compartments
@@ -118,12 +122,13 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
   gcint* in_src = gptr(tpp->in_src);
   gcfloat* in_w = gptr(tpp->in_w);
   gcint* order = gptr(tpp->mix_order);
-  const bool staged = tpp->stage_mix != 0;
+  constexpr bool staged = STAGED;
   // This step's area factor and the external force's age weights, read by
   // every cell in (C): from LDS, so that no global load there waits behind the
   // trajectory stores still in flight (loads and stores share one counter).
   float* saf = sinf + C;                               // [A]
-  const int nE = tpp->nE, grouped = tpp->nR > 1 || nE > 1;
+  constexpr bool grouped = GROUPED;
+  const int nE = grouped ? tpp->nE : 1;
   float* sage = saf + A;                               // [nE][G] age weights of each external-force group
   // With R or external-force groups: this step's beta of every area and
   // external force of every (strain, area), and each (strain, area)'s group.
@@ -144,7 +149,7 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
   // Strains: each strain-0 cell's susceptibles pooled over the strains of its
   // dp (src/state.cc:395-404), after the queue's indices.
   int* spool = (int*)((char*)qidx + ((size_t)qcap * (q16 ? 2 : 4) + 3) / 4 * 4);
-  if (staged) {
+  if constexpr (staged) {
     for (int i = tid; i < A; i += nt) { sdiag[i] = diag[i]; sfac[i] = fac[i]; sord[i] = order[i]; }
     for (int i = tid; i <= A; i += nt) sptr[i] = in_ptr[i];
     for (int i = tid; i < tpp->nnz; i += nt) { ssrc[i] = in_src[i]; sw[i] = in_w[i]; }
@@ -162,12 +167,12 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
     for (int i = tid; i < G; i += nt) ssus[i] = tab[tpp->off_sus + i];
     for (int i = tid; i < C; i += nt) sinf[i] = tab[tpp->off_inf + i];
     for (int i = tid; i < nE * G; i += nt) sage[i] = gptr(tpp->agedist)[i];
-    if (grouped)
+    if constexpr (grouped)
       for (int i = tid; i < NSTRAIN * A; i += nt) segrp[i] = tpp->nE > 1 ? gptr(tpp->egrp)[i] : 0;
     if (tid == 0) qcount[0] = 0;
   }
-  const bool af_static = tpp->af_static != 0;
-  if (af_static) {
+  constexpr bool af_static = AF_STATIC;
+  if constexpr (af_static) {
     gcfloat* af0 = af_row(tpp, tab, 0);
     for (int i = tid; i < A; i += nt) saf[i] = af0[i];
   }
@@ -205,19 +210,16 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
     const bool newrow = !af_static && (s == t0 || s % spd == 0);
     float afr = 0.f;
     if (newrow && tid < A) afr = af_s[tid];
-    if (grouped) {
+    if constexpr (grouped) {
       const int nR = tpp->nR;
       for (int i = tid; i < A; i += nt) sbeta[i] = tab[tpp->off_beta + (size_t)s * nR + (nR > 1 ? gptr(tpp->rgrp)[i] : 0)];
       for (int i = tid; i < NSTRAIN * A; i += nt) sefoi[i] = tab[tpp->off_efoi + (size_t)s * nE + segrp[i]];
     }
     // A time-varying age matrix: this step's.  Step s-1's reads of sN in (C)
     // ended at the barrier after (C); these writes are seen after (B)'s.
-    if (tpp->N_tv) {
+    if constexpr (N_TV) {
       for (int i = tid; i < G * G; i += nt) sN[i] = tab[tpp->off_N + (size_t)s * G * G + i];
     }
-    int* tn_s = jb.tn ? jb.tn + (size_t)s * TAG : nullptr;
-    float* tm_s = jb.tm ? jb.tm + (size_t)s * TAG : nullptr;
-    int* pt_s = jb.pt ? jb.pt + (size_t)s * CAG : nullptr;
     gcint* itn = mode == MODE_MBP ? gptr(jb.init_tn) + (size_t)s * TAG : nullptr;
     gcfloat* itm = mode == MODE_MBP ? gptr(jb.init_tm) + (size_t)s * TAG : nullptr;
     gcint* tn_r = mode == MODE_REPLAY ? gptr(jb.tn) + (size_t)s * TAG : nullptr;
@@ -241,7 +243,7 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
       }
     };
     // (B) area mixing, from LDS when the CSR is staged there.
-    if (staged)
+    if constexpr (staged)
       mix_cells((lcfloat*)sdiag, (lcfloat*)sfac, (lcint*)sptr, (lcint*)ssrc, (lcfloat*)sw, (lcint*)sord, sdinf, sI, m,
                 G, AG, tid, nt);
     else
@@ -255,7 +257,10 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
     const bool update = s < S - 1;           // the last step is not applied (src/state.cc:634)
     const int upd = update ? -1 : 0;
     const uint32_t c0 = (uint32_t)s | (stream << 16);
-    const rsrc_t tn_b = slab(tn_s, TAG * 4), tm_b = slab(tm_s, TAG * 4), pt_b = slab(pt_s, CAG * 4);
+    rsrc_t tn_b, tm_b, pt_b;                 // this step's slabs
+    if constexpr (KEEP_TN) tn_b = slab(jb.tn + (size_t)s * TAG, TAG * 4);
+    if constexpr (KEEP_TM) tm_b = slab(jb.tm + (size_t)s * TAG, TAG * 4);
+    if constexpr (KEEP_PT) pt_b = slab(jb.pt + (size_t)s * CAG, CAG * 4);
     for (int cell = tid; cell < AG; cell += nt) {
       const int j = cell / G, g = cell - j * G;
       const uint32_t off = 4u * (uint32_t)cell;
@@ -282,7 +287,7 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
       for (int gg = 0; gg < G; gg++) nmi += sN[g * G + gg] * sI[j * G + gg];
       if (nmi < 0.f) nmi = 0.f;
       float afc = saf[j], agc, bet = beta_s, ef = efoi_s;
-      if (grouped) {
+      if constexpr (grouped) {
         const int k = (g / DPM) * A + j;
         bet = sbeta[j];
         ef = sefoi[k];
@@ -290,7 +295,7 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
       } else {
         agc = sage[g];
       }
-      mod_foi_factors(tpp, s, cell, afc, agc);
+      if constexpr (MODS) mod_foi_factors(tpp, s, cell, afc, agc);
       const float foi = foi_mean(bet, afc, nmi, ef, agc);
       // All means first, without a branch.
       float lp[T];
@@ -304,7 +309,7 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
         const float mean = tr == INF_TR ? dt * popu * ssus[g] * foi : dt * popu * srate[tr * G + g];
         lp[tr] = popu > 0.f ? mean : 0.f;
       }
-      if (tpp->mod_trans) {
+      if constexpr (MODS) {
 #pragma unroll
         for (int tr = 0; tr < T; tr++) lp[tr] = mod_mean(tpp, s, tr, cell, lp[tr]);
       }
@@ -317,11 +322,11 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
       if (wave_any(bad != 0)) {
         if (bad) atomicOr(jb.err, bad);
       }
-      if (pt_s) {
+      if constexpr (KEEP_PT) {
 #pragma unroll
         for (int c = 0; c < C; c++) st_slab(pt_b, p[c], off, (uint32_t)(4 * c * AG));
       }
-      if (tm_s) {
+      if constexpr (KEEP_TM) {
 #pragma unroll
         for (int tr = 0; tr < T; tr++) st_slab(tm_b, __float_as_int(lp[tr]), off, (uint32_t)(4 * tr * AG));
       }
@@ -377,7 +382,7 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
           }
           n = qv[tr] != 0.f ? 0 : n;
           // Lanes that queue have the store dropped by the slab's range check.
-          if (tn_s) st_slab(tn_b, n, qv[tr] != 0.f ? 0x80000000u : off, (uint32_t)(4 * tr * AG));
+          if constexpr (KEEP_TN) st_slab(tn_b, n, qv[tr] != 0.f ? 0x80000000u : off, (uint32_t)(4 * tr * AG));
           q[FROM[tr]] -= n & upd;
           q[TO[tr]] += n & upd;
         }
@@ -432,7 +437,7 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
             const int kind = v < 0.f ? ITEM_POIS_ADD : (v < 1.f ? ITEM_BINOM : ITEM_POIS);
             n = draw_item_inline(kind, fabsf(v), itn[tr * AG + cell], k0, k1, c0, (uint32_t)cell, (uint32_t)tr, jb.key);
           }
-          if (tn_s) st_slab(tn_b, n, 4u * (uint32_t)(tr * AG + cell), 0);
+          if constexpr (KEEP_TN) st_slab(tn_b, n, 4u * (uint32_t)(tr * AG + cell), 0);
           if (update && n != 0) {
             int fr = 0, to = 0;
 #pragma unroll
@@ -462,6 +467,7 @@ __device__ inline void fused_spec_body(const Job* __restrict__ jobs, uint64_t se
 
 }  // namespace beepdev
 
+#ifdef BEEP_SPEC_FUSED
 extern "C" __global__ void __launch_bounds__(BEEP_SPEC_MAX_BLOCK, beepspec::MIN_WAVES)
     beep_fused_spec_sim(const beepdev::Job* jobs, uint64_t seed, uint32_t stream) {
   beepdev::fused_spec_body<beepdev::MODE_SIM>(jobs, seed, stream);
@@ -476,3 +482,4 @@ extern "C" __global__ void __launch_bounds__(BEEP_SPEC_MAX_BLOCK, beepspec::MIN_
     beep_fused_spec_replay(const beepdev::Job* jobs, uint64_t seed, uint32_t stream) {
   beepdev::fused_spec_body<beepdev::MODE_REPLAY>(jobs, seed, stream);
 }
+#endif

@@ -31,7 +31,7 @@ __device__ inline void step_spec_body(const Job* __restrict__ jobs, const float*
   __shared__ float srate[T * G], sN[G * G], ssus[G], sinf[C];
   gcfloat* tab = gptr(jb.tab);
   for (int i = tid; i < T * G; i += BEEP_STEP_BLOCK) srate[i] = tab[tp->off_rate + i];
-  const size_t offN = tp->off_N + (tp->N_tv ? (size_t)s * G * G : 0);   // a time-varying age matrix: step s's
+  const size_t offN = tp->off_N + (N_TV ? (size_t)s * G * G : 0);   // a time-varying age matrix: step s's
   for (int i = tid; i < G * G; i += BEEP_STEP_BLOCK) sN[i] = tab[offN + i];
   for (int i = tid; i < G; i += BEEP_STEP_BLOCK) ssus[i] = tab[tp->off_sus + i];
   for (int i = tid; i < C; i += BEEP_STEP_BLOCK) sinf[i] = tab[tp->off_inf + i];
@@ -39,9 +39,9 @@ __device__ inline void step_spec_body(const Job* __restrict__ jobs, const float*
   __syncthreads();
 
   const size_t TAG = (size_t)T * AG, CAG = (size_t)C * AG;
-  int* tn_s = jb.tn ? jb.tn + (size_t)s * TAG : nullptr;
-  float* tm_s = jb.tm ? jb.tm + (size_t)s * TAG : nullptr;
-  int* pt_s = jb.pt ? jb.pt + (size_t)s * CAG : nullptr;
+  int* tn_s = KEEP_TN ? jb.tn + (size_t)s * TAG : nullptr;
+  float* tm_s = KEEP_TM ? jb.tm + (size_t)s * TAG : nullptr;
+  int* pt_s = KEEP_PT ? jb.pt + (size_t)s * CAG : nullptr;
   gcint* itn = MODE == MODE_MBP ? gptr(jb.init_tn) + (size_t)s * TAG : nullptr;
   gcfloat* itm = MODE == MODE_MBP ? gptr(jb.init_tm) + (size_t)s * TAG : nullptr;
   gcint* tn_r = MODE == MODE_REPLAY ? gptr(jb.tn) + (size_t)s * TAG : nullptr;
@@ -56,7 +56,7 @@ __device__ inline void step_spec_body(const Job* __restrict__ jobs, const float*
     int p[CP];
 #pragma unroll
     for (int c = 0; c < CP; c++) p[c] = c < C ? state[c * AG + cell] : 0;
-    if (pt_s) {
+    if constexpr (KEEP_PT) {
 #pragma unroll
       for (int c = 0; c < C; c++) st_nt(pt_s, c * AG + cell, p[c]);
     }
@@ -71,7 +71,7 @@ __device__ inline void step_spec_body(const Job* __restrict__ jobs, const float*
     float bet, ef, agc;
     foi_groups(tp, tab, s, j, g, DPM, bet, ef, agc);
     float afc = af_row(tp, tab, s)[j];
-    mod_foi_factors(tp, s, cell, afc, agc);
+    if constexpr (MODS) mod_foi_factors(tp, s, cell, afc, agc);
     const float foi = foi_mean(bet, afc, nmi, ef, agc);
     const bool simu = MODE == MODE_MBP ? (jb.simu ? gptr(jb.simu)[(size_t)s * A + j] != 0 : false) : true;
     CellRng rng;
@@ -83,10 +83,10 @@ __device__ inline void step_spec_body(const Job* __restrict__ jobs, const float*
       float popu = (float)p[fr];
       float lp = 0.f;
       if (popu > 0.f) lp = tr == INF_TR ? dt * popu * ssus[g] * foi : dt * popu * srate[tr * G + g];
-      lp = mod_mean(tp, s, tr, cell, lp);
+      if constexpr (MODS) lp = mod_mean(tp, s, tr, cell, lp);
       if (lp != lp) { atomicOr(jb.err, 1); lp = 0.f; }
       else if (lp > 1e9f) { atomicOr(jb.err, 2); lp = 0.f; }
-      if (tm_s) st_nt(tm_s, tr * AG + cell, lp);
+      if constexpr (KEEP_TM) st_nt(tm_s, tr * AG + cell, lp);
       int n = 0, kind = -1;
       float val = 0.f;
       if (MODE == MODE_REPLAY) {
@@ -117,7 +117,7 @@ __device__ inline void step_spec_body(const Job* __restrict__ jobs, const float*
         qcode[slot] = (uint32_t)tid | ((uint32_t)tr << 20) | ((uint32_t)kind << 28);
         qval[slot] = val;
       } else {
-        if (tn_s && MODE != MODE_REPLAY) st_nt(tn_s, tr * AG + cell, n);
+        if constexpr (KEEP_TN && MODE != MODE_REPLAY) st_nt(tn_s, tr * AG + cell, n);
         if (update) {
           q[fr] -= n;
           q[to] += n;
@@ -135,7 +135,7 @@ __device__ inline void step_spec_body(const Job* __restrict__ jobs, const float*
     int c2 = blockIdx.y * BEEP_STEP_BLOCK + t2;
     int ni = MODE == MODE_MBP ? itn[tr * AG + c2] : 0;
     int n = draw_item_inline(kind, qval[i], ni, k0, k1, c0, (uint32_t)c2, (uint32_t)tr, jb.key);
-    if (tn_s) st_nt(tn_s, tr * AG + c2, n);
+    if constexpr (KEEP_TN) st_nt(tn_s, tr * AG + c2, n);
     if (update && n != 0) {
       int fr = 0, to = 0;
 #pragma unroll
@@ -163,6 +163,7 @@ __device__ inline void step_spec_body(const Job* __restrict__ jobs, const float*
 
 }  // namespace beepdev
 
+#ifdef BEEP_SPEC_STEP
 extern "C" __global__ void __launch_bounds__(BEEP_STEP_BLOCK, beepspec::STEP_WAVES)
     beep_step_spec_sim(const beepdev::Job* jobs, const float* I, float* D, int Apad, int s, const uint64_t* rngp) {
   beepdev::step_spec_body<beepdev::MODE_SIM>(jobs, I, D, Apad, s, rngp);
@@ -175,3 +176,4 @@ extern "C" __global__ void __launch_bounds__(BEEP_STEP_BLOCK, beepspec::STEP_WAV
     beep_step_spec_replay(const beepdev::Job* jobs, const float* I, float* D, int Apad, int s, const uint64_t* rngp) {
   beepdev::step_spec_body<beepdev::MODE_REPLAY>(jobs, I, D, Apad, s, rngp);
 }
+#endif
