@@ -1625,38 +1625,87 @@ int beep_put_transnum(beep_ctx* c, int inst, int slot, const int32_t* tn) {
   return check_device_error(c);
 }
 
+}  // extern "C"
+
+namespace {
+
+// Copies of 4-byte rows within the arrays `arr` (pointer, values per row), for
+// pairs dst[i] <- src[i] in order; pairs with dst == src do nothing.  When no
+// row is both read and written and none is written twice the order is
+// immaterial and each array takes one launch; otherwise each pair is a copy
+// command of its own, in order.
+int copy_rows(beep_ctx* c, int n, const int32_t* dst, const int32_t* src, const std::vector<std::pair<void*, size_t>>& arr) {
+  std::vector<int32_t> d, s;
+  std::vector<char> use(c->capacity, 0);
+  bool free_order = true;
+  for (int i = 0; i < n; i++) {
+    if (dst[i] == src[i]) continue;
+    d.push_back(dst[i]);
+    s.push_back(src[i]);
+    if (use[dst[i]]) free_order = false;
+    use[dst[i]] = 2;
+    if (use[src[i]] == 2) free_order = false;
+    else use[src[i]] = 1;
+  }
+  if (d.empty()) return BEEP_OK;
+  const size_t m = d.size();
+  if (!free_order || m == 1) {
+    for (size_t i = 0; i < m; i++)
+      for (const auto& a : arr)
+        HIPCHK(c, hipMemcpyAsync((char*)a.first + (size_t)d[i] * a.second * 4, (const char*)a.first + (size_t)s[i] * a.second * 4,
+                                 a.second * 4, hipMemcpyDeviceToDevice, c->stream));
+    return BEEP_OK;
+  }
+  int rc;
+  if ((rc = ensure_scratch(c, 2 * m * sizeof(int)))) return rc;
+  int* d_idx = (int*)c->d_scratch;
+  d.insert(d.end(), s.begin(), s.end());
+  HIPCHK(c, hipMemcpyAsync(d_idx, d.data(), 2 * m * sizeof(int), hipMemcpyHostToDevice, c->stream));
+  for (const auto& a : arr) {
+    // 16 bytes a lane where every row starts on 16 bytes.
+    const size_t row = a.second % 4 ? a.second : a.second / 4;
+    const unsigned gy = (unsigned)std::max<size_t>(1, std::min<size_t>(64, (row + 255) / 256));
+    if (a.second % 4)
+      hipLaunchKernelGGL(beepdev::k_copy_rows<int>, dim3((unsigned)m, gy), dim3(256), 0, c->stream, (int*)a.first, row,
+                         (const int*)d_idx, (const int*)(d_idx + m));
+    else
+      hipLaunchKernelGGL(beepdev::k_copy_rows<int4>, dim3((unsigned)m, gy), dim3(256), 0, c->stream, (int4*)a.first, row,
+                         (const int*)d_idx, (const int*)(d_idx + m));
+    HIPCHK(c, hipGetLastError());
+  }
+  HIPCHK(c, hipStreamSynchronize(c->stream));     // d is the source of an async copy
+  return BEEP_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
 int beep_copy_instances(beep_ctx* c, int n, const int32_t* dst, const int32_t* src) {
   if (!c || n < 0 || (n > 0 && (!dst || !src))) return fail(c, BEEP_EINVAL, "beep_copy_instances: bad arguments");
-  for (int i = 0; i < n; i++) {
+  for (int i = 0; i < n; i++)
     if (!valid_inst(c, dst[i]) || !valid_inst(c, src[i])) return fail(c, BEEP_EINVAL, "instance out of range");
-    if (dst[i] == src[i]) continue;
-    HIPCHK(c, hipMemcpyAsync(c->d_state + (size_t)dst[i] * c->state_sz, c->d_state + (size_t)src[i] * c->state_sz,
-                             c->state_sz * sizeof(int), hipMemcpyDeviceToDevice, c->stream));
-    if (c->d_tn)
-      HIPCHK(c, hipMemcpyAsync(c->d_tn + (size_t)dst[i] * c->traj_sz, c->d_tn + (size_t)src[i] * c->traj_sz,
-                               c->traj_sz * sizeof(int), hipMemcpyDeviceToDevice, c->stream));
-    if (c->d_tm)
-      HIPCHK(c, hipMemcpyAsync(c->d_tm + (size_t)dst[i] * c->traj_sz, c->d_tm + (size_t)src[i] * c->traj_sz,
-                               c->traj_sz * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
-    if (c->d_pt)
-      HIPCHK(c, hipMemcpyAsync(c->d_pt + (size_t)dst[i] * c->pop_traj_sz, c->d_pt + (size_t)src[i] * c->pop_traj_sz,
-                               c->pop_traj_sz * sizeof(int), hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->d_EF + dst[i], c->d_EF + src[i], sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-    c->inst_slot[dst[i]] = c->inst_slot[src[i]];     // the trajectory's parameters go with it
-    c->inst_slot_dirty = true;
-  }
+  std::vector<std::pair<void*, size_t>> arr = {{c->d_state, c->state_sz}, {c->d_EF, 2}};
+  if (c->d_tn) arr.emplace_back(c->d_tn, c->traj_sz);
+  if (c->d_tm) arr.emplace_back(c->d_tm, c->traj_sz);
+  if (c->d_pt) arr.emplace_back(c->d_pt, c->pop_traj_sz);
+  int rc;
+  if ((rc = copy_rows(c, n, dst, src, arr))) return rc;
+  for (int i = 0; i < n; i++)
+    if (dst[i] != src[i]) {
+      c->inst_slot[dst[i]] = c->inst_slot[src[i]];     // the trajectory's parameters go with it
+      c->inst_slot_dirty = true;
+    }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return BEEP_OK;
 }
 
 int beep_copy_states(beep_ctx* c, int n, const int32_t* dst, const int32_t* src) {
   if (!c || n < 0 || (n > 0 && (!dst || !src))) return fail(c, BEEP_EINVAL, "beep_copy_states: bad arguments");
-  for (int i = 0; i < n; i++) {
+  for (int i = 0; i < n; i++)
     if (!valid_inst(c, dst[i]) || !valid_inst(c, src[i])) return fail(c, BEEP_EINVAL, "instance out of range");
-    if (dst[i] == src[i]) continue;
-    HIPCHK(c, hipMemcpyAsync(c->d_state + (size_t)dst[i] * c->state_sz, c->d_state + (size_t)src[i] * c->state_sz,
-                             c->state_sz * sizeof(int), hipMemcpyDeviceToDevice, c->stream));
-  }
+  int rc;
+  if ((rc = copy_rows(c, n, dst, src, {{c->d_state, c->state_sz}}))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return BEEP_OK;
 }
