@@ -72,6 +72,8 @@ struct beep_ctx {
   // observations
   beepdev::ObsDev obs;
   beepdev::ObsDev* d_obs = nullptr;
+  std::vector<int> dt_ptr;          // per data table: its stored observations d_dt_obs[dt_ptr[d] .. dt_ptr[d+1])
+  int* d_dt_obs = nullptr;
   std::vector<int> sec_ptr;
   int* d_sec_ptr = nullptr;
   int* d_sec_obs = nullptr;
@@ -600,7 +602,7 @@ int sync_inst_slot(beep_ctx* c) {
 
 // Defined with the mixed batches, which share it.
 int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const std::vector<const int32_t*>& inst,
-                       const std::vector<int>& ninst, bool store_EF, double* out, int ev0);
+                       const std::vector<int>& ninst, bool store_EF, double* out, double* out_dt, int ev0);
 
 Job make_job(beep_ctx* c, int inst, int slot, uint32_t key, int t0, int t1) {
   Job j;
@@ -965,7 +967,15 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
     od.S = m.S;
     if ((rc = dalloc(c, (void**)&c->d_obs, sizeof(beepdev::ObsDev)))) return rc;
     HIPCHK(c, hipMemcpy(c->d_obs, &od, sizeof od, hipMemcpyHostToDevice));
-    // Sections as lists of stored positions, ascending.
+    // Data tables and sections as lists of stored positions, ascending.
+    std::vector<int> dt_obs;
+    c->dt_ptr.assign(1, 0);
+    for (int d = 0; d < m.ndatatable; d++) {
+      for (int k = 0; k < nobs; k++)
+        if (dtab[k] == d) dt_obs.push_back(k);
+      c->dt_ptr.push_back((int)dt_obs.size());
+    }
+    if ((rc = upload(c, &c->d_dt_obs, dt_obs))) return rc;
     std::vector<int> sptr(1, 0), sobs;
     for (const auto& l : m.section_obs) {
       std::vector<int> v;
@@ -1412,13 +1422,13 @@ int beep_obs_loglik(beep_ctx* c, int n, const int32_t* inst, int section, double
         return fail(c, BEEP_EINVAL, "instance %d has no parameter slot for its observation splines", inst[i]);
     if ((rc = sync_inst_slot(c))) return rc;
   }
-  if (section < 0 && !EF_dt_out) {
+  if (section < 0) {
     // The whole observation model: the mixed batches' chunked kernels, so a
     // batch and this call give the same sums.
     std::vector<beep_ctx*> cs(1, c);
     std::vector<const int32_t*> ip(1, inst);
     std::vector<int> ni(1, n);
-    if ((rc = obs_loglik_chunked(c, cs, ip, ni, true, L_out, 2))) return rc;
+    if ((rc = obs_loglik_chunked(c, cs, ip, ni, true, L_out, EF_dt_out, 2))) return rc;
     c->timing[1] = elapsed(c, 2, 3);
     for (int i = 0; i < n; i++)
       if (std::isnan(L_out[i])) return fail(c, BEEP_ENAN, "NaN observation log-likelihood");   // obsmodel.cc:32
@@ -2070,18 +2080,20 @@ int pow2_ceil(int x) {
   return p;
 }
 
-// The device's batch streams (made by the first batch) and c0's events.
-int ensure_bstreams(beep_ctx* c0, std::vector<hipStream_t>& out) {
+// `want` of the device's batch streams, at most kBatchStreams (made as batches
+// first want them: 4.5 ms each), and c0's events.
+int ensure_bstreams(beep_ctx* c0, size_t want, std::vector<hipStream_t>& out) {
+  want = std::min<size_t>(want, kBatchStreams);
   {
     std::lock_guard<std::mutex> lk(g_bstream_mu);
     BatchStreams& b = g_bstream[c0->device];
-    if (b.st.empty()) {
+    if (b.st.size() < want) {
       hipDeviceProp_t prop;
       HIPCHK(c0, hipGetDeviceProperties(&prop, c0->device));
       const int ncu = prop.multiProcessorCount;
       std::vector<uint32_t> mask((ncu + 31) / 32, 0u);
       for (int i = 0; i < ncu; i++) mask[i / 32] |= 1u << (i % 32);
-      for (int k = 0; k < kBatchStreams; k++) {
+      while (b.st.size() < want) {
         hipStream_t st = nullptr;
         if (hipExtStreamCreateWithCUMask(&st, (uint32_t)mask.size(), mask.data()) != hipSuccess) {
           (void)hipGetLastError();
@@ -2090,7 +2102,7 @@ int ensure_bstreams(beep_ctx* c0, std::vector<hipStream_t>& out) {
         b.st.push_back(st);
       }
     }
-    out = b.st;
+    out.assign(b.st.begin(), b.st.begin() + want);
   }
   if (!c0->bstart) HIPCHK(c0, hipEventCreateWithFlags(&c0->bstart, hipEventDisableTiming));
   while (c0->bend.size() < out.size()) {
@@ -2114,29 +2126,44 @@ int ensure_bstreams(beep_ctx* c0, std::vector<hipStream_t>& out) {
 // kernel variant (k_obs_chunks), then each instance's chunk sums added in
 // chunk order (k_obs_reduce), which also stores its EF when store_EF.  An
 // instance's result depends only on its own trajectory and its context's
-// observations.  Staging in c0's scratch, work on c0's stream; with ev0 >= 0
+// observations.  With out_dt the observations are taken table by table, and
+// out_dt gets each instance's -2 x (sum of each data table) (get_EF_datatable,
+// src/obsmodel.cc:309-322), [instance][ndatatable] per context; the totals are
+// then the sums over the tables' chunks.  Staging in c0's scratch, work on c0's stream; with ev0 >= 0
 // the kernels are bracketed by c0's timing events ev0 and ev0 + 1.  Returns
 // after the results are back.
 int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const std::vector<const int32_t*>& inst,
-                       const std::vector<int>& ninst, bool store_EF, double* out, int ev0) {
+                       const std::vector<int>& ninst, bool store_EF, double* out, double* out_dt, int ev0) {
   hipStream_t st = c0->stream;
   using beepdev::ObsGroup;
   using beepdev::ObsItem;
   constexpr int GN = beepdev::OBS_GROUP;
-  size_t N = 0;
-  for (int v : ninst) N += (size_t)v;
+  size_t N = 0, NI = 0;                            // instances, and sums wanted
+  for (size_t k = 0; k < ctxs.size(); k++) {
+    N += (size_t)ninst[k];
+    NI += (size_t)ninst[k] * (out_dt ? 1 + ctxs[k]->m.ndatatable : 1);
+  }
   if (N == 0) return BEEP_OK;
-  // Group and item counts first, to lay out the staging.
-  size_t ngroups = 0;
-  for (size_t k = 0; k < ctxs.size(); k++) ngroups += ((size_t)ninst[k] + GN - 1) / GN;
+  // A context's lists of observations: all, or one per data table.
+  auto lists = [&](const beep_ctx* c) {
+    std::vector<std::pair<int, int>> r;
+    if (!out_dt) r.emplace_back(0, c->obs.nobs);
+    for (int d = 0; out_dt && d < c->m.ndatatable; d++) r.emplace_back(c->dt_ptr[d], c->dt_ptr[d + 1]);
+    return r;
+  };
+  auto chunks = [](const std::pair<int, int>& r) { return (r.second - r.first + BEEP_OBS_CHUNK - 1) / BEEP_OBS_CHUNK; };
+  // Group, partial and sum counts first, to lay out the staging.
+  size_t ngroups = 0, nparts = 0;
+  for (size_t k = 0; k < ctxs.size(); k++) {
+    const size_t ng = ((size_t)ninst[k] + GN - 1) / GN;
+    for (const auto& r : lists(ctxs[k])) {
+      ngroups += ng;
+      nparts += ng * chunks(r);
+    }
+  }
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t b_inst = al(N * sizeof(int32_t)), b_groups = al(ngroups * sizeof(ObsGroup)),
-               b_items = al(N * sizeof(ObsItem)), b_out = al(N * sizeof(double));
-  size_t nparts = 0;
-  for (size_t k = 0; k < ctxs.size(); k++) {
-    const size_t nchunk = ((size_t)ctxs[k]->obs.nobs + BEEP_OBS_CHUNK - 1) / BEEP_OBS_CHUNK;
-    nparts += nchunk * (((size_t)ninst[k] + GN - 1) / GN);
-  }
+               b_items = al(NI * sizeof(ObsItem)), b_out = al(NI * sizeof(double));
   const size_t b_part = al(nparts * GN * sizeof(double));
   const size_t up = b_inst + b_groups + b_items;
   int rc;
@@ -2151,15 +2178,17 @@ int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const s
   int32_t* h_inst = (int32_t*)h.data();
   ObsItem* h_items = (ObsItem*)(h.data() + b_inst + b_groups);
   // Groups by kernel variant (general / population elements / splines), each
-  // variant's groups contiguous and numbered by workgroup from 0.
+  // variant's groups contiguous and numbered by workgroup from 0.  Sums: the
+  // instances' totals in order, then the tables of each instance in order.
   std::vector<ObsGroup> byv[8];
   long long wgs[8] = {};
-  size_t ii = 0;
+  size_t ii = 0, id = N;
   int part = 0;
   for (size_t k = 0; k < ctxs.size(); k++) {
     beep_ctx* c = ctxs[k];
     const int v = (c->obs_general ? 4 : 0) | (c->obs_pop ? 2 : 0) | (c->nospl ? 1 : 0);
-    const int nchunk = (int)(((size_t)c->obs.nobs + BEEP_OBS_CHUNK - 1) / BEEP_OBS_CHUNK);
+    const auto ls = lists(c);
+    const size_t ndt = out_dt ? ls.size() : 0;
     for (int g0 = 0; g0 < ninst[k]; g0 += GN) {
       ObsGroup G;
       std::memset(&G, 0, sizeof G);
@@ -2169,21 +2198,30 @@ int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const s
       G.ospl = c->nospl ? c->d_ospl : nullptr;
       G.inst_slot = c->nospl ? c->d_inst_slot : nullptr;
       G.inst = d_inst + ii;
+      G.sel = out_dt ? c->d_dt_obs : nullptr;
       G.traj_sz = c->traj_sz;
       G.pop_traj_sz = c->pop_traj_sz;
       G.ninst = std::min(GN, ninst[k] - g0);
-      G.nchunk = nchunk;
-      G.wg0 = (int)wgs[v];
-      G.part0 = part;
+      const int part0 = part;
+      for (size_t t = 0; t < ls.size(); t++) {
+        G.k0 = ls[t].first;
+        G.k1 = ls[t].second;
+        G.nchunk = chunks(ls[t]);
+        G.wg0 = (int)wgs[v];
+        G.part0 = part;
+        for (int q = 0; ndt && q < G.ninst; q++)
+          h_items[id + (size_t)q * ndt + t] = ObsItem{part, G.nchunk, q, -2.f, nullptr};
+        if (G.nchunk > 0) byv[v].push_back(G);
+        wgs[v] += G.nchunk;
+        part += G.nchunk;
+      }
       for (int q = 0; q < G.ninst; q++) {
         const int32_t in = inst[k][g0 + q];
         h_inst[ii] = in;
-        h_items[ii] = ObsItem{part, nchunk, q, store_EF ? c->d_EF + in : nullptr};
+        h_items[ii] = ObsItem{part0, part - part0, q, 1.f, store_EF ? c->d_EF + in : nullptr};
         ii++;
       }
-      if (nchunk > 0) byv[v].push_back(G);
-      wgs[v] += nchunk;
-      part += nchunk;
+      id += (size_t)G.ninst * ndt;
     }
   }
   size_t goff[8], gsum = 0;
@@ -2207,11 +2245,13 @@ int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const s
                        (int)byv[v].size(), d_part);
     HIPCHK(c0, hipGetLastError());
   }
-  hipLaunchKernelGGL(beepdev::k_obs_reduce, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st,
-                     (const ObsItem*)d_items, (int)N, (const double*)d_part, d_out);
+  hipLaunchKernelGGL(beepdev::k_obs_reduce, dim3((unsigned)((NI + 255) / 256)), dim3(256), 0, st,
+                     (const ObsItem*)d_items, (int)NI, (const double*)d_part, d_out);
   HIPCHK(c0, hipGetLastError());
   if (ev0 >= 0) record(c0, ev0 + 1);
   HIPCHK(c0, hipMemcpyAsync(out, d_out, N * sizeof(double), hipMemcpyDeviceToHost, st));
+  if (out_dt && NI > N)
+    HIPCHK(c0, hipMemcpyAsync(out_dt, d_out + N, (NI - N) * sizeof(double), hipMemcpyDeviceToHost, st));
   HIPCHK(c0, hipStreamSynchronize(st));
   return BEEP_OK;
 }
@@ -2251,7 +2291,7 @@ int batch_loglik(beep_ctx* c0, int n, const beep_work* w, double* L_out) {
     }
   // The kernels are timed on the context stream (timing[1]).
   std::vector<double> h(n);
-  if ((rc = obs_loglik_chunked(c0, ctxs, ip, ni, true, h.data(), 2))) return rc;
+  if ((rc = obs_loglik_chunked(c0, ctxs, ip, ni, true, h.data(), nullptr, 2))) return rc;
   c0->timing[1] = elapsed(c0, 2, 3);
   size_t o = 0;
   for (size_t k = 0; k < ctxs.size(); k++)
@@ -2390,8 +2430,8 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
     // device idle; each stream starts after the job upload.  (Autotuning
     // launches run alone on the context stream to be timed.)
     std::vector<hipStream_t> bst;
-    if ((rc = ensure_bstreams(c0, bst))) return rc;
-    const int nbs = (int)std::min(bst.size(), launches.size());
+    if ((rc = ensure_bstreams(c0, launches.size(), bst))) return rc;
+    const int nbs = (int)bst.size();
     std::vector<double> load(nbs, 0.0);
     // The fused phase is timed on the context stream from before the batch
     // streams start to after they have all ended (timing[0]).
