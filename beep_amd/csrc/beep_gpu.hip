@@ -1491,14 +1491,25 @@ int beep_pois_loglik(beep_ctx* c, int n, const int32_t* inst, double* L_out) {
     if (!valid_inst(c, inst[i])) return fail(c, BEEP_EINVAL, "instance %d out of range", inst[i]);
   if (n == 0) return BEEP_OK;
   int rc;
-  if ((rc = ensure_scratch(c, (size_t)n * (sizeof(double) + sizeof(int))))) return rc;
+  // Instances on the grid's y: at most 65535 of them a launch.
+  const size_t nchunk = (c->traj_sz + BEEP_POIS_CHUNK - 1) / BEEP_POIS_CHUNK;
+  constexpr int kRows = 65535;
+  const size_t nb = (size_t)std::min(n, kRows);
+  if ((rc = ensure_scratch(c, (size_t)n * (sizeof(double) + sizeof(int)) + 8 + nb * nchunk * sizeof(double)))) return rc;
   double* d_out = (double*)c->d_scratch;
-  int* d_inst = (int*)(d_out + n);
+  double* d_part = d_out + n;
+  int* d_inst = (int*)(d_part + nb * nchunk);
   HIPCHK(c, hipMemcpyAsync(d_inst, inst, n * sizeof(int), hipMemcpyHostToDevice, c->stream));
   record(c, 4);
-  hipLaunchKernelGGL(beepdev::k_pois_loglik, dim3(n), dim3(256), 0, c->stream, d_inst, c->d_tn, c->d_tm, c->traj_sz,
-                     d_out);
-  HIPCHK(c, hipGetLastError());
+  for (int i0 = 0; i0 < n; i0 += kRows) {
+    const unsigned m = (unsigned)std::min(n - i0, kRows);
+    hipLaunchKernelGGL(beepdev::k_pois_chunks, dim3((unsigned)nchunk, m), dim3(256), 0, c->stream, (const int*)(d_inst + i0),
+                       c->d_tn, c->d_tm, c->traj_sz, (int)nchunk, d_part);
+    HIPCHK(c, hipGetLastError());
+    hipLaunchKernelGGL(beepdev::k_pois_reduce, dim3(m), dim3(64), 0, c->stream, (int)nchunk, (const double*)d_part,
+                       d_out + i0);
+    HIPCHK(c, hipGetLastError());
+  }
   record(c, 5);
   HIPCHK(c, hipMemcpyAsync(L_out, d_out, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
