@@ -1553,49 +1553,77 @@ int beep_accept(beep_ctx* c, int n, const int32_t* init, const int32_t* prop, in
 
 // ---- state transfer ----
 
+}  // extern "C"
+
+namespace {
+
+// S steps of X rows (transitions or compartments) of an instance between its
+// device trajectory `dev` ([s][x][area * group]) and host memory `host`
+// ([s][area][x][group]): slabs of steps are reordered by a kernel next to their
+// copy.  A slab is at most 16 MiB of staging, or what the context already
+// holds; without any, and for up to 4096 values (8 us of host loop, about a
+// kernel launch), the host does the reordering.
+int move_trajectory(beep_ctx* c, int* dev, int* host, int S, int X, bool to_host) {
+  const auto& m = c->m;
+  const size_t row = (size_t)X * m.AG, total = (size_t)S * row;
+  size_t steps = std::min<size_t>((size_t)S, std::max<size_t>(1, ((size_t)16 << 20) / (row * sizeof(int))));
+  if (total <= 4096) {
+    steps = 0;
+  } else if (ensure_scratch(c, steps * row * sizeof(int)) != BEEP_OK) {
+    steps = c->scratch_cap / (row * sizeof(int));
+    (void)hipGetLastError();
+  }
+  if (steps == 0) {
+    std::vector<int> h(total);
+    if (to_host) {
+      HIPCHK(c, hipMemcpyAsync(h.data(), dev, total * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+      HIPCHK(c, hipStreamSynchronize(c->stream));
+    }
+    for (int s = 0; s < S; s++)
+      for (int a = 0; a < m.A; a++)
+        for (int x = 0; x < X; x++)
+          for (int g = 0; g < m.G; g++) {
+            int& o = host[(((size_t)s * m.A + a) * X + x) * m.G + g];
+            int& i = h[((size_t)s * X + x) * m.AG + a * m.G + g];
+            if (to_host) o = i;
+            else i = o;
+          }
+    if (!to_host) {
+      HIPCHK(c, hipMemcpyAsync(dev, h.data(), total * sizeof(int), hipMemcpyHostToDevice, c->stream));
+      HIPCHK(c, hipStreamSynchronize(c->stream));
+    }
+    return BEEP_OK;
+  }
+  int* stage = (int*)c->d_scratch;
+  for (size_t s0 = 0; s0 < (size_t)S; s0 += steps) {
+    const size_t n = std::min(steps, (size_t)S - s0) * row;
+    if (!to_host) HIPCHK(c, hipMemcpyAsync(stage, host + s0 * row, n * sizeof(int), hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(beepdev::k_reorder, dim3((unsigned)std::min<size_t>((n + 255) / 256, 65535)), dim3(256), 0,
+                       c->stream, stage, dev + s0 * row, n, m.A, X, m.G, to_host ? 1 : 0);
+    HIPCHK(c, hipGetLastError());
+    if (to_host) HIPCHK(c, hipMemcpyAsync(host + s0 * row, stage, n * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  }
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return BEEP_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
 int beep_get_transnum(beep_ctx* c, int inst, int32_t* out) {
   if (!c || !valid_inst(c, inst) || !out || !c->d_tn) return fail(c, BEEP_EINVAL, "beep_get_transnum: bad arguments");
-  const auto& m = c->m;
-  std::vector<int> h(c->traj_sz);
-  HIPCHK(c, hipMemcpyAsync(h.data(), c->d_tn + (size_t)inst * c->traj_sz, c->traj_sz * sizeof(int),
-                           hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int s = 0; s < m.S; s++)
-    for (int a = 0; a < m.A; a++)
-      for (int t = 0; t < m.T; t++)
-        for (int g = 0; g < m.G; g++)
-          out[(((size_t)s * m.A + a) * m.T + t) * m.G + g] = h[((size_t)s * m.T + t) * m.AG + a * m.G + g];
-  return BEEP_OK;
+  return move_trajectory(c, c->d_tn + (size_t)inst * c->traj_sz, out, c->m.S, c->m.T, true);
 }
 
 int beep_get_transmean(beep_ctx* c, int inst, float* out) {
   if (!c || !valid_inst(c, inst) || !out || !c->d_tm) return fail(c, BEEP_EINVAL, "beep_get_transmean: bad arguments");
-  const auto& m = c->m;
-  std::vector<float> h(c->traj_sz);
-  HIPCHK(c, hipMemcpyAsync(h.data(), c->d_tm + (size_t)inst * c->traj_sz, c->traj_sz * sizeof(float),
-                           hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int s = 0; s < m.S; s++)
-    for (int a = 0; a < m.A; a++)
-      for (int t = 0; t < m.T; t++)
-        for (int g = 0; g < m.G; g++)
-          out[(((size_t)s * m.A + a) * m.T + t) * m.G + g] = h[((size_t)s * m.T + t) * m.AG + a * m.G + g];
-  return BEEP_OK;
+  return move_trajectory(c, (int*)(c->d_tm + (size_t)inst * c->traj_sz), (int*)out, c->m.S, c->m.T, true);
 }
 
 int beep_get_pop(beep_ctx* c, int inst, int32_t* out) {
   if (!c || !valid_inst(c, inst) || !out || !c->d_pt) return fail(c, BEEP_EINVAL, "beep_get_pop: bad arguments");
-  const auto& m = c->m;
-  std::vector<int> h(c->pop_traj_sz);
-  HIPCHK(c, hipMemcpyAsync(h.data(), c->d_pt + (size_t)inst * c->pop_traj_sz, c->pop_traj_sz * sizeof(int),
-                           hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int s = 0; s < m.S; s++)
-    for (int a = 0; a < m.A; a++)
-      for (int co = 0; co < m.C; co++)
-        for (int g = 0; g < m.G; g++)
-          out[(((size_t)s * m.A + a) * m.C + co) * m.G + g] = h[((size_t)s * m.C + co) * m.AG + a * m.G + g];
-  return BEEP_OK;
+  return move_trajectory(c, c->d_pt + (size_t)inst * c->pop_traj_sz, out, c->m.S, c->m.C, true);
 }
 
 int beep_get_state(beep_ctx* c, int inst, int32_t* out) {
@@ -1628,17 +1656,10 @@ int beep_put_transnum(beep_ctx* c, int inst, int slot, const int32_t* tn) {
   if (!c || !valid_inst(c, inst) || !tn || !c->d_tn) return fail(c, BEEP_EINVAL, "beep_put_transnum: bad arguments");
   if (!valid_slot(c, slot) || !c->slot_set[slot]) return fail(c, BEEP_EINVAL, "slot %d not set", slot);
   const auto& m = c->m;
-  std::vector<int> h(c->traj_sz);
-  for (int s = 0; s < m.S; s++)
-    for (int a = 0; a < m.A; a++)
-      for (int t = 0; t < m.T; t++)
-        for (int g = 0; g < m.G; g++)
-          h[((size_t)s * m.T + t) * m.AG + a * m.G + g] = tn[(((size_t)s * m.A + a) * m.T + t) * m.G + g];
-  HIPCHK(c, hipMemcpyAsync(c->d_tn + (size_t)inst * c->traj_sz, h.data(), c->traj_sz * sizeof(int),
-                           hipMemcpyHostToDevice, c->stream));
+  int rc;
+  if ((rc = move_trajectory(c, c->d_tn + (size_t)inst * c->traj_sz, const_cast<int32_t*>(tn), m.S, m.T, false))) return rc;
   std::vector<Job> jobs(1, make_job(c, inst, slot, 0, 0, m.S));
   jobs[0].mode = beepdev::MODE_REPLAY;
-  int rc;
   if ((rc = put_jobs(c, jobs))) return rc;
   if (c->stepwise) rc = launch_stepwise(c, beepdev::MODE_REPLAY, c->d_jobs, 1, 0, m.S, 0, 0);
   else rc = launch_fused(c, beepdev::MODE_REPLAY, c->d_jobs, 1, 0, 0);

@@ -500,6 +500,25 @@ __global__ void __launch_bounds__(256) k_copy_rows(V* __restrict__ base, size_t 
   for (size_t k = blockIdx.y * blockDim.x + threadIdx.x; k < row; k += (size_t)gridDim.y * blockDim.x) d_[k] = s_[k];
 }
 
+// Rows of a step between the reference's order [area][x][group] (`outer`) and
+// the device's [x][area * group]: element k of steps' outer order is outer[k],
+// its place in the device order inner[...]; to_outer says which side is
+// written.  Consecutive lanes take consecutive outer elements.  X = transitions
+// or compartments; grid over the elements of the steps.  On the host these
+// loops took 1-1.5 ms per 640,000-element trajectory.
+__global__ void __launch_bounds__(256) k_reorder(int* __restrict__ outer, int* __restrict__ inner, size_t n, int A, int X,
+                                                 int G, int to_outer) {
+  const size_t row = (size_t)A * X * G;
+  for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (size_t)gridDim.x * blockDim.x) {
+    const size_t s = k / row;
+    const uint32_t e = (uint32_t)(k - s * row);
+    const uint32_t g = e % (uint32_t)G, ax = e / (uint32_t)G, x = ax % (uint32_t)X, a = ax / (uint32_t)X;
+    const size_t i = s * row + ((size_t)x * A + a) * G + g;
+    if (to_outer) outer[k] = inner[i];
+    else inner[i] = outer[k];
+  }
+}
+
 // Parameter slots written from a packed upload: tab[slot[i]] = packed[i]
 // (n blocks of `stride` floats); grid (n, chunks): slot on x.
 __global__ void k_scatter_slots(float* __restrict__ tab, size_t stride, const float* __restrict__ packed,
