@@ -11,7 +11,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libbeep_gpu.so")
 SOURCES = ["beep_gpu.hip", "host_model.cc", "host/gpu_state.cc"]
-HEADERS = ["device_rng.hh", "fused_common.hh", "fused_spec.hh", "step_spec.hh", "kernels.hh", "obs_kernels.hh", "pmcmc_kernels.hh",
+HEADERS = ["device_rng.hh", "fused_common.hh", "fused_spec.hh", "step_spec.hh", "kernels.hh", "obs_kernels.hh", "pmcmc_kernels.hh", "replay_kernels.hh",
            "step_kernels.hh", "host_model.hh", "host/gpu_state.hh"]
 # Headers the library compiles at run time (hiprtc) for each compartment
 # structure, embedded as string constants.

@@ -25,6 +25,7 @@
 #include "kernels.hh"
 #include "obs_kernels.hh"
 #include "pmcmc_kernels.hh"
+#include "replay_kernels.hh"
 #include "step_kernels.hh"
 // kJitDeviceRng, kJitFusedCommon, kJitFusedSpec, kJitStepSpec: the texts of
 // device_rng.hh, fused_common.hh, fused_spec.hh and step_spec.hh (generated
@@ -1658,9 +1659,29 @@ int beep_put_transnum(beep_ctx* c, int inst, int slot, const int32_t* tn) {
   const auto& m = c->m;
   int rc;
   if ((rc = move_trajectory(c, c->d_tn + (size_t)inst * c->traj_sz, const_cast<int32_t*>(tn), m.S, m.T, false))) return rc;
-  std::vector<Job> jobs(1, make_job(c, inst, slot, 0, 0, m.S));
-  jobs[0].mode = beepdev::MODE_REPLAY;
-  if ((rc = put_jobs(c, jobs))) return rc;
+  Job job = make_job(c, inst, slot, 0, 0, m.S);
+  if (!c->stepwise && m.nstrain == 1) {
+    // Steps side by side; the populations go to the kept trajectory or else to
+    // scratch (without room for them, step by step below).
+    int* pop = job.pt;
+    if (!pop && ensure_scratch(c, c->pop_traj_sz * sizeof(int)) == BEEP_OK) pop = (int*)c->d_scratch;
+    if (pop) {
+      hipLaunchKernelGGL(beepdev::k_replay_pops, dim3((unsigned)((m.AG + 63) / 64), (unsigned)m.C), dim3(64), 0, c->stream,
+                         job.topo, (const int*)job.tn, pop, job.state);
+      HIPCHK(c, hipGetLastError());
+      const size_t lds = (size_t)8 * m.AG;
+      if (lds > 65536)
+        HIPCHK(c, hipFuncSetAttribute((const void*)beepdev::k_replay_means, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      const unsigned block = (unsigned)std::min(512, (m.AG + 63) / 64 * 64);
+      hipLaunchKernelGGL(beepdev::k_replay_means, dim3((unsigned)m.S), dim3(block), lds, c->stream, job.topo, job.tab,
+                         (const int*)pop, job.tm, job.err);
+      HIPCHK(c, hipGetLastError());
+      return check_device_error(c);
+    }
+    (void)hipGetLastError();
+  }
+  job.mode = beepdev::MODE_REPLAY;
+  if ((rc = put_jobs(c, std::vector<Job>(1, job)))) return rc;
   if (c->stepwise) rc = launch_stepwise(c, beepdev::MODE_REPLAY, c->d_jobs, 1, 0, m.S, 0, 0);
   else rc = launch_fused(c, beepdev::MODE_REPLAY, c->d_jobs, 1, 0, 0);
   if (rc) return rc;

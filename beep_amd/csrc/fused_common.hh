@@ -109,6 +109,13 @@ typedef const __attribute__((address_space(4))) TopoDev ctopo;
 // I are the mixing arrays' element types, qualified with the address space
 // they are read from (LDS when staged).
 //
+// The two terms' roundings are fixed (mix_value), so that every kernel and
+// compiler computes the same FP32 value from the same row sum.
+__device__ inline float mix_value(float diag, float fac, float dinf, float imp, float m) {
+  const float idg = diag * dinf;
+  return __builtin_fmaf(__builtin_fmaf(diag, dinf, imp), m, fac * idg * (1.f - m));
+}
+
 // Lanes take areas in the order `order` (most incoming entries first), so
 // the areas of one wavefront have similar row lengths and the gather loop,
 // whose trip count is the wavefront's longest row, wastes few iterations.
@@ -120,7 +127,6 @@ __device__ inline void mix_cells(F* diag, F* fac, I* in_ptr, I* in_src, F* in_w,
   for (int t = tid; t < AG; t += nt) {
     const int jo = t / G, g = t - jo * G;
     const int j = order[jo], cell = j * G + g;
-    float idg = diag[j] * sdinf[cell];
     float imp = 0.f;
     int e = in_ptr[j];
     const int e1 = in_ptr[j + 1];
@@ -128,13 +134,13 @@ __device__ inline void mix_cells(F* diag, F* fac, I* in_ptr, I* in_src, F* in_w,
       const int s0 = in_src[e], s1 = in_src[e + 1], s2 = in_src[e + 2], s3 = in_src[e + 3];
       const float w0 = in_w[e], w1 = in_w[e + 1], w2 = in_w[e + 2], w3 = in_w[e + 3];
       const float d0 = sdinf[s0 * G + g], d1 = sdinf[s1 * G + g], d2 = sdinf[s2 * G + g], d3 = sdinf[s3 * G + g];
-      imp += w0 * d0;
-      imp += w1 * d1;
-      imp += w2 * d2;
-      imp += w3 * d3;
+      imp = __builtin_fmaf(w0, d0, imp);
+      imp = __builtin_fmaf(w1, d1, imp);
+      imp = __builtin_fmaf(w2, d2, imp);
+      imp = __builtin_fmaf(w3, d3, imp);
     }
-    for (; e < e1; e++) imp += in_w[e] * sdinf[in_src[e] * G + g];
-    sI[cell] = (idg + imp) * m + fac[j] * idg * (1.f - m);
+    for (; e < e1; e++) imp = __builtin_fmaf(in_w[e], sdinf[in_src[e] * G + g], imp);
+    sI[cell] = mix_value(diag[j], fac[j], sdinf[cell], imp, m);
   }
 }
 
