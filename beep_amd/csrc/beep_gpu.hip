@@ -499,7 +499,8 @@ int launch_stepwise(beep_ctx* c, int mode, const Job* djobs, int n, int t0, int 
   hipGraph_t graph;
   (void)hipGetLastError();               // a stale error of an earlier call is not this loop's
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  hipLaunchKernelGGL(beepdev::k_step_init, gcell, dim3(BEEP_STEP_BLOCK), 0, c->stream, djobs, c->d_D, c->Apad);
+  hipLaunchKernelGGL(beepdev::k_step_init, gcell, dim3(BEEP_STEP_BLOCK), 0, c->stream, djobs, c->d_D, c->Apad,
+                     c->spec && c->d_pt ? 1 : 0);
   for (int s = t0; s < t1; s++) {
     if (c->dense) {
       beepdev::DenseMix p{c->d_D, c->d_M, c->d_I, c->h_topo.diag, c->h_topo.fac, djobs, rows, m.A, c->Apad, m.G, s,

@@ -81,11 +81,13 @@ __device__ inline void st_nt(float* p, uint32_t i, float v) { __builtin_nontempo
 // One step's slab of an instance's trajectory as a buffer: a store's address is
 // the slab's base, a scalar offset (the row of a transition or compartment)
 // and the lane's byte offset, and the hardware drops a store whose lane offset
-// lies past the slab, so a lane opts out without a branch.
+// lies past the slab, so a lane opts out without a branch.  Plain stores, not
+// non-temporal ones: step-wise simulation of 512 x 2853 cells x 300 steps takes
+// 33.6 ms with them, 34.2 without; the fused kernel shows no difference.
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ inline rsrc_t slab(void* p, uint32_t bytes) { return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00020000); }
 __device__ inline void st_slab(rsrc_t r, int v, uint32_t lane_off, uint32_t row_off) {
-  __builtin_amdgcn_raw_buffer_store_b32(v, r, (int)lane_off, (int)row_off, 2);       // 2: non-temporal
+  __builtin_amdgcn_raw_buffer_store_b32(v, r, (int)lane_off, (int)row_off, 0);
 }
 
 // Pointers typed by address space.  A plain pointer read out of a job

@@ -215,8 +215,11 @@ __global__ void __launch_bounds__(256) k_sparse_contract(SparseMix p) {
 
 // Start of a step-wise run: the state at t0 (the spec's initial populations
 // when t0 == 0) and its infectivity D[(b,g)][j] = sum_c inf_c pop_c.
-// Grid (nb, ceil(AG/256)): job on x, block of cells on y.
-__global__ void __launch_bounds__(256) k_step_init(const Job* __restrict__ jobs, float* __restrict__ D, int Apad) {
+// With to_traj the populations go to the kept trajectory's step t0, where the
+// specialised transition kernel reads them.  Grid (nb, ceil(AG/256)): job on x,
+// block of cells on y.
+__global__ void __launch_bounds__(256) k_step_init(const Job* __restrict__ jobs, float* __restrict__ D, int Apad,
+                                                   int to_traj) {
   const Job jb = jobs[blockIdx.x];
   ctopo* tp = (ctopo*)jb.topo;
   const int AG = tp->AG, C = tp->C, G = tp->G;
@@ -227,6 +230,7 @@ __global__ void __launch_bounds__(256) k_step_init(const Job* __restrict__ jobs,
   for (int c = 0; c < C; c++) {
     int v = jb.from_init ? gptr(tp->pop_init)[c * AG + cell] : state[c * AG + cell];
     if (jb.from_init) state[c * AG + cell] = v;
+    if (to_traj && jb.t0 < tp->S) ((gint*)jb.pt)[((size_t)jb.t0 * C + c) * AG + cell] = v;
     float w = gptr(jb.tab)[tp->off_inf + c];
     if (w != 0.f) d += w * (float)v;
   }
