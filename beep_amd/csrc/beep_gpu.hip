@@ -567,10 +567,18 @@ int launch_fused(beep_ctx* c, int mode, const Job* djobs, int njobs, uint64_t se
   return launch_fused_t<beepdev::MODE_REPLAY>(c, djobs, njobs, lds, block, seed, stream);
 }
 
-// The observation log-likelihood of n instances over the observations sel
-// (all when null), into out[b * (1 + ndatatable)].
-void launch_obs_loglik(beep_ctx* c, int n, const int* d_inst, const int* sel, int nsel, double* out, int store_EF,
-                       bool want_dt, hipStream_t st = nullptr) {
+// Chunks of a section's nsel observations (k_obs_loglik without data tables; the
+// chunks are the grid's second dimension).
+int section_chunks(int nsel) {
+  const int k = std::max(1, (nsel + BEEP_OBS_CHUNK - 1) / BEEP_OBS_CHUNK);
+  return k <= 65535 ? k : 1;
+}
+
+// The observation log-likelihood of n instances over the nsel observations
+// sel, in nchunk chunks (1: the whole list): into out[c * n + b], or with
+// want_dt (one chunk) the data tables' sums too, into out[b * (1 + ndatatable)].
+void launch_obs_loglik(beep_ctx* c, int n, const int* d_inst, const int* sel, int nsel, int nchunk, double* out,
+                       bool want_dt) {
   using K = decltype(&beepdev::k_obs_loglik<true, true, true, false>);
   // With observation splines only the general variants are used.
   static const K ks[12] = {
@@ -586,9 +594,17 @@ void launch_obs_loglik(beep_ctx* c, int n, const int* d_inst, const int* sel, in
   // Per-table sums: one pass per eight data tables.
   const int npass = want_dt ? (c->m.ndatatable + 7) / 8 : 1;
   for (int p = 0; p < npass; p++)
-    hipLaunchKernelGGL(k, dim3((n + ni - 1) / ni), dim3(256), 0, st ? st : c->stream, c->d_obs, n, d_inst, c->d_tn,
-                       c->d_pt, c->traj_sz, c->pop_traj_sz, sel, nsel, out, c->d_EF, store_EF, c->d_ospl,
-                       c->d_inst_slot, 8 * p);
+    hipLaunchKernelGGL(k, dim3((n + ni - 1) / ni, (unsigned)nchunk), dim3(256), 0, c->stream, c->d_obs, n, d_inst,
+                       c->d_tn, c->d_pt, c->traj_sz, c->pop_traj_sz, sel, nsel,
+                       nchunk > 1 ? BEEP_OBS_CHUNK : std::max(1, nsel), out, c->d_ospl, c->d_inst_slot, 8 * p);
+}
+
+// A section's bootstrap, its work arrays in LDS where they fit.
+void launch_bootstrap(hipStream_t st, int n, const double* d_L, int nchunk, double invT, uint64_t seed, uint32_t stream,
+                      int sec, int* bp, double* d_w, int* d_first, int* d_draw, int* d_extra, double* d_ob, int* d_err) {
+  const auto k = n <= BEEP_BOOT_LDS ? beepdev::k_bootstrap<true> : beepdev::k_bootstrap<false>;
+  hipLaunchKernelGGL(k, dim3(1), dim3(BEEP_BOOT_BLOCK), 0, st, n, d_L, nchunk, invT, seed, stream, sec, bp, d_w, d_first,
+                     d_draw, d_extra, d_ob, d_err);
 }
 
 // Before an observation kernel reads inst_slot: the host copy, uploaded when
@@ -1437,19 +1453,21 @@ int beep_obs_loglik(beep_ctx* c, int n, const int32_t* inst, int section, double
     return BEEP_OK;
   }
   const int ndt = c->m.ndatatable;
-  size_t out_doubles = (size_t)n * (1 + ndt);
-  if ((rc = ensure_scratch(c, out_doubles * sizeof(double) + (size_t)n * sizeof(int)))) return rc;
+  const int nsel = c->sec_ptr[section + 1] - c->sec_ptr[section];
+  int nchunk = EF_dt_out ? 1 : section_chunks(nsel);
+  auto doubles = [&] { return EF_dt_out ? (size_t)n * (1 + ndt) : (size_t)n * nchunk; };
+  rc = ensure_scratch(c, doubles() * sizeof(double) + (size_t)n * sizeof(int));
+  if (rc && nchunk > 1) {
+    nchunk = 1;
+    rc = ensure_scratch(c, doubles() * sizeof(double) + (size_t)n * sizeof(int));
+  }
+  if (rc) return rc;
+  const size_t out_doubles = doubles();
   double* d_out = (double*)c->d_scratch;
   int* d_inst = (int*)(d_out + out_doubles);
   HIPCHK(c, hipMemcpyAsync(d_inst, inst, n * sizeof(int), hipMemcpyHostToDevice, c->stream));
-  const int* sobs = nullptr;
-  int nsel = c->m.obs.size();
-  if (section >= 0) {
-    sobs = c->d_sec_obs + c->sec_ptr[section];
-    nsel = c->sec_ptr[section + 1] - c->sec_ptr[section];
-  }
   record(c, 2);
-  launch_obs_loglik(c, n, d_inst, sobs, nsel, d_out, section < 0 ? 1 : 0, EF_dt_out != nullptr);
+  launch_obs_loglik(c, n, d_inst, c->d_sec_obs + c->sec_ptr[section], nsel, nchunk, d_out, EF_dt_out != nullptr);
   HIPCHK(c, hipGetLastError());
   record(c, 3);
   std::vector<double> h(out_doubles);
@@ -1457,10 +1475,12 @@ int beep_obs_loglik(beep_ctx* c, int n, const int32_t* inst, int section, double
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->timing[1] = elapsed(c, 2, 3);
   for (int i = 0; i < n; i++) {
-    L_out[i] = h[(size_t)i * (1 + ndt)];
+    const size_t row = EF_dt_out ? 1 + ndt : 1;
+    L_out[i] = h[i * row];
+    for (int k = 1; k < nchunk; k++) L_out[i] += h[(size_t)k * n + i];
     if (std::isnan(L_out[i])) return fail(c, BEEP_ENAN, "NaN observation log-likelihood");   // obsmodel.cc:32
     if (EF_dt_out)
-      for (int d = 0; d < ndt; d++) EF_dt_out[(size_t)i * ndt + d] = h[(size_t)i * (1 + ndt) + 1 + d];
+      for (int d = 0; d < ndt; d++) EF_dt_out[(size_t)i * ndt + d] = h[i * row + 1 + d];
   }
   return BEEP_OK;
 }
@@ -1884,16 +1904,24 @@ int beep_pmcmc_obs_prob(beep_ctx* c, int n, const int32_t* inst, int slot, const
   for (int i = 0; i < n; i++) head[i] = i;
   HIPCHK(c, hipMemcpyAsync(d_bp, head.data(), n * sizeof(int), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(d_inst, inst, n * sizeof(int), hipMemcpyHostToDevice, c->stream));
-  // Scratch: L rows, bootstrap work arrays, the estimate.
-  const int Lstride = 1 + m.ndatatable;
-  size_t bytes = (size_t)n * Lstride * sizeof(double) + (size_t)n * sizeof(double) + 3 * (size_t)n * sizeof(int) + 64;
-  if ((rc = ensure_scratch(c, bytes))) return rc;
+  // Scratch: the estimate, the chunk sums of the longest section, the
+  // bootstrap's work arrays.  Where the chunks do not fit, one chunk.
+  int maxsel = 0;
+  for (int k = 0; k < nsec; k++) maxsel = std::max(maxsel, c->sec_ptr[k + 1] - c->sec_ptr[k]);
+  bool chunked = section_chunks(maxsel) > 1;
+  auto bytes = [&](int nchunk) { return (size_t)n * (nchunk + 1) * sizeof(double) + (3 * (size_t)n * sizeof(int) + 71) / 8 * 8; };
+  rc = ensure_scratch(c, bytes(section_chunks(maxsel)));
+  if (rc && chunked) {
+    chunked = false;
+    rc = ensure_scratch(c, bytes(1));
+  }
+  if (rc) return rc;
   double* d_ob = (double*)c->d_scratch;
-  double* d_L = d_ob + 1;
-  double* d_w = d_L + (size_t)n * Lstride;
+  double* d_w = d_ob + 1;
   int* d_first = (int*)(d_w + n);
   int* d_draw = d_first + n;
   int* d_extra = d_draw + n;
+  double* d_L = (double*)((char*)c->d_scratch + bytes(0));
   HIPCHK(c, hipMemsetAsync(d_ob, 0, sizeof(double), c->stream));
   // Jobs of every section.
   std::vector<Job> jobs;
@@ -1915,10 +1943,11 @@ int beep_pmcmc_obs_prob(beep_ctx* c, int n, const int32_t* inst, int slot, const
     else rc = launch_fused(c, beepdev::MODE_SIM, dj, n, seed, stream);
     if (rc) return rc;
     const int nsel = c->sec_ptr[k + 1] - c->sec_ptr[k];
-    launch_obs_loglik(c, n, d_inst, c->d_sec_obs + c->sec_ptr[k], nsel, d_L, 0, false);
+    const int nchunk = chunked ? section_chunks(nsel) : 1;
+    launch_obs_loglik(c, n, d_inst, c->d_sec_obs + c->sec_ptr[k], nsel, nchunk, d_L, false);
     HIPCHK(c, hipGetLastError());
-    hipLaunchKernelGGL(beepdev::k_bootstrap, dim3(1), dim3(BEEP_BOOT_BLOCK), 0, c->stream, n, d_L, Lstride, invT, seed,
-                       stream, k, d_bp + (size_t)(k + 1) * n, d_w, d_first, d_draw, d_extra, d_ob, c->d_err);
+    launch_bootstrap(c->stream, n, d_L, nchunk, invT, seed, stream, k, d_bp + (size_t)(k + 1) * n, d_w, d_first, d_draw,
+                     d_extra, d_ob, c->d_err);
     HIPCHK(c, hipGetLastError());
   }
   record(c, 1);
@@ -2069,8 +2098,7 @@ int beep_bootstrap(int device, int n, const double* L, double invT, uint64_t see
   if (hipMemset(d, 0, 16) != hipSuccess || hipMemcpy(d_L, L, n * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
     rc = BEEP_EHIP;
   if (!rc) {
-    hipLaunchKernelGGL(beepdev::k_bootstrap, dim3(1), dim3(BEEP_BOOT_BLOCK), 0, 0, n, d_L, 1, invT, seed, stream, sec,
-                       d_bp, d_w, d_first, d_draw, d_extra, d_ob, d_err);
+    launch_bootstrap(nullptr, n, d_L, 1, invT, seed, stream, sec, d_bp, d_w, d_first, d_draw, d_extra, d_ob, d_err);
     if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) rc = BEEP_EHIP;
   }
   if (!rc && (hipMemcpy(bp_out, d_bp, n * sizeof(int), hipMemcpyDeviceToHost) != hipSuccess ||

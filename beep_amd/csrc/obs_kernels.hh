@@ -133,23 +133,28 @@ __device__ inline void obs_terms(const ObsDev& od, const int* __restrict__ sel, 
                                  const int* (&tnb)[NI], const int* (&ptb)[NI], const double* (&splv)[NI],
                                  double (&L)[NI], double (&acc)[8]);
 
-// One workgroup per OBS_INSTANCES instances.  out[b*(1+ndt)] = log-likelihood,
-// out[b*(1+ndt)+1+d] = -2 * (sum over data table d)  (get_EF_datatable),
-// written when WANT_DT.  The counts of an observation are summed as
-// integers and scaled by its factor once; normal terms use the per-
-// observation constants lc and iv.  GENERAL: the model has observations
-// other than plain normal ones (Poisson, negative binomial, thresholds,
-// unknowns); without it the kernel holds only the normal path, which keeps
-// its register use, and so its occupancy, low.  POP: some observation counts
-// population elements.  SPL: some observations carry an observation spline;
-// their counts are weighted per step by the values of the instance's slot,
-// ospl_tab + inst_slot[instance] * nospl * S.
+// One workgroup per OBS_INSTANCES instances and chunk of the list sel, of
+// `chunk` observations (chunk blockIdx.y): the particle filter's sections.
+// Bound by the gathers (nine counts to an observation, 36 bytes apart by lane):
+// 512 instances x 9,510 observations 98 us, 178 us as one chunk, which left half
+// the device idle (128 workgroups).  Without WANT_DT out[c * n + b] is
+// instance b's sum over chunk c, and the reader adds the chunks in order.  With
+// it the grid has one chunk, out[b*(1+ndt)] = log-likelihood, and
+// out[b*(1+ndt)+1+d] = -2 * (sum over data table d)  (get_EF_datatable).  The
+// counts of an observation are summed as integers and scaled by its factor
+// once; normal terms use the per-observation constants lc and iv.  GENERAL:
+// the model has observations other than plain normal ones (Poisson, negative
+// binomial, thresholds, unknowns); without it the kernel holds only the normal
+// path, which keeps its register use, and so its occupancy, low.  POP: some
+// observation counts population elements.  SPL: some observations carry an
+// observation spline; their counts are weighted per step by the values of the
+// instance's slot, ospl_tab + inst_slot[instance] * nospl * S.
 template <bool WANT_DT, bool GENERAL, bool POP, bool SPL>
 __global__ void __launch_bounds__(256) k_obs_loglik(const ObsDev* __restrict__ odp, int n, const int* __restrict__ inst,
                                                     const int* __restrict__ tn, const int* __restrict__ pt,
                                                     size_t traj_sz, size_t pop_traj_sz, const int* __restrict__ sel,
-                                                    int nsel, double* __restrict__ out, double* __restrict__ EF,
-                                                    int store_EF, const double* __restrict__ ospl_tab,
+                                                    int nsel, int chunk, double* __restrict__ out,
+                                                    const double* __restrict__ ospl_tab,
                                                     const int* __restrict__ inst_slot, int d0) {
   // Instances per workgroup: they share the observation structure, so one
   // thread reads an observation's elements once and gathers the counts of
@@ -158,6 +163,7 @@ __global__ void __launch_bounds__(256) k_obs_loglik(const ObsDev* __restrict__ o
   __shared__ double red[8];
   const ObsDev od = *odp;
   const int b0 = blockIdx.x * NI;
+  const int kbeg = (int)blockIdx.y * chunk, kend = min(nsel, kbeg + chunk);
   int ins[NI];
   const int* tnb[NI];
   const int* ptb[NI];
@@ -171,19 +177,17 @@ __global__ void __launch_bounds__(256) k_obs_loglik(const ObsDev* __restrict__ o
 #pragma unroll
   for (int q = 0; q < NI; q++) splv[q] = SPL ? ospl_tab + (size_t)inst_slot[ins[q]] * od.nospl * od.S : nullptr;
   double L[NI], acc[8];
-  obs_terms<WANT_DT, GENERAL, POP, SPL, NI>(od, sel, 0, nsel, d0, tnb, ptb, splv, L, acc);
+  obs_terms<WANT_DT, GENERAL, POP, SPL, NI>(od, sel, kbeg, kend, d0, tnb, ptb, splv, L, acc);
+  const size_t row = WANT_DT ? 1 + (size_t)od.ndt : 1;
 #pragma unroll
   for (int q = 0; q < NI; q++) {
     const double Lt = block_sum(L[q], red);
-    if (threadIdx.x == 0 && b0 + q < n && d0 == 0) {
-      out[(size_t)(b0 + q) * (1 + od.ndt)] = Lt;
-      if (store_EF) EF[ins[q]] = -2.0 * Lt;
-    }
+    if (threadIdx.x == 0 && b0 + q < n && d0 == 0) out[(size_t)blockIdx.y * n + (size_t)(b0 + q) * row] = Lt;
   }
   if (WANT_DT) {
     // Data tables d0 .. d0 + 7 in this pass (the launcher makes one pass per
     // eight tables; the total above is written by the first).
-    double* o = out + (size_t)b0 * (1 + od.ndt);
+    double* o = out + (size_t)b0 * row;
     const int nd = min(8, od.ndt - d0);
     for (int d = 0; d < nd; d++) {
       double t = block_sum(acc[d], red);
