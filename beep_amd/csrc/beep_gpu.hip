@@ -94,6 +94,8 @@ struct beep_ctx {
   float* d_D = nullptr;            // [capacity*G padded to 64][Apad], fragment order
   float* d_I = nullptr;            // [capacity*G][Apad]
   uint64_t* d_rngp = nullptr;      // seed, stream read by the captured step kernels
+  uint64_t rng[2] = {0, 0};        // what d_rngp holds, once rng_set
+  bool rng_set = false;
   struct Graph {
     int mode = -1, n = 0, t0 = 0, t1 = 0;
     const Job* jobs = nullptr;
@@ -212,6 +214,7 @@ std::vector<float> to_f32(const std::vector<double>& v) { return std::vector<flo
 int ensure_jobs(beep_ctx* c, size_t n) {
   if (n <= c->jobs_cap) return BEEP_OK;
   if (c->d_jobs) {
+    HIPCHK(c, hipStreamSynchronize(c->stream));   // graphs of a call that failed halfway may still run
     for (auto& g : c->graphs)     // captured graphs refer to the old job buffer
       if (g.jobs >= c->d_jobs && g.jobs < c->d_jobs + c->jobs_cap) {
         HIPCHK(c, hipGraphExecDestroy(g.exec));
@@ -475,9 +478,17 @@ int launch_stepwise(beep_ctx* c, int mode, const Job* djobs, int n, int t0, int 
   // reads them there at every replay.
   if (!c->d_jobs || djobs < c->d_jobs || djobs + n > c->d_jobs + c->jobs_cap)
     return fail(c, BEEP_EINVAL, "step-wise launch: job descriptors outside the context's job buffer");
-  uint64_t rp[2] = {seed, (uint64_t)stream};
-  HIPCHK(c, hipMemcpyAsync(c->d_rngp, rp, sizeof rp, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  // Uploaded when the device's copy (written only here) holds other values: the
+  // sections of a particle filter then queue one behind the other, where a wait
+  // at each left the device idle for a graph launch (ten sections: 0.2 ms of 33).
+  if (!c->rng_set || c->rng[0] != seed || c->rng[1] != stream) {
+    c->rng_set = false;
+    c->rng[0] = seed;
+    c->rng[1] = stream;
+    HIPCHK(c, hipMemcpyAsync(c->d_rngp, c->rng, sizeof c->rng, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->rng_set = true;
+  }
   for (const auto& g : c->graphs)
     if (g.mode == mode && g.n == n && g.t0 == t0 && g.t1 == t1 && g.jobs == djobs) {
       // A cached graph is replayed only with the geometry it was captured with.
@@ -1923,12 +1934,17 @@ int beep_pmcmc_obs_prob(beep_ctx* c, int n, const int32_t* inst, int slot, const
   int* d_extra = d_draw + n;
   double* d_L = (double*)((char*)c->d_scratch + bytes(0));
   HIPCHK(c, hipMemsetAsync(d_ob, 0, sizeof(double), c->stream));
-  // Jobs of every section.
+  // Jobs of every section: the first section's are copied, the others are made
+  // of them on the device.
   std::vector<Job> jobs;
-  jobs.reserve((size_t)nsec * n);
-  for (int k = 0; k < nsec; k++)
-    for (int i = 0; i < n; i++) jobs.push_back(make_job(c, inst[i], slot, key[i], m.section_ti[k], m.section_tf[k]));
-  if ((rc = put_jobs(c, jobs))) return rc;
+  jobs.reserve((size_t)n);
+  for (int i = 0; i < n; i++) jobs.push_back(make_job(c, inst[i], slot, key[i], m.section_ti[0], m.section_tf[0]));
+  if ((rc = ensure_jobs(c, (size_t)nsec * n)) || (rc = put_jobs(c, jobs))) return rc;
+  if (nsec > 1) {
+    hipLaunchKernelGGL(beepdev::k_section_jobs, dim3((unsigned)((n + 255) / 256), (unsigned)(nsec - 1)), dim3(256), 0,
+                       c->stream, c->d_jobs, n, c->d_sec_ti, c->d_sec_tf);
+    HIPCHK(c, hipGetLastError());
+  }
   if ((rc = sync_inst_slot(c))) return rc;
   const unsigned mv_x = (unsigned)std::min<size_t>(16, (c->state_sz + 255) / 256);
   record(c, 0);
