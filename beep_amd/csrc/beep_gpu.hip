@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cstdlib>
 #include <fstream>
 #include <sstream>
@@ -2233,103 +2234,102 @@ int ensure_bstreams(beep_ctx* c0, size_t want, std::vector<hipStream_t>& out) {
 int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const std::vector<const int32_t*>& inst,
                        const std::vector<int>& ninst, bool store_EF, double* out, double* out_dt, int ev0) {
   hipStream_t st = c0->stream;
-  using beepdev::ObsGroup;
-  using beepdev::ObsItem;
+  using beepdev::ObsSet;
+  using beepdev::ObsSum;
   constexpr int GN = beepdev::OBS_GROUP;
-  size_t N = 0, NI = 0;                            // instances, and sums wanted
-  for (size_t k = 0; k < ctxs.size(); k++) {
-    N += (size_t)ninst[k];
-    NI += (size_t)ninst[k] * (out_dt ? 1 + ctxs[k]->m.ndatatable : 1);
+  // Sets and sums, and the chunks' ranges and tables of all of them one after
+  // the other; pointers into the staging are set once its layout is known.
+  const size_t nset = ctxs.size();
+  std::vector<ObsSum> sums(nset);
+  std::vector<size_t> range0(nset), tab0(nset);
+  std::vector<int2> range;
+  std::vector<int> tab;
+  long long N = 0, ND = 0, nparts = 0;
+  int max_ndt = 0;
+  for (size_t k = 0; k < nset; k++) {
+    const beep_ctx* c = ctxs[k];
+    ObsSum& su = sums[k];
+    range0[k] = range.size();
+    tab0[k] = tab.size();
+    su.ndt = out_dt ? c->m.ndatatable : 0;
+    for (int t = 0; t < (out_dt ? su.ndt : 1); t++) {
+      tab.push_back((int)(range.size() - range0[k]));
+      const int k1 = out_dt ? c->dt_ptr[t + 1] : c->obs.nobs;
+      for (int x = out_dt ? c->dt_ptr[t] : 0; x < k1; x += BEEP_OBS_CHUNK)
+        range.push_back(make_int2(x, std::min(k1, x + BEEP_OBS_CHUNK)));
+    }
+    su.nchunk = (int)(range.size() - range0[k]);
+    tab.push_back(su.nchunk);
+    su.part0 = (int)nparts;
+    su.out0 = (int)N;
+    su.dt0 = (int)ND;
+    N += ninst[k];
+    ND += (long long)ninst[k] * su.ndt;
+    nparts += ((long long)ninst[k] + GN - 1) / GN * su.nchunk;
+    max_ndt = std::max(max_ndt, su.ndt);
+    if (nparts > beephost::kGridMaxX || ND > INT_MAX)
+      return fail(c0, BEEP_EINVAL, "observation log-likelihood: too many chunks");
   }
   if (N == 0) return BEEP_OK;
-  // A context's lists of observations: all, or one per data table.
-  auto lists = [&](const beep_ctx* c) {
-    std::vector<std::pair<int, int>> r;
-    if (!out_dt) r.emplace_back(0, c->obs.nobs);
-    for (int d = 0; out_dt && d < c->m.ndatatable; d++) r.emplace_back(c->dt_ptr[d], c->dt_ptr[d + 1]);
-    return r;
-  };
-  auto chunks = [](const std::pair<int, int>& r) { return (r.second - r.first + BEEP_OBS_CHUNK - 1) / BEEP_OBS_CHUNK; };
-  // Group, partial and sum counts first, to lay out the staging.
-  size_t ngroups = 0, nparts = 0;
-  for (size_t k = 0; k < ctxs.size(); k++) {
-    const size_t ng = ((size_t)ninst[k] + GN - 1) / GN;
-    for (const auto& r : lists(ctxs[k])) {
-      ngroups += ng;
-      nparts += ng * chunks(r);
-    }
-  }
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-  const size_t b_inst = al(N * sizeof(int32_t)), b_groups = al(ngroups * sizeof(ObsGroup)),
-               b_items = al(NI * sizeof(ObsItem)), b_out = al(NI * sizeof(double));
-  const size_t b_part = al(nparts * GN * sizeof(double));
-  const size_t up = b_inst + b_groups + b_items;
+  const size_t b_inst = al(N * sizeof(int32_t)), b_sets = al(nset * sizeof(ObsSet)), b_sums = al(nset * sizeof(ObsSum)),
+               b_range = al(range.size() * sizeof(int2)), b_tab = al(tab.size() * sizeof(int));
+  const size_t up = b_inst + b_sets + b_sums + b_range + b_tab;
+  const size_t b_out = al((size_t)(N + ND) * sizeof(double)), b_part = al(nparts * GN * sizeof(double));
   int rc;
   if ((rc = ensure_scratch(c0, up + b_out + b_part))) return rc;
   char* d = (char*)c0->d_scratch;
   const int32_t* d_inst = (const int32_t*)d;
-  ObsGroup* d_groups = (ObsGroup*)(d + b_inst);
-  ObsItem* d_items = (ObsItem*)(d + b_inst + b_groups);
+  ObsSet* d_sets = (ObsSet*)(d + b_inst);
+  ObsSum* d_sums = (ObsSum*)(d + b_inst + b_sets);
+  const int2* d_range = (const int2*)(d + b_inst + b_sets + b_sums);
+  const int* d_tab = (const int*)(d + b_inst + b_sets + b_sums + b_range);
   double* d_out = (double*)(d + up);
   double* d_part = (double*)(d + up + b_out);
   std::vector<char> h(up, 0);
   int32_t* h_inst = (int32_t*)h.data();
-  ObsItem* h_items = (ObsItem*)(h.data() + b_inst + b_groups);
-  // Groups by kernel variant (general / population elements / splines), each
-  // variant's groups contiguous and numbered by workgroup from 0.  Sums: the
-  // instances' totals in order, then the tables of each instance in order.
-  std::vector<ObsGroup> byv[8];
+  // Sets by kernel variant (general / population elements / splines), each
+  // variant's contiguous and numbered by workgroup from 0; none without work.
+  std::vector<ObsSet> byv[8];
   long long wgs[8] = {};
-  size_t ii = 0, id = N;
-  int part = 0;
-  for (size_t k = 0; k < ctxs.size(); k++) {
+  for (size_t k = 0; k < nset; k++) {
     beep_ctx* c = ctxs[k];
+    ObsSum& su = sums[k];
+    su.inst = d_inst + su.out0;
+    su.EF = store_EF ? c->d_EF : nullptr;
+    su.tab = d_tab + tab0[k];
+    std::copy(inst[k], inst[k] + ninst[k], h_inst + su.out0);
+    if (ninst[k] == 0 || su.nchunk == 0) continue;
     const int v = (c->obs_general ? 4 : 0) | (c->obs_pop ? 2 : 0) | (c->nospl ? 1 : 0);
-    const auto ls = lists(c);
-    const size_t ndt = out_dt ? ls.size() : 0;
-    for (int g0 = 0; g0 < ninst[k]; g0 += GN) {
-      ObsGroup G;
-      std::memset(&G, 0, sizeof G);
-      G.od = c->obs;
-      G.tn = c->d_tn;
-      G.pt = c->d_pt;
-      G.ospl = c->nospl ? c->d_ospl : nullptr;
-      G.inst_slot = c->nospl ? c->d_inst_slot : nullptr;
-      G.inst = d_inst + ii;
-      G.sel = out_dt ? c->d_dt_obs : nullptr;
-      G.traj_sz = c->traj_sz;
-      G.pop_traj_sz = c->pop_traj_sz;
-      G.ninst = std::min(GN, ninst[k] - g0);
-      const int part0 = part;
-      for (size_t t = 0; t < ls.size(); t++) {
-        G.k0 = ls[t].first;
-        G.k1 = ls[t].second;
-        G.nchunk = chunks(ls[t]);
-        G.wg0 = (int)wgs[v];
-        G.part0 = part;
-        for (int q = 0; ndt && q < G.ninst; q++)
-          h_items[id + (size_t)q * ndt + t] = ObsItem{part, G.nchunk, q, -2.f, nullptr};
-        if (G.nchunk > 0) byv[v].push_back(G);
-        wgs[v] += G.nchunk;
-        part += G.nchunk;
-      }
-      for (int q = 0; q < G.ninst; q++) {
-        const int32_t in = inst[k][g0 + q];
-        h_inst[ii] = in;
-        h_items[ii] = ObsItem{part0, part - part0, q, 1.f, store_EF ? c->d_EF + in : nullptr};
-        ii++;
-      }
-      id += (size_t)G.ninst * ndt;
-    }
+    ObsSet S;
+    std::memset((void*)&S, 0, sizeof S);
+    S.od = c->obs;
+    S.tn = c->d_tn;
+    S.pt = c->d_pt;
+    S.ospl = c->nospl ? c->d_ospl : nullptr;
+    S.inst_slot = c->nospl ? c->d_inst_slot : nullptr;
+    S.inst = su.inst;
+    S.sel = out_dt ? c->d_dt_obs : nullptr;
+    S.range = d_range + range0[k];
+    S.traj_sz = c->traj_sz;
+    S.pop_traj_sz = c->pop_traj_sz;
+    S.ninst = ninst[k];
+    S.nchunk = su.nchunk;
+    S.part0 = su.part0;
+    S.wg0 = (int)wgs[v];
+    wgs[v] += ((long long)ninst[k] + GN - 1) / GN * su.nchunk;
+    byv[v].push_back(S);
   }
   size_t goff[8], gsum = 0;
   for (int v = 0; v < 8; v++) {
     goff[v] = gsum;
     if (!byv[v].empty())
-      std::memcpy(h.data() + b_inst + gsum * sizeof(ObsGroup), byv[v].data(), byv[v].size() * sizeof(ObsGroup));
+      std::memcpy(h.data() + b_inst + gsum * sizeof(ObsSet), byv[v].data(), byv[v].size() * sizeof(ObsSet));
     gsum += byv[v].size();
-    if (wgs[v] > beephost::kGridMaxX) return fail(c0, BEEP_EINVAL, "observation log-likelihood: too many chunks");
   }
+  std::memcpy(h.data() + b_inst + b_sets, sums.data(), nset * sizeof(ObsSum));
+  std::memcpy(h.data() + b_inst + b_sets + b_sums, range.data(), range.size() * sizeof(int2));
+  std::memcpy(h.data() + b_inst + b_sets + b_sums + b_range, tab.data(), tab.size() * sizeof(int));
   HIPCHK(c0, hipMemcpyAsync(d, h.data(), up, hipMemcpyHostToDevice, st));
   if (ev0 >= 0) record(c0, ev0);
   using KC = decltype(&beepdev::k_obs_chunks<false, false, false>);
@@ -2339,17 +2339,17 @@ int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const s
                            beepdev::k_obs_chunks<true, true, false>,   beepdev::k_obs_chunks<true, true, true>};
   for (int v = 0; v < 8; v++) {
     if (byv[v].empty()) continue;
-    hipLaunchKernelGGL(kc[v], dim3((unsigned)wgs[v]), dim3(256), 0, st, (const ObsGroup*)(d_groups + goff[v]),
+    hipLaunchKernelGGL(kc[v], dim3((unsigned)wgs[v]), dim3(256), 0, st, (const ObsSet*)(d_sets + goff[v]),
                        (int)byv[v].size(), d_part);
     HIPCHK(c0, hipGetLastError());
   }
-  hipLaunchKernelGGL(beepdev::k_obs_reduce, dim3((unsigned)((NI + 255) / 256)), dim3(256), 0, st,
-                     (const ObsItem*)d_items, (int)NI, (const double*)d_part, d_out);
+  hipLaunchKernelGGL(beepdev::k_obs_reduce, dim3((unsigned)((N + 255) / 256), (unsigned)std::min(1 + max_ndt, 1024)),
+                     dim3(256), 0, st,
+                     (const ObsSum*)d_sums, (int)nset, (int)N, (const double*)d_part, d_out, d_out + N);
   HIPCHK(c0, hipGetLastError());
   if (ev0 >= 0) record(c0, ev0 + 1);
   HIPCHK(c0, hipMemcpyAsync(out, d_out, N * sizeof(double), hipMemcpyDeviceToHost, st));
-  if (out_dt && NI > N)
-    HIPCHK(c0, hipMemcpyAsync(out_dt, d_out + N, (NI - N) * sizeof(double), hipMemcpyDeviceToHost, st));
+  if (ND) HIPCHK(c0, hipMemcpyAsync(out_dt, d_out + N, ND * sizeof(double), hipMemcpyDeviceToHost, st));
   HIPCHK(c0, hipStreamSynchronize(st));
   return BEEP_OK;
 }

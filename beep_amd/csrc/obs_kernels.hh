@@ -197,95 +197,119 @@ __global__ void __launch_bounds__(256) k_obs_loglik(const ObsDev* __restrict__ o
 }
 
 // ---- observation log-likelihoods in chunks of observations ----
-// A group is up to OBS_GROUP instances of one context and a list of
-// observations (all of them in stored order, or those of one data table); the
-// list is cut into chunks of BEEP_OBS_CHUNK, one workgroup each, and each
-// workgroup writes one partial sum per instance.  k_obs_reduce then adds an
-// instance's partials in chunk order.  Work is spread over the whole device
-// however few instances a context has, and the sum of an instance depends only
-// on its context's observations, not on the call or batch it is in.  Sums per
-// data table come of one group per table (512 instances x 40,000 observations
-// in two tables: one workgroup per instance 328 us, now 115 us).
+// A set is one context's instances and a list of its observations (all in
+// stored order, or data table by data table), cut into chunks of at most
+// BEEP_OBS_CHUNK, none of which crosses from one table's list to the next.  One
+// workgroup takes one chunk for up to OBS_GROUP instances of the set and writes
+// one partial sum per instance.  k_obs_reduce then adds an instance's partials
+// in chunk order.  Work is spread over the whole device however few instances a
+// context has, and the sum of an instance depends only on its context's
+// observations, not on the call or batch it is in.  (Two data tables of 20,000
+// observations, 512 instances: 115 us; one workgroup per instance 328.)  A
+// workgroup's instances and chunk follow from its number, so a call uploads a
+// set per context and the instances' numbers: descriptors per group of instances
+// and per sum took a call over 4,096 instances of one short list 210 us, now 69.
 #define BEEP_OBS_CHUNK 2048
 constexpr int OBS_GROUP = 4;
 
-struct ObsGroup {
+struct ObsSet {
   ObsDev od;                        // the context's observation structure (a copy: read
                                     // with scalar loads, as a kernel argument would be)
   const int* tn;                    // its transnum, [instance][S][T][AG]
   const int* pt;                    // its population trajectories, or null
   const double* ospl;               // its observation-spline values per slot, or null
   const int* inst_slot;             // its instances' slots (splines), or null
-  const int* inst;                  // the group's instances
+  const int* inst;                  // the instances [ninst]
   unsigned long long traj_sz, pop_traj_sz;
-  const int* sel;                   // its observations sel[k0 .. k1), or k0 .. k1 themselves when null
-  int k0, k1;
-  int ninst;                        // 1..OBS_GROUP
-  int nchunk;                       // ceil((k1 - k0) / BEEP_OBS_CHUNK), at least 1
-  int wg0;                          // first workgroup of the group in its launch
-  int part0;                        // first partial record of the group
+  const int* sel;                   // its list of observations, or null: all in stored order
+  const int2* range;                // places [x, y) of the list taken by each chunk
+  int ninst;
+  int nchunk;                       // at least 1
+  int wg0;                          // first workgroup of the set in its launch
+  int part0;                        // first partial record of the set
 };
 
-// Partial sums: record p holds OBS_GROUP doubles, one per instance of its
-// group.  Grid: one workgroup per (group, chunk), groups in wg0 order.
+// Partial sums: record part0 + g * nchunk + c holds OBS_GROUP doubles, chunk c's
+// sums of instances g * OBS_GROUP and on.  Grid: one workgroup per record, sets
+// in wg0 order.
 template <bool GENERAL, bool POP, bool SPL>
-__global__ void __launch_bounds__(256) k_obs_chunks(const ObsGroup* __restrict__ groups, int ngroups,
+__global__ void __launch_bounds__(256) k_obs_chunks(const ObsSet* __restrict__ sets, int nset,
                                                     double* __restrict__ partial) {
   constexpr int NI = OBS_GROUP;
   __shared__ double red[8];
-  // The group of this workgroup: the last one whose wg0 is at most blockIdx.x.
-  int lo = 0, hi = ngroups - 1;
+  // The set of this workgroup: the last one whose wg0 is at most blockIdx.x.
+  int lo = 0, hi = nset - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (groups[mid].wg0 <= (int)blockIdx.x) lo = mid;
+    if (sets[mid].wg0 <= (int)blockIdx.x) lo = mid;
     else hi = mid - 1;
   }
-  const ObsGroup& gr = groups[lo];
-  const ObsDev& od = gr.od;
-  const int c = (int)blockIdx.x - gr.wg0;
-  const int kbeg = gr.k0 + c * BEEP_OBS_CHUNK;
-  const int kend = min(kbeg + BEEP_OBS_CHUNK, gr.k1);
+  const ObsSet& st = sets[lo];
+  const ObsDev& od = st.od;
+  const int w = (int)blockIdx.x - st.wg0, g = w / st.nchunk, c = w - g * st.nchunk;
+  const int nin = min(NI, st.ninst - g * NI);
+  const int kbeg = gview(st.range)[c].x, kend = gview(st.range)[c].y;
   int ins[NI];
   const int* tnb[NI];
   const int* ptb[NI];
   const double* splv[NI];
-  // The pointers read from the group are generic; derived from global views,
+  // The pointers read from the set are generic; derived from global views,
   // the trajectory gathers compile to global (not flat) loads, as they do
   // from kernel arguments.
 #pragma unroll
   for (int q = 0; q < NI; q++) {
-    ins[q] = gview(gr.inst)[q < gr.ninst ? q : 0];  // past the group's end: instance 0 again, not written
-    tnb[q] = (const int*)(gview(gr.tn) + (size_t)ins[q] * gr.traj_sz);
-    ptb[q] = gr.pt ? (const int*)(gview(gr.pt) + (size_t)ins[q] * gr.pop_traj_sz) : nullptr;
-    splv[q] = SPL ? (const double*)(gview(gr.ospl) + (size_t)gview(gr.inst_slot)[ins[q]] * od.nospl * od.S) : nullptr;
+    ins[q] = gview(st.inst)[g * NI + (q < nin ? q : 0)];   // past the end: the group's first again, not written
+    tnb[q] = (const int*)(gview(st.tn) + (size_t)ins[q] * st.traj_sz);
+    ptb[q] = st.pt ? (const int*)(gview(st.pt) + (size_t)ins[q] * st.pop_traj_sz) : nullptr;
+    splv[q] = SPL ? (const double*)(gview(st.ospl) + (size_t)gview(st.inst_slot)[ins[q]] * od.nospl * od.S) : nullptr;
   }
   double L[NI], acc[8];
-  obs_terms<false, GENERAL, POP, SPL, NI>(od, gr.sel, kbeg, kend, 0, tnb, ptb, splv, L, acc);
+  obs_terms<false, GENERAL, POP, SPL, NI>(od, st.sel, kbeg, kend, 0, tnb, ptb, splv, L, acc);
 #pragma unroll
   for (int q = 0; q < NI; q++) {
     const double Lt = block_sum(L[q], red);
-    if (threadIdx.x == 0 && q < gr.ninst) partial[(size_t)(gr.part0 + c) * NI + q] = Lt;
+    if (threadIdx.x == 0 && q < nin) partial[(size_t)(st.part0 + w) * NI + q] = Lt;
   }
 }
 
-// An instance's place among the partials, the factor of its sum (1, or -2 for
-// an error function), and where its EF goes (or null).
-struct ObsItem {
-  int part0, nchunk, q;
-  float factor;
+// A set's sums: its instances' totals from out[out0], and with ndt > 0 their
+// tables' -2 x sums from dt_out[dt0], [instance][ndt], table t being chunks
+// [tab[t], tab[t + 1]); the totals' EF too unless null.
+struct ObsSum {
+  const int* inst;
   double* EF;
+  const int* tab;
+  int part0, nchunk, out0, ndt, dt0;
 };
 
-// out[i] = sum over the chunks of item i's partials, in chunk order; EF too.
-__global__ void __launch_bounds__(256) k_obs_reduce(const ObsItem* __restrict__ items, int n,
-                                                    const double* __restrict__ partial, double* __restrict__ out) {
+// Grid (ceil(n / 256), 1 + the most tables of a set, or fewer rows): thread x of
+// row 0 makes total x, of row 1 + t the sum of table t of the same instance (and
+// of the tables a grid's height on); each adds its chunks' partials in order.
+__global__ void __launch_bounds__(256) k_obs_reduce(const ObsSum* __restrict__ sums, int nset, int n,
+                                                    const double* __restrict__ partial, double* __restrict__ out,
+                                                    double* __restrict__ dt_out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const ObsItem it = items[i];
-  double L = 0;
-  for (int c = 0; c < it.nchunk; c++) L += partial[(size_t)(it.part0 + c) * OBS_GROUP + it.q];
-  out[i] = it.factor * L;
-  if (it.EF) *it.EF = -2.0 * L;
+  int lo = 0, hi = nset - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (sums[mid].out0 <= i) lo = mid;
+    else hi = mid - 1;
+  }
+  const ObsSum& su = sums[lo];
+  const int k = i - su.out0;
+  const double* p = partial + ((size_t)su.part0 + (size_t)(k / OBS_GROUP) * su.nchunk) * OBS_GROUP + k % OBS_GROUP;
+  for (int t = (int)blockIdx.y - 1; t < su.ndt; t += gridDim.y) {
+    const int c0 = t < 0 ? 0 : gview(su.tab)[t], c1 = t < 0 ? su.nchunk : gview(su.tab)[t + 1];
+    double L = 0;
+    for (int c = c0; c < c1; c++) L += p[(size_t)c * OBS_GROUP];
+    if (t >= 0) {
+      dt_out[su.dt0 + (size_t)k * su.ndt + t] = -2.0 * L;
+    } else {
+      out[i] = L;
+      if (su.EF) su.EF[gview(su.inst)[k]] = -2.0 * L;
+    }
+  }
 }
 
 // The log-likelihood terms of observations [kbeg, kend) of the list sel (all
