@@ -517,8 +517,10 @@ int launch_stepwise(beep_ctx* c, int mode, const Job* djobs, int n, int t0, int 
     if (c->dense) {
       beepdev::DenseMix p{c->d_D, c->d_M, c->d_I, c->h_topo.diag, c->h_topo.fac, djobs, rows, m.A, c->Apad, m.G, s,
                           c->h_topo.off_geo};
-      hipLaunchKernelGGL(beepdev::k_dense_contract, dim3((unsigned)geo.dense.x, (unsigned)geo.dense.y), dim3(256), 0,
-                         c->stream, p);
+      if (geo.narrow)
+        hipLaunchKernelGGL(beepdev::k_dense_contract<1>, dim3((unsigned)geo.dense32.x), dim3(256), 0, c->stream, p);
+      else
+        hipLaunchKernelGGL(beepdev::k_dense_contract<2>, dim3((unsigned)geo.dense.x), dim3(256), 0, c->stream, p);
     } else {
       beepdev::SparseMix p{c->d_D, c->d_I, c->h_topo.diag, c->h_topo.fac, c->h_topo.in_ptr, c->h_topo.in_src,
                            c->h_topo.in_w, djobs, rows, m.A, c->Apad, m.G, s, c->h_topo.off_geo};
@@ -2782,8 +2784,12 @@ int beep_debug_gemm(int device, int rows, int K, const float* A, const float* B,
     for (int j = 0; j < K; j++) Btf[beepdev::frag_at(j, k, K)] = B[(size_t)k * K + j];
   return debug_run(device, Af.size() * 4, Af.data(), Btf.size() * 4, Btf.data(), (size_t)rows * K * 4, C,
                    [&](void* a, void* b, void* o) {
-                     hipLaunchKernelGGL(beepdev::k_dbg_gemm, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, 0,
-                                        (const float*)a, (const float*)b, (float*)o, rows, K);
+                     if (beephost::narrow_tiles(tiles))
+                       hipLaunchKernelGGL(beepdev::k_dbg_gemm<1>, dim3((unsigned)((2 * tiles + 7) / 8 * 8)), dim3(256), 0,
+                                          0, (const float*)a, (const float*)b, (float*)o, rows, K);
+                     else
+                       hipLaunchKernelGGL(beepdev::k_dbg_gemm<2>, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, 0,
+                                          (const float*)a, (const float*)b, (float*)o, rows, K);
                    });
 }
 

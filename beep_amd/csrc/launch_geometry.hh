@@ -48,6 +48,14 @@ inline std::string fused_geometry(long long njobs, int block, size_t lds, size_t
   return "";
 }
 
+// Whether a product of `tiles` tiles of 64x64 is done in tiles of 32 columns:
+// twice the workgroups of half the length, where those of 64 columns leave some
+// of the 256 CUs with one and others with two.  Contraction and transitions of a
+// step, 64 columns against 32: 45 tiles 21.9 and 18.5 us, 288 tiles 58.6 and
+// 56.5, 360 tiles 93.0 and 90.7, 510 tiles 125.1 and 126.3, 720 tiles 183.7 and
+// 182.9, 1440 tiles 370.4 and 368.
+inline bool narrow_tiles(long long tiles) { return tiles < 432; }
+
 // The step-wise path's launches for n jobs of one context (A areas, G age
 // groups, Apad the padded area count of its D / I buffers, which hold
 // capacity * G rows): the initial infectivity and transition kernels (grid
@@ -57,7 +65,9 @@ inline std::string fused_geometry(long long njobs, int block, size_t lds, size_t
 // contiguous runs) or the sparse one (rows x ceil(A/256)).
 struct StepGeometry {
   Dim cell;       // k_step_init and the transition kernels
-  Dim dense;      // k_dense_contract
+  Dim dense;      // k_dense_contract in 64x64 tiles
+  Dim dense32;    // and in tiles of 32 columns
+  bool narrow = false;   // the tiles of 32 columns are the faster ones
   Dim sparse;     // k_sparse_contract
   long long rows = 0;
 };
@@ -76,6 +86,9 @@ inline std::string stepwise_geometry(int A, int G, int Apad, long long n, long l
   const long long tiles = ((g.rows + 63) / 64) * (Apad / 64);
   g.dense.x = (tiles + 7) / 8 * 8;
   g.dense.y = 1;
+  g.dense32.x = (2 * tiles + 7) / 8 * 8;
+  g.dense32.y = 1;
+  g.narrow = narrow_tiles(tiles);
   g.sparse.x = g.rows;
   g.sparse.y = (A + 255) / 256;
   Dim b256;

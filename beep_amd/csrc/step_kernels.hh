@@ -27,145 +27,190 @@ struct DenseMix {
 
 typedef float f16v __attribute__((ext_vector_type(16)));
 
-// One 64x64 output tile of C = A x B (origin (tm, tn)) per workgroup of four
-// wavefronts.  A (rows padded to a multiple of 64) and B transposed are in
-// fragment order (frag_at), K a multiple of 64.  K is split four ways: each
-// wavefront computes the whole 64x64 tile over its quarter of K with four
-// accumulators (each 16-byte operand load feeds two MFMAs, and the four
-// accumulation chains interleave), streaming its row blocks of A and column
-// blocks of B from L2 straight into registers, the next block's four loads in
-// flight while the current block's 16 MFMAs run.  The four partial tiles are
-// then summed through LDS (48 KB): wavefront w returns the sum of quadrant w
-// (rows 32 (w / 2), columns 32 (w % 2) of the tile).  2880 wavefronts for the
-// 9216 x 320 x 320 product of 1024 particles of 9 groups, 2.8 per SIMD.
+// One output tile of C = A x B, 64 rows x 32 NB columns (origin (tm, tn)), per
+// workgroup of four wavefronts.  A (rows padded to a multiple of 64) and B
+// transposed are in fragment order (frag_at), K a multiple of 64.  K is split
+// four ways: each wavefront computes the whole tile over its quarter of K with
+// 2 NB accumulators (the accumulation chains interleave), streaming its row
+// blocks of A and column blocks of B from L2 straight into registers, the next
+// block's loads in flight while the current block's MFMAs run.  The four partial
+// tiles are then summed through LDS, quadrant by quadrant of 32 x 32: quadrant
+// qd of the 64 x 64 tile around is wavefront qd's partial plus the others' in
+// wavefront order, whatever NB.  With NB = 2 wavefront w returns quadrant w (rows
+// 32 (w / 2), columns 32 (w % 2)) in 16 registers; with NB = 1 registers 8 (w % 2)
+// and on of the quadrant at rows 32 (w / 2).
+// NB = 2 loads less per MFMA, NB = 1 gives twice the workgroups of half the
+// length (narrow_tiles).  4608 x 320 x 320, the product of 512 particles of 9
+// groups: 17.3 us with NB = 2 and two blocks of operands in flight, 15.5 with
+// NB = 1 and four; 6.5 of them are a launch's own (the product of one particle),
+// 6.2 the MFMAs of the three workgroups of a CU.
 // Accumulator layout of the 32x32 MFMA: lane l holds column l % 32 and, in
 // register v, row 8*(v/4) + 4*(l/32) + v%4.
-__device__ inline f16v mfma_tile_ksplit(const float* __restrict__ Af, const float* __restrict__ Btf, int K, int tm,
-                                        int tn) {
-  __shared__ float red[4][3][16][64];       // [writer][its other quadrants][register][lane]
+template <int NB>
+struct TileSums {
+  float v[8 * NB];
+};
+
+template <int NB>
+__device__ inline TileSums<NB> mfma_tile_ksplit(const float* __restrict__ Af, const float* __restrict__ Btf, int K,
+                                                int tm, int tn) {
+  // Partial sums of the tile's quadrants, [wavefront][quadrant][register][lane];
+  // with NB = 2 without the wavefront's own, which stays in registers (48 KB, so
+  // that three workgroups fit a CU).
+  constexpr int NQ = NB == 2 ? 3 : 2;
+  __shared__ float red[4][NQ][16][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nq = K >> 3, nqw = nq >> 2, q0 = wave * nqw, qe = q0 + nqw;
   const float4* __restrict__ a4[2];
-  const float4* __restrict__ b4[2];
+  const float4* __restrict__ b4[NB];
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
-    a4[i] = (const float4*)Af + (size_t)((tm >> 5) + i) * nq * 64 + lane;
-    b4[i] = (const float4*)Btf + (size_t)((tn >> 5) + i) * nq * 64 + lane;
-  }
-  f16v acc[2][2];
+  for (int i = 0; i < 2; i++) a4[i] = (const float4*)Af + (size_t)((tm >> 5) + i) * nq * 64 + lane;
+#pragma unroll
+  for (int j = 0; j < NB; j++) b4[j] = (const float4*)Btf + (size_t)((tn >> 5) + j) * nq * 64 + lane;
+  f16v acc[2][NB];
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int j = 0; j < NB; j++)
 #pragma unroll
       for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-  float4 a0[2], b0[2], a1[2], b1[2];
-  // A scheduling barrier after each group of loads keeps the compiler from
-  // sinking them next to their MFMAs (which would wait out every load's
-  // latency).  The loop body has no condition around its loads, so each
-  // wait before a block's MFMAs leaves the next block's loads in flight.
-  auto load = [&](float4(&a)[2], float4(&b)[2], int q) {
+  // Four blocks of operands in flight: they were written by other XCDs, so the
+  // first reads of a launch go past its L2.  A scheduling barrier after each group of loads keeps the compiler from sinking them next
+  // to their MFMAs, and the loop body has no condition around its loads (past the
+  // end they read the last block again), so each wait before a block's MFMAs
+  // leaves the later blocks' loads in flight.
+  float4 av[4][2], bv[4][NB];
+  auto load = [&](int slot, int q) {
+    q = min(q, qe - 1);
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-      a[i] = a4[i][q * 64];
-      b[i] = b4[i][q * 64];
-    }
+    for (int i = 0; i < 2; i++) av[slot][i] = a4[i][q * 64];
+#pragma unroll
+    for (int j = 0; j < NB; j++) bv[slot][j] = b4[j][q * 64];
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto mfma4 = [&](float x0, float x1, float y0, float y1) {
-    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(x0, y0, acc[0][0], 0, 0, 0);
-    acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(x0, y1, acc[0][1], 0, 0, 0);
-    acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(x1, y0, acc[1][0], 0, 0, 0);
-    acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(x1, y1, acc[1][1], 0, 0, 0);
+  // Block component k is the operand of the block's MFMA k.
+  auto compute = [&](int slot) {
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+          acc[i][j] =
+              __builtin_amdgcn_mfma_f32_32x32x2f32((&av[slot][i].x)[k], (&bv[slot][j].x)[k], acc[i][j], 0, 0, 0);
   };
-  // Block component i is the operand of the block's MFMA i.
-  auto compute = [&](const float4(&a)[2], const float4(&b)[2]) {
-    mfma4(a[0].x, a[1].x, b[0].x, b[1].x);
-    mfma4(a[0].y, a[1].y, b[0].y, b[1].y);
-    mfma4(a[0].z, a[1].z, b[0].z, b[1].z);
-    mfma4(a[0].w, a[1].w, b[0].w, b[1].w);
-  };
-  load(a0, b0, q0);
-  int q = q0;
-  for (; q + 2 < qe; q += 2) {
-    load(a1, b1, q + 1);
-    compute(a0, b0);
-    load(a0, b0, q + 2);
-    compute(a1, b1);
+#pragma unroll
+  for (int u = 0; u < 4; u++) load(u, q0 + u);
+  int q = q0;                                  // K / 32 blocks, an even number
+  for (; q + 4 <= qe; q += 4) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      compute(u);
+      load(u, q + 4 + u);
+    }
   }
-  load(a1, b1, q + 1);
-  compute(a0, b0);
-  compute(a1, b1);
-  // Quadrant qd of writer w goes to slot qd - (qd > w) of its three.
-#pragma unroll
-  for (int qd = 0; qd < 4; qd++) {
-    if (qd == wave) continue;
-#pragma unroll
-    for (int v = 0; v < 16; v++) red[wave][qd - (qd > wave)][v][lane] = acc[qd >> 1][qd & 1][v];
+  if (q < qe) {
+    compute(0);
+    compute(1);
   }
-  __syncthreads();
-  f16v s;
+  TileSums<NB> s;
+  if constexpr (NB == 2) {
+    // Quadrant qd of writer w goes to slot qd - (qd > w) of its three.
 #pragma unroll
-  for (int qd = 0; qd < 4; qd++)
-    if (qd == wave) s = acc[qd >> 1][qd & 1];
+    for (int qd = 0; qd < 4; qd++) {
+      if (qd == wave) continue;
 #pragma unroll
-  for (int w2 = 0; w2 < 4; w2++) {
-    if (w2 == wave) continue;
-    const int slot = wave - (wave > w2);
+      for (int v = 0; v < 16; v++) red[wave][qd - (qd > wave)][v][lane] = acc[qd >> 1][qd & 1][v];
+    }
+    __syncthreads();
 #pragma unroll
-    for (int v = 0; v < 16; v++) s[v] += red[w2][slot][v][lane];
+    for (int qd = 0; qd < 4; qd++)
+      if (qd == wave) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) s.v[v] = acc[qd >> 1][qd & 1][v];
+      }
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      if (w == wave) continue;
+      const int slot = wave - (wave > w);
+#pragma unroll
+      for (int v = 0; v < 16; v++) s.v[v] += red[w][slot][v][lane];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) red[wave][i][v][lane] = acc[i][0][v];
+    __syncthreads();
+    const int i = wave >> 1, v0 = 8 * (wave & 1);
+    const int first = 2 * i + ((tn >> 5) & 1);         // the quadrant of the 64 x 64 tile around
+#pragma unroll
+    for (int v = 0; v < 8; v++) s.v[v] = red[first][i][v0 + v][lane];
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      if (w == first) continue;
+#pragma unroll
+      for (int v = 0; v < 8; v++) s.v[v] += red[w][i][v0 + v][lane];
+    }
   }
   return s;
 }
 
-// Tiles of a 64x64-tiled product for a one-dimensional grid of
+// Tiles of 64 x cols of a product for a one-dimensional grid of
 // 8 * ceil(tiles / 8) workgroups.  Workgroups are dealt to the eight XCDs in
 // turn (workgroup w runs on XCD w % 8), so XCD x is given the contiguous run
 // of tiles [x * per, (x + 1) * per) in row-major tile order: the column tiles
 // of one row tile share an XCD and its L2, which then reads that row tile of
 // the left operand once instead of once per column tile.  Returns false for
 // the few workgroups past the last tile (the whole workgroup returns).
-__device__ inline bool xcd_tile(int ntm, int ntn, int* tm, int* tn) {
+__device__ inline bool xcd_tile(int ntm, int ntn, int cols, int* tm, int* tn) {
   const int total = ntm * ntn;
   const int per = (total + 7) >> 3;
   const int t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
   if (t >= total) return false;
   *tm = (t / ntn) * 64;
-  *tn = (t - (t / ntn) * ntn) * 64;
+  *tn = (t - (t / ntn) * ntn) * cols;
   return true;
 }
 
 // The dense contraction with its FOI epilogue, one-dimensional grid of
-// 8 * ceil(ceil(rows / 64) * (Apad / 64) / 8) workgroups (xcd_tile).
-// Three workgroups per CU (48 KB of LDS each) hold the grid of 720
-// workgroups of the 9216-row product at once: registers are capped for three
-// wavefronts per SIMD.
+// 8 * ceil(ceil(rows / 64) * (Apad / (32 NB)) / 8) workgroups (xcd_tile).
+// Every load of the epilogue is issued before the first store: the stores to I
+// may alias the job table and D as far as the compiler knows, so loads
+// interleaved with them would wait out one latency per row.  With NB = 1 they
+// are issued before the product too, whose loop hides their latency (three
+// dependent loads to a row's m(t)); with NB = 2 there are no registers for them:
+// they are capped for three wavefronts per SIMD, so that three workgroups per CU
+// hold the grid of 720 workgroups of a 9216-row product at once.
+template <int NB>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) k_dense_contract(DenseMix p) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int tm, tn;
-  if (!xcd_tile((p.rows + 63) / 64, p.Apad / 64, &tm, &tn)) return;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  f16v acc = mfma_tile_ksplit(p.D, p.Mt, p.Apad, tm, tn);
-  const int col = tn + wn + (lane & 31);
+  if (!xcd_tile((p.rows + 63) / 64, p.Apad / (32 * NB), 32 * NB, &tm, &tn)) return;
+  const int col = tn + (NB == 2 ? (wave & 1) * 32 : 0) + (lane & 31);
+  const int rbase = tm + (wave >> 1) * 32 + 4 * (lane >> 5) + (NB == 2 ? 0 : 16 * (wave & 1));
+  const int ccol = min(col, p.A - 1);
+  float dg, fc, mv[8 * NB], dv[8 * NB];
+  auto operands = [&] {
+    dg = p.diag[ccol];
+    fc = p.fac[ccol];
+#pragma unroll
+    for (int v = 0; v < 8 * NB; v++) {
+      const int row = min(rbase + 8 * (v >> 2) + (v & 3), p.rows - 1);
+      mv[v] = p.jobs[row / p.G].tab[p.off_geo + p.s];
+      dv[v] = p.D[frag_at(row, ccol, p.Apad)];
+    }
+  };
+  if constexpr (NB == 1) operands();
+  const TileSums<NB> acc = mfma_tile_ksplit<NB>(p.D, p.Mt, p.Apad, tm, tn);
   if (col >= p.A) return;
-  const float dg = p.diag[col], fc = p.fac[col];
-  // Every load of the epilogue is issued before the first store: the stores
-  // to I may alias the job table and D as far as the compiler knows, so
-  // loads interleaved with them would wait out one latency per row.
-  const int rbase = tm + wm + 4 * (lane >> 5);
-  float mv[16], dv[16];
+  if constexpr (NB == 2) operands();
 #pragma unroll
-  for (int v = 0; v < 16; v++) {
-    const int row = min(rbase + 8 * (v >> 2) + (v & 3), p.rows - 1);
-    mv[v] = p.jobs[row / p.G].tab[p.off_geo + p.s];
-    dv[v] = p.D[frag_at(row, col, p.Apad)];
-  }
-#pragma unroll
-  for (int v = 0; v < 16; v++) {
+  for (int v = 0; v < 8 * NB; v++) {
     const int row = rbase + 8 * (v >> 2) + (v & 3);
     if (row < p.rows) {
       const float idg = dg * dv[v];
-      p.I[(size_t)row * p.Apad + col] = (idg + acc[v]) * mv[v] + fc * idg * (1.f - mv[v]);
+      p.I[(size_t)row * p.Apad + col] = (idg + acc.v[v]) * mv[v] + fc * idg * (1.f - mv[v]);
     }
   }
 }
@@ -173,18 +218,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))
 // Plain GEMM with the same tiling (no epilogue) for the tests of the operand
 // order and accumulator layout: C[rows][Apad] = A x B, A and B transposed in
 // fragment order.
+template <int NB>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4)))
 k_dbg_gemm(const float* Af, const float* Btf, float* C_, int rows, int Apad) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int tm, tn;
-  if (!xcd_tile((rows + 63) / 64, Apad / 64, &tm, &tn)) return;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  f16v acc = mfma_tile_ksplit(Af, Btf, Apad, tm, tn);
-  const int col = tn + wn + (lane & 31);
+  if (!xcd_tile((rows + 63) / 64, Apad / (32 * NB), 32 * NB, &tm, &tn)) return;
+  const TileSums<NB> acc = mfma_tile_ksplit<NB>(Af, Btf, Apad, tm, tn);
+  const int col = tn + (NB == 2 ? (wave & 1) * 32 : 0) + (lane & 31);
+  const int r0 = tm + (wave >> 1) * 32 + 4 * (lane >> 5) + (NB == 2 ? 0 : 16 * (wave & 1));
 #pragma unroll
-  for (int v = 0; v < 16; v++) {
-    int row = tm + wm + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-    if (row < rows) C_[(size_t)row * Apad + col] = acc[v];
+  for (int v = 0; v < 8 * NB; v++) {
+    const int row = r0 + 8 * (v >> 2) + (v & 3);
+    if (row < rows) C_[(size_t)row * Apad + col] = acc.v[v];
   }
 }
 
