@@ -305,6 +305,7 @@ __device__ inline int binomial_inversion(int n, float p, float ufirst, ExtraUnif
         const float x = fmaxf(__builtin_fmaf(a, __builtin_amdgcn_rcpf((float)(t + j)), -s), 0.f);
         u -= rr;
         rr *= x;
+        asm("" : "+v"(rr));        // rounded: the next u - rr is no fused u - rr * x
         k += u > rr;
       }
     }

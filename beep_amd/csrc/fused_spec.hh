@@ -41,8 +41,9 @@
 // Replaced: a branch per transition for each null check, error check, queue
 // push and masked store, and four global loads per step behind the stores
 // (92 branches per step of a single-cell instance, half of a wavefront's time in
-// waits).  Proposals of 256 x 400 cells x 200 steps: 2.87 -> 1.96 ms; one
-// single-cell instance, 100 steps: 0.395 -> 0.32 ms.
+// waits).  Proposals of 256 x 400 cells x 200 steps: 2.87 -> 1.96 ms, and 1.75
+// with the context's choices at compile time and binomials drawn by counting; one
+// single-cell instance, 100 steps: 0.395 -> 0.32 -> 0.235 ms.
 #pragma once
 
 namespace beepdev {
