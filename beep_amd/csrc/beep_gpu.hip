@@ -194,6 +194,7 @@ int dalloc(beep_ctx* c, void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();     // reported here, not by the next launch's check
     return fail(c, BEEP_ENOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
   }
   c->allocated += bytes;
@@ -236,20 +237,39 @@ int ensure_jobs(beep_ctx* c, size_t n) {
   return BEEP_OK;
 }
 
+// At least `bytes` of scratch.  A call that cannot have them leaves the context
+// the scratch that it held: one beyond the budget fails before anything is
+// freed, and where the device has no room the old size is taken again.
 int ensure_scratch(beep_ctx* c, size_t bytes) {
   if (bytes <= c->scratch_cap) return BEEP_OK;
+  const size_t cap = std::max<size_t>(bytes, 1 << 16), held = c->scratch_cap;
+  if (c->budget && c->allocated - held + cap > c->budget)
+    return fail(c, BEEP_ENOMEM, "HBM budget exceeded: %zu + %zu > %zu bytes", c->allocated - held, cap, c->budget);
   if (c->d_scratch) {
     HIPCHK(c, hipFree(c->d_scratch));
     c->allocs.erase(std::find(c->allocs.begin(), c->allocs.end(), c->d_scratch));
-    c->allocated -= c->scratch_cap;
+    c->allocated -= held;
     c->d_scratch = nullptr;
     c->scratch_cap = 0;
   }
-  size_t cap = std::max<size_t>(bytes, 1 << 16);
   int rc = dalloc(c, &c->d_scratch, cap);
-  if (rc) return rc;
+  if (rc) {
+    const std::string err = c->err;
+    if (held && dalloc(c, &c->d_scratch, held) == BEEP_OK) c->scratch_cap = held;
+    c->err = err;
+    return rc;
+  }
   c->scratch_cap = cap;
   return BEEP_OK;
+}
+
+// ensure_scratch for a caller that can do with less: no error is left behind,
+// neither the context's text nor the runtime's last error.
+bool try_scratch(beep_ctx* c, size_t bytes) {
+  const std::string err = c->err;
+  if (ensure_scratch(c, bytes) == BEEP_OK) return true;
+  c->err = err;
+  return false;
 }
 
 void record(beep_ctx* c, int k) { (void)hipEventRecord(c->ev[k], c->stream); }
@@ -1491,12 +1511,9 @@ int beep_obs_loglik(beep_ctx* c, int n, const int32_t* inst, int section, double
   const int nsel = c->sec_ptr[section + 1] - c->sec_ptr[section];
   int nchunk = EF_dt_out ? 1 : section_chunks(nsel);
   auto doubles = [&] { return EF_dt_out ? (size_t)n * (1 + ndt) : (size_t)n * nchunk; };
-  rc = ensure_scratch(c, doubles() * sizeof(double) + (size_t)n * sizeof(int));
-  if (rc && nchunk > 1) {
-    nchunk = 1;
-    rc = ensure_scratch(c, doubles() * sizeof(double) + (size_t)n * sizeof(int));
-  }
-  if (rc) return rc;
+  auto bytes = [&] { return doubles() * sizeof(double) + (size_t)n * sizeof(int); };
+  if (nchunk > 1 && !try_scratch(c, bytes())) nchunk = 1;
+  if ((rc = ensure_scratch(c, bytes()))) return rc;
   const size_t out_doubles = doubles();
   double* d_out = (double*)c->d_scratch;
   int* d_inst = (int*)(d_out + out_doubles);
@@ -1617,19 +1634,15 @@ namespace {
 // S steps of X rows (transitions or compartments) of an instance between its
 // device trajectory `dev` ([s][x][area * group]) and host memory `host`
 // ([s][area][x][group]): slabs of steps are reordered by a kernel next to their
-// copy.  A slab is at most 16 MiB of staging, or what the context already
-// holds; without any, and for up to 4096 values (8 us of host loop, about a
-// kernel launch), the host does the reordering.
+// copy.  A slab is at most 16 MiB of staging, or whole steps of what the context
+// already holds; without room for one step, and for up to 4096 values (8 us of
+// host loop, about a kernel launch), the host does the reordering.
 int move_trajectory(beep_ctx* c, int* dev, int* host, int S, int X, bool to_host) {
   const auto& m = c->m;
   const size_t row = (size_t)X * m.AG, total = (size_t)S * row;
   size_t steps = std::min<size_t>((size_t)S, std::max<size_t>(1, ((size_t)16 << 20) / (row * sizeof(int))));
-  if (total <= 4096) {
-    steps = 0;
-  } else if (ensure_scratch(c, steps * row * sizeof(int)) != BEEP_OK) {
-    steps = c->scratch_cap / (row * sizeof(int));
-    (void)hipGetLastError();
-  }
+  if (total <= 4096) steps = 0;
+  else if (!try_scratch(c, steps * row * sizeof(int))) steps = c->scratch_cap / (row * sizeof(int));
   if (steps == 0) {
     std::vector<int> h(total);
     if (to_host) {
@@ -1720,7 +1733,7 @@ int beep_put_transnum(beep_ctx* c, int inst, int slot, const int32_t* tn) {
     // Steps side by side; the populations go to the kept trajectory or else to
     // scratch (without room for them, step by step below).
     int* pop = job.pt;
-    if (!pop && ensure_scratch(c, c->pop_traj_sz * sizeof(int)) == BEEP_OK) pop = (int*)c->d_scratch;
+    if (!pop && try_scratch(c, c->pop_traj_sz * sizeof(int))) pop = (int*)c->d_scratch;
     if (pop) {
       hipLaunchKernelGGL(beepdev::k_replay_pops, dim3((unsigned)((m.AG + 63) / 64), (unsigned)m.C), dim3(64), 0, c->stream,
                          job.topo, (const int*)job.tn, pop, job.state);
@@ -1734,7 +1747,6 @@ int beep_put_transnum(beep_ctx* c, int inst, int slot, const int32_t* tn) {
       HIPCHK(c, hipGetLastError());
       return check_device_error(c);
     }
-    (void)hipGetLastError();
   }
   job.mode = beepdev::MODE_REPLAY;
   if ((rc = put_jobs(c, std::vector<Job>(1, job)))) return rc;
@@ -1946,12 +1958,8 @@ int beep_pmcmc_obs_prob(beep_ctx* c, int n, const int32_t* inst, int slot, const
   for (int k = 0; k < nsec; k++) maxsel = std::max(maxsel, c->sec_ptr[k + 1] - c->sec_ptr[k]);
   bool chunked = section_chunks(maxsel) > 1;
   auto bytes = [&](int nchunk) { return (size_t)n * (nchunk + 1) * sizeof(double) + (3 * (size_t)n * sizeof(int) + 71) / 8 * 8; };
-  rc = ensure_scratch(c, bytes(section_chunks(maxsel)));
-  if (rc && chunked) {
-    chunked = false;
-    rc = ensure_scratch(c, bytes(1));
-  }
-  if (rc) return rc;
+  chunked = chunked && try_scratch(c, bytes(section_chunks(maxsel)));
+  if ((rc = ensure_scratch(c, bytes(1)))) return rc;
   double* d_ob = (double*)c->d_scratch;
   double* d_w = d_ob + 1;
   int* d_first = (int*)(d_w + n);

@@ -1,0 +1,50 @@
+"""Calls of a context whose HBM budget leaves no room for more scratch: what
+has a way to do with less gives the results of a context without a budget,
+keeps the scratch that was held and leaves no error text behind."""
+import numpy as np
+import pytest
+
+from beep_amd import _lib, configs
+
+pytestmark = pytest.mark.gpu
+
+
+def _error(ctx):
+    return _lib.lib().beep_last_error(ctx._h).decode()
+
+
+def _pair(spec, capacity, start, **kw):
+    """Two contexts after start(ctx): one without a budget, one whose budget is
+    what the first then holds."""
+    free = _lib.Context(spec, capacity=capacity, nslot=1, **kw)
+    start(free)
+    tight = _lib.Context(spec, capacity=capacity, nslot=1, hbm_budget=free.device_bytes, **kw)
+    start(tight)
+    assert tight.device_bytes == free.device_bytes
+    return free, tight
+
+
+@pytest.mark.parametrize("keep", [_lib.KEEP_ALL, _lib.KEEP_TRANSNUM | _lib.KEEP_TRANSMEAN])
+def test_transfers_within_held_scratch(gpu_lib, keep):
+    """Trajectories of 60 steps move through the scratch that is there."""
+    spec, truth = configs.seir_areas(100, 4, 60, seed=3, daily_obs=True)
+
+    def start(ctx):
+        ctx.set_param([0], truth[None, :])
+        ctx.simulate([0], [0], [5], seed=4)
+        ctx.obs_loglik([0])                         # takes the first 64 KB of scratch: 13 steps
+
+    free, tight = _pair(spec, 2, start, keep=keep)
+    held = tight.device_bytes
+    for ctx in (free, tight):
+        ctx.tn = ctx.get_transnum(0)
+        ctx.put_transnum(1, 0, ctx.tn)
+        ctx.tm = ctx.get_transmean(1)
+    assert free.device_bytes > held                 # the slabs wanted more than was held
+    assert tight.device_bytes == held
+    assert _error(tight) == ""
+    assert np.array_equal(free.tn, tight.tn)
+    assert np.array_equal(free.tm.view(np.int32), tight.tm.view(np.int32))
+    assert np.array_equal(free.get_state(1), tight.get_state(1))
+    free.close()
+    tight.close()
