@@ -1763,8 +1763,8 @@ namespace {
 // Copies of 4-byte rows within the arrays `arr` (pointer, values per row), for
 // pairs dst[i] <- src[i] in order; pairs with dst == src do nothing.  When no
 // row is both read and written and none is written twice the order is
-// immaterial and each array takes one launch; otherwise each pair is a copy
-// command of its own, in order.
+// immaterial and each array takes one launch; otherwise, and without scratch for
+// the list, each pair is a copy command of its own, in order.
 int copy_rows(beep_ctx* c, int n, const int32_t* dst, const int32_t* src, const std::vector<std::pair<void*, size_t>>& arr) {
   std::vector<int32_t> d, s;
   std::vector<char> use(c->capacity, 0);
@@ -1780,15 +1780,13 @@ int copy_rows(beep_ctx* c, int n, const int32_t* dst, const int32_t* src, const 
   }
   if (d.empty()) return BEEP_OK;
   const size_t m = d.size();
-  if (!free_order || m == 1) {
+  if (!free_order || m == 1 || !try_scratch(c, 2 * m * sizeof(int))) {
     for (size_t i = 0; i < m; i++)
       for (const auto& a : arr)
         HIPCHK(c, hipMemcpyAsync((char*)a.first + (size_t)d[i] * a.second * 4, (const char*)a.first + (size_t)s[i] * a.second * 4,
                                  a.second * 4, hipMemcpyDeviceToDevice, c->stream));
     return BEEP_OK;
   }
-  int rc;
-  if ((rc = ensure_scratch(c, 2 * m * sizeof(int)))) return rc;
   int* d_idx = (int*)c->d_scratch;
   d.insert(d.end(), s.begin(), s.end());
   HIPCHK(c, hipMemcpyAsync(d_idx, d.data(), 2 * m * sizeof(int), hipMemcpyHostToDevice, c->stream));

@@ -48,3 +48,25 @@ def test_transfers_within_held_scratch(gpu_lib, keep):
     assert np.array_equal(free.get_state(1), tight.get_state(1))
     free.close()
     tight.close()
+
+
+def test_copies_without_scratch(gpu_lib):
+    """Lists of independent pairs need no memory."""
+    spec, truth = configs.seir_areas(9, 4, 12, seed=3, daily_obs=True)
+
+    def start(ctx):
+        ctx.set_param([0], truth[None, :])
+        ctx.simulate(range(6), [0] * 6, range(5, 11), seed=4)
+
+    free, tight = _pair(spec, 6, start)
+    held = tight.device_bytes
+    for ctx in (free, tight):
+        ctx.copy_instances([3, 4, 5], [0, 1, 0])
+        ctx.copy_states([1, 2], [4, 0])
+    assert free.device_bytes > held and tight.device_bytes == held
+    assert _error(tight) == ""
+    for i in range(6):
+        for get in ("get_transnum", "get_transmean", "get_pop", "get_state"):
+            assert np.array_equal(getattr(free, get)(i), getattr(tight, get)(i)), (get, i)
+    free.close()
+    tight.close()
