@@ -1565,21 +1565,31 @@ int beep_pois_loglik(beep_ctx* c, int n, const int32_t* inst, double* L_out) {
     if (!valid_inst(c, inst[i])) return fail(c, BEEP_EINVAL, "instance %d out of range", inst[i]);
   if (n == 0) return BEEP_OK;
   int rc;
-  // Instances on the grid's y: at most 65535 of them a launch.
-  const size_t nchunk = (c->traj_sz + BEEP_POIS_CHUNK - 1) / BEEP_POIS_CHUNK;
-  constexpr int kRows = 65535;
-  const size_t nb = (size_t)std::min(n, kRows);
-  if ((rc = ensure_scratch(c, (size_t)n * (sizeof(double) + sizeof(int)) + 8 + nb * nchunk * sizeof(double)))) return rc;
+  // Instances on the grid's y: at most 65535 of them a launch, fewer where the
+  // chunk sums of so many do not fit, and without room for those of one instance
+  // one workgroup goes over all its chunks and writes the result.
+  size_t nchunk = (c->traj_sz + BEEP_POIS_CHUNK - 1) / BEEP_POIS_CHUNK;
+  size_t nb = (size_t)std::min(n, 65535);
+  auto bytes = [&] { return (size_t)n * (sizeof(double) + sizeof(int)) + nb * nchunk * sizeof(double); };
+  while (nb > 1 && !try_scratch(c, bytes())) nb /= 2;
+  const bool direct = !try_scratch(c, bytes());
+  if (direct) {
+    nchunk = 1;
+    nb = 0;
+    if ((rc = ensure_scratch(c, bytes()))) return rc;
+    nb = (size_t)std::min(n, 65535);
+  }
   double* d_out = (double*)c->d_scratch;
   double* d_part = d_out + n;
-  int* d_inst = (int*)(d_part + nb * nchunk);
+  int* d_inst = (int*)(d_part + (direct ? 0 : nb * nchunk));
   HIPCHK(c, hipMemcpyAsync(d_inst, inst, n * sizeof(int), hipMemcpyHostToDevice, c->stream));
   record(c, 4);
-  for (int i0 = 0; i0 < n; i0 += kRows) {
-    const unsigned m = (unsigned)std::min(n - i0, kRows);
+  for (int i0 = 0; i0 < n; i0 += (int)nb) {
+    const unsigned m = (unsigned)std::min<size_t>(n - i0, nb);
     hipLaunchKernelGGL(beepdev::k_pois_chunks, dim3((unsigned)nchunk, m), dim3(256), 0, c->stream, (const int*)(d_inst + i0),
-                       c->d_tn, c->d_tm, c->traj_sz, (int)nchunk, d_part);
+                       c->d_tn, c->d_tm, c->traj_sz, direct ? d_out + i0 : d_part);
     HIPCHK(c, hipGetLastError());
+    if (direct) continue;
     hipLaunchKernelGGL(beepdev::k_pois_reduce, dim3(m), dim3(64), 0, c->stream, (int)nchunk, (const double*)d_part,
                        d_out + i0);
     HIPCHK(c, hipGetLastError());

@@ -417,34 +417,35 @@ __constant__ double kLogFactorial[64] = {
 
 // State::likelihood (src/state.cc:812-826), the sum of log Pois(transnum |
 // transmean) over an instance's trajectory: in chunks of BEEP_POIS_CHUNK
-// elements, one workgroup each, whose sums k_pois_reduce adds in chunk order.
-// Most counts are small, and log k! of those is a table's entry.  One workgroup
-// per instance with the Gamma function's series for every count left 6
-// instances of 640,000 elements on 6 compute units for 2.9 ms; this takes
-// 21 us.
+// elements, one workgroup each (or fewer workgroups, each going on a grid's
+// width further), whose sums k_pois_reduce adds in chunk order.  Most counts are
+// small, and log k! of those is a table's entry.  One workgroup per instance with
+// the Gamma function's series for every count left 6 instances of 640,000
+// elements on 6 compute units for 2.9 ms; this takes 21 us.
 #define BEEP_POIS_CHUNK 4096
 __global__ void __launch_bounds__(256) k_pois_chunks(const int* __restrict__ inst, const int* __restrict__ tn,
-                                                     const float* __restrict__ tm, size_t traj_sz, int nchunk,
+                                                     const float* __restrict__ tm, size_t traj_sz,
                                                      double* __restrict__ partial) {
   __shared__ double red[8];
   __shared__ double lf[64];
   if (threadIdx.x < 64) lf[threadIdx.x] = kLogFactorial[threadIdx.x];
   __syncthreads();
   const int in = inst[blockIdx.y];
-  const size_t e0 = (size_t)blockIdx.x * BEEP_POIS_CHUNK;
-  const int ne = (int)min((size_t)BEEP_POIS_CHUNK, traj_sz - e0);
-  const int* n = tn + (size_t)in * traj_sz + e0;
-  const float* l = tm + (size_t)in * traj_sz + e0;
   double L = 0;
-  for (int e = threadIdx.x; e < ne; e += blockDim.x) {
-    const int k = n[e];
-    const double lam = (double)l[e];
-    if (lam == 0 || k < 0 || k >= 64) L += poisson_lpmf((double)k, lam);
-    else if (k == 0) L -= lam;
-    else L += (double)k * log(lam) - lam - lf[k];
+  for (size_t e0 = (size_t)blockIdx.x * BEEP_POIS_CHUNK; e0 < traj_sz; e0 += (size_t)gridDim.x * BEEP_POIS_CHUNK) {
+    const int ne = (int)min((size_t)BEEP_POIS_CHUNK, traj_sz - e0);
+    const int* n = tn + (size_t)in * traj_sz + e0;
+    const float* l = tm + (size_t)in * traj_sz + e0;
+    for (int e = threadIdx.x; e < ne; e += blockDim.x) {
+      const int k = n[e];
+      const double lam = (double)l[e];
+      if (lam == 0 || k < 0 || k >= 64) L += poisson_lpmf((double)k, lam);
+      else if (k == 0) L -= lam;
+      else L += (double)k * log(lam) - lam - lf[k];
+    }
   }
   const double t = block_sum(L, red);
-  if (threadIdx.x == 0) partial[(size_t)blockIdx.y * nchunk + blockIdx.x] = t;
+  if (threadIdx.x == 0) partial[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = t;
 }
 
 // out[b] = the sum of instance b's partials; one wavefront per instance.

@@ -70,3 +70,30 @@ def test_copies_without_scratch(gpu_lib):
             assert np.array_equal(getattr(free, get)(i), getattr(tight, get)(i)), (get, i)
     free.close()
     tight.close()
+
+
+@pytest.mark.parametrize("n", [512, 5461])
+def test_state_likelihood_within_held_scratch(gpu_lib, n):
+    """18 chunks of elements an instance: the chunk sums of 512 instances pass
+    64 KB, 5,461 results alone fill it."""
+    spec, truth = configs.seir_areas(100, 4, 60, seed=3, daily_obs=True)
+
+    def start(ctx):
+        ctx.set_param([0], truth[None, :])
+        ctx.simulate(range(5), [0] * 5, range(5, 10), seed=4)
+        ctx.obs_loglik([0])                         # takes the first 64 KB of scratch
+
+    free, tight = _pair(spec, 5, start)
+    held = tight.device_bytes
+    ids = np.arange(n) % 5
+    a, b = free.pois_loglik(ids), tight.pois_loglik(ids)
+    assert free.device_bytes > held and tight.device_bytes == held
+    assert _error(tight) == ""
+    if n == 512:
+        assert np.array_equal(a, b)                 # the same chunks, fewer instances at a time
+    else:
+        # One sum of 72,000 terms instead of 18: 72,000 x 2^-53 of the terms' magnitude (about |a|, all of one sign
+        # but for log lam above 1).
+        assert np.all(np.abs(a - b) <= 1e-10 * np.abs(a))
+    free.close()
+    tight.close()
