@@ -1501,14 +1501,20 @@ int beep_obs_loglik(beep_ctx* c, int n, const int32_t* inst, int section, double
     std::vector<beep_ctx*> cs(1, c);
     std::vector<const int32_t*> ip(1, inst);
     std::vector<int> ni(1, n);
-    if ((rc = obs_loglik_chunked(c, cs, ip, ni, true, L_out, EF_dt_out, 2))) return rc;
-    c->timing[1] = elapsed(c, 2, 3);
-    for (int i = 0; i < n; i++)
-      if (std::isnan(L_out[i])) return fail(c, BEEP_ENAN, "NaN observation log-likelihood");   // obsmodel.cc:32
-    return BEEP_OK;
+    const std::string err = c->err;
+    rc = obs_loglik_chunked(c, cs, ip, ni, true, L_out, EF_dt_out, 2);
+    if (rc != BEEP_ENOMEM) {
+      if (rc) return rc;
+      c->timing[1] = elapsed(c, 2, 3);
+      for (int i = 0; i < n; i++)
+        if (std::isnan(L_out[i])) return fail(c, BEEP_ENAN, "NaN observation log-likelihood");   // obsmodel.cc:32
+      return BEEP_OK;
+    }
+    c->err = err;      // no room for the chunk sums: as a section that holds every observation
   }
   const int ndt = c->m.ndatatable;
-  const int nsel = c->sec_ptr[section + 1] - c->sec_ptr[section];
+  const int* sel = section < 0 ? nullptr : c->d_sec_obs + c->sec_ptr[section];
+  const int nsel = section < 0 ? c->obs.nobs : c->sec_ptr[section + 1] - c->sec_ptr[section];
   int nchunk = EF_dt_out ? 1 : section_chunks(nsel);
   auto doubles = [&] { return EF_dt_out ? (size_t)n * (1 + ndt) : (size_t)n * nchunk; };
   auto bytes = [&] { return doubles() * sizeof(double) + (size_t)n * sizeof(int); };
@@ -1519,7 +1525,7 @@ int beep_obs_loglik(beep_ctx* c, int n, const int32_t* inst, int section, double
   int* d_inst = (int*)(d_out + out_doubles);
   HIPCHK(c, hipMemcpyAsync(d_inst, inst, n * sizeof(int), hipMemcpyHostToDevice, c->stream));
   record(c, 2);
-  launch_obs_loglik(c, n, d_inst, c->d_sec_obs + c->sec_ptr[section], nsel, nchunk, d_out, EF_dt_out != nullptr);
+  launch_obs_loglik(c, n, d_inst, sel, nsel, nchunk, d_out, EF_dt_out != nullptr);
   HIPCHK(c, hipGetLastError());
   record(c, 3);
   std::vector<double> h(out_doubles);
@@ -1530,6 +1536,17 @@ int beep_obs_loglik(beep_ctx* c, int n, const int32_t* inst, int section, double
     const size_t row = EF_dt_out ? 1 + ndt : 1;
     L_out[i] = h[i * row];
     for (int k = 1; k < nchunk; k++) L_out[i] += h[(size_t)k * n + i];
+  }
+  if (section < 0) {               // every observation: the instances' error functions too
+    std::vector<double> ef(n);
+    for (int i = 0; i < n; i++) {
+      ef[i] = -2.0 * L_out[i];
+      HIPCHK(c, hipMemcpyAsync(c->d_EF + inst[i], &ef[i], sizeof(double), hipMemcpyHostToDevice, c->stream));
+    }
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+  }
+  for (int i = 0; i < n; i++) {
+    const size_t row = EF_dt_out ? 1 + ndt : 1;
     if (std::isnan(L_out[i])) return fail(c, BEEP_ENAN, "NaN observation log-likelihood");   // obsmodel.cc:32
     if (EF_dt_out)
       for (int d = 0; d < ndt; d++) EF_dt_out[(size_t)i * ndt + d] = h[i * row + 1 + d];

@@ -4,7 +4,7 @@ keeps the scratch that was held and leaves no error text behind."""
 import numpy as np
 import pytest
 
-from beep_amd import _lib, configs
+from beep_amd import _lib, configs, spec as specmod
 
 pytestmark = pytest.mark.gpu
 
@@ -95,5 +95,38 @@ def test_state_likelihood_within_held_scratch(gpu_lib, n):
         # One sum of 72,000 terms instead of 18: 72,000 x 2^-53 of the terms' magnitude (about |a|, all of one sign
         # but for log lam above 1).
         assert np.all(np.abs(a - b) <= 1e-10 * np.abs(a))
+    free.close()
+    tight.close()
+
+
+@pytest.mark.parametrize("dt", [True, False])
+def test_observations_within_held_scratch(gpu_lib, dt):
+    """2,000 instances of two data tables: their chunk sums pass 64 KB, the sums
+    of whole lists do not; the error functions are stored either way."""
+    spec, truth = configs.seir_areas(12, 1, 30, seed=3, daily_obs=True)
+    spec = specmod.expand_obs(spec)
+    for k, o in enumerate(spec["obs"]):
+        o["datatable"] = k % 2
+
+    def start(ctx):
+        ctx.set_param([0], truth[None, :])
+        ctx.simulate(range(5), [0] * 5, range(5, 10), seed=4)
+        ctx.obs_loglik([0])                         # takes the first 64 KB of scratch
+
+    free, tight = _pair(spec, 5, start)
+    held = tight.device_bytes
+    ids = np.arange(2000 if dt else 4800) % 5
+    a, b = free.obs_loglik(ids, with_dt=dt), tight.obs_loglik(ids, with_dt=dt)
+    assert free.device_bytes > held and tight.device_bytes == held
+    assert _error(tight) == ""
+    if dt:
+        assert np.all(np.abs(a[1] - b[1]) <= 1e-12 * np.abs(a[1]))      # a few hundred FP64 terms of one sign
+        a, b = a[0], b[0]
+    assert np.all(np.abs(a - b) <= 1e-12 * np.abs(a))
+    pairs = [0, 1, 2, 3, 4], [1, 2, 3, 4, 0]
+    acc = [ctx.accept(*pairs, mode=1, dlogq=np.zeros(5), key=np.arange(5), invT=1e-3)[0] for ctx in (free, tight)]
+    # exp of invT / 2 times differences of error functions, each to 1e-12 of its size.
+    assert np.all(np.abs(acc[0] - acc[1]) <= 1e-12 * (1 + 2 * np.abs(a).max()) * acc[0])
+    assert len(set(np.round(acc[0], 12))) > 2
     free.close()
     tight.close()
