@@ -11,6 +11,7 @@
 #include <sstream>
 #include <map>
 #include <mutex>
+#include <shared_mutex>
 #include <tuple>
 #include <cmath>
 #include <cstdarg>
@@ -158,10 +159,16 @@ constexpr int kMaxDevices = 64;
 // mask (here of every unit) has a queue of its own (16 launches of 16
 // workgroups each: 22.8 ms on 16 ordinary streams, 5.7 ms on 16 masked ones,
 // 6.1 ms for one launch).  Batches of several host threads share the streams:
-// each joins on events of its own.
+// each places its launches by what all of them have queued (BatchLease) and
+// joins on events of its own.  Twelve: a sweep over 1,120 unlike instances, whose
+// longest launch lasts 10.9 ms, takes 24.8 ms on 4 streams, 16.2 on 8, 12.7 on 12
+// and 12.3 on 16, and each costs 3.6 ms to make.
 constexpr int kBatchStreams = 12;
 struct BatchStreams {
   std::vector<hipStream_t> st;
+  std::vector<double> load;        // cost of the launches placed and not yet joined
+  std::vector<int> queued;         // and their number
+  size_t wanted = 0;               // launches of the batches under way
   int users = 0;                   // contexts of the device
 };
 std::mutex g_bstream_mu;
@@ -1078,6 +1085,8 @@ int beep_destroy(beep_ctx* c) {
         (void)hipStreamDestroy(st);
       }
       b.st.clear();
+      b.load.clear();
+      b.queued.clear();
     }
   }
   if (c->bstart) (void)hipEventDestroy(c->bstart);
@@ -2197,7 +2206,8 @@ struct TuneKey {
     return std::tie(ag2, C, T, spec, mode) < std::tie(o.ag2, o.C, o.T, o.spec, o.mode);
   }
 };
-std::mutex g_tune_mu;
+std::shared_mutex g_tune_mu;       // the table: shared by batches under way, exclusive while one is tuned
+std::mutex g_tune_gate;
 std::map<TuneKey, int> g_tune;
 bool g_tune_loaded = false;
 
@@ -2236,38 +2246,100 @@ int pow2_ceil(int x) {
   return p;
 }
 
-// `want` of the device's batch streams, at most kBatchStreams (made as batches
-// first want them: 4.5 ms each), and c0's events.
-int ensure_bstreams(beep_ctx* c0, size_t want, std::vector<hipStream_t>& out) {
-  want = std::min<size_t>(want, kBatchStreams);
-  {
+// A batch's use of its device's batch streams: every launch goes to the stream
+// with the least work queued by any thread's batch (two threads with one launch
+// of 5.1 ms each: 5.3 ms for both, 10.4 one after the other).  Destroyed, it gives back what it placed, and waits for it where the
+// batch did not reach join().
+class BatchLease {
+ public:
+  explicit BatchLease(beep_ctx* c0) : c0_(c0), b_(g_bstream[c0->device]) {}
+  BatchLease(const BatchLease&) = delete;
+  BatchLease& operator=(const BatchLease&) = delete;
+  ~BatchLease() {
+    if (!joined_)
+      for (int k : used_) (void)hipStreamSynchronize(stream(k));
     std::lock_guard<std::mutex> lk(g_bstream_mu);
-    BatchStreams& b = g_bstream[c0->device];
-    if (b.st.size() < want) {
-      hipDeviceProp_t prop;
-      HIPCHK(c0, hipGetDeviceProperties(&prop, c0->device));
-      const int ncu = prop.multiProcessorCount;
-      std::vector<uint32_t> mask((ncu + 31) / 32, 0u);
-      for (int i = 0; i < ncu; i++) mask[i / 32] |= 1u << (i % 32);
-      while (b.st.size() < want) {
+    b_.wanted -= want_;
+    for (const auto& p : placed_) b_.load[p.first] = --b_.queued[p.first] == 0 ? 0.0 : b_.load[p.first] - p.second;
+  }
+
+  // The batch's launches, `want` of them: streams for the launches of every
+  // batch under way, up to kBatchStreams (made as batches first want them: 3.6 ms
+  // each, and 3.1 to destroy).  The launches start after what c0's stream holds
+  // now, from where its timing event 0 is taken.
+  int start(size_t want) {
+    HIPCHK(c0_, hipSetDevice(c0_->device));
+    {
+      std::lock_guard<std::mutex> lk(g_bstream_mu);
+      b_.wanted += want_ = want;
+      std::vector<uint32_t> mask;
+      while (b_.st.size() < std::min<size_t>(b_.wanted, kBatchStreams)) {
+        if (mask.empty()) {
+          hipDeviceProp_t prop;
+          HIPCHK(c0_, hipGetDeviceProperties(&prop, c0_->device));
+          mask.assign((prop.multiProcessorCount + 31) / 32, 0u);
+          for (int i = 0; i < prop.multiProcessorCount; i++) mask[i / 32] |= 1u << (i % 32);
+        }
         hipStream_t st = nullptr;
         if (hipExtStreamCreateWithCUMask(&st, (uint32_t)mask.size(), mask.data()) != hipSuccess) {
           (void)hipGetLastError();
-          HIPCHK(c0, hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+          HIPCHK(c0_, hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
         }
-        b.st.push_back(st);
+        b_.st.push_back(st);
+        b_.load.push_back(0.0);
+        b_.queued.push_back(0);
       }
     }
-    out.assign(b.st.begin(), b.st.begin() + want);
+    if (!c0_->bstart) HIPCHK(c0_, hipEventCreateWithFlags(&c0_->bstart, hipEventDisableTiming));
+    record(c0_, 0);
+    HIPCHK(c0_, hipEventRecord(c0_->bstart, c0_->stream));
+    return BEEP_OK;
   }
-  if (!c0->bstart) HIPCHK(c0, hipEventCreateWithFlags(&c0->bstart, hipEventDisableTiming));
-  while (c0->bend.size() < out.size()) {
-    hipEvent_t e = nullptr;
-    HIPCHK(c0, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    c0->bend.push_back(e);
+
+  // The stream of a launch of the given cost.
+  int place(double cost, hipStream_t* out) {
+    int k;
+    {
+      std::lock_guard<std::mutex> lk(g_bstream_mu);
+      k = (int)(std::min_element(b_.load.begin(), b_.load.end()) - b_.load.begin());
+      b_.load[k] += cost;
+      b_.queued[k]++;
+      placed_.emplace_back(k, cost);
+    }
+    *out = stream(k);
+    if (std::find(used_.begin(), used_.end(), k) != used_.end()) return BEEP_OK;
+    HIPCHK(c0_, hipStreamWaitEvent(*out, c0_->bstart, 0));
+    used_.push_back(k);
+    return BEEP_OK;
   }
-  return BEEP_OK;
-}
+
+  // c0's stream goes on after everything placed.
+  int join() {
+    while (c0_->bend.size() < used_.size()) {
+      hipEvent_t e = nullptr;
+      HIPCHK(c0_, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      c0_->bend.push_back(e);
+    }
+    for (size_t i = 0; i < used_.size(); i++) {
+      HIPCHK(c0_, hipEventRecord(c0_->bend[i], stream(used_[i])));
+      HIPCHK(c0_, hipStreamWaitEvent(c0_->stream, c0_->bend[i], 0));
+    }
+    joined_ = true;
+    return BEEP_OK;
+  }
+
+ private:
+  hipStream_t stream(int k) {
+    std::lock_guard<std::mutex> lk(g_bstream_mu);      // another thread may be adding streams
+    return b_.st[k];
+  }
+  beep_ctx* c0_;
+  BatchStreams& b_;
+  size_t want_ = 0;
+  std::vector<std::pair<int, double>> placed_;
+  std::vector<int> used_;
+  bool joined_ = false;
+};
 
 // ObservationModel::calculate (src/obsmodel.cc:22-109) of every item's
 // instance after a batch: per context one observation-kernel launch over its
@@ -2584,17 +2656,22 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
     // instances of one launch overlap the next launch instead of leaving the
     // device idle; each stream starts after the job upload.  (Autotuning
     // launches run alone on the context stream to be timed.)
-    std::vector<hipStream_t> bst;
-    if ((rc = ensure_bstreams(c0, launches.size(), bst))) return rc;
-    const int nbs = (int)bst.size();
-    std::vector<double> load(nbs, 0.0);
     // The fused phase is timed on the context stream from before the batch
     // streams start to after they have all ended (timing[0]).
-    record(c0, 0);
-    HIPCHK(c0, hipEventRecord(c0->bstart, c0->stream));
-    for (int k = 0; k < nbs; k++) HIPCHK(c0, hipStreamWaitEvent(bst[k], c0->bstart, 0));
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    tune_load();
+    const bool autotune = (flags & BEEP_BATCH_AUTOTUNE) != 0;
+    BatchLease lease(c0);
+    if ((rc = lease.start(autotune ? 0 : launches.size()))) return rc;
+    // An autotuning call has the batch kernels to itself, so that the timed
+    // candidates run alone; other batches run side by side.  The gate lets no
+    // batch past a waiting autotuning call.
+    std::shared_lock<std::shared_mutex> beside(g_tune_mu, std::defer_lock);
+    std::unique_lock<std::shared_mutex> alone(g_tune_mu, std::defer_lock);
+    {
+      std::lock_guard<std::mutex> gate(g_tune_gate);
+      tune_load();
+      if (autotune) alone.lock();
+      else beside.lock();
+    }
     bool tuned_any = false;
     for (auto& L : launches) {
       const TuneKey key = std::get<0>(L);
@@ -2612,7 +2689,7 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
       int block = sk ? spec_block(maxAG) : fused_block(maxAG);
       auto f = g_tune.find(key);
       if (f != g_tune.end()) block = f->second;
-      else if ((flags & BEEP_BATCH_AUTOTUNE) && rerunnable) {
+      else if (autotune && rerunnable) {
         // Same keys give the same trajectories whatever the workgroup size,
         // and every job of the class starts from the initial state (t0 = 0:
         // simulations from the start, MBPs), so each candidate run recomputes
@@ -2649,24 +2726,17 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
       // An autotuning call keeps every launch on the context stream, so that
       // the timed candidates run alone.
       hipStream_t st = nullptr;
-      if (!(flags & BEEP_BATCH_AUTOTUNE)) {
-        const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        load[k] += std::get<7>(L);
-        st = bst[k];
-      }
+      if (!autotune && (rc = lease.place(std::get<7>(L), &st))) return rc;
       if ((rc = launch_any(block, st))) return rc;
       nlaunch++;
     }
     if (tuned_any) tune_save();
-    // Join: the context stream waits for every batch stream, then records the
-    // end of the fused phase.
-    for (int k = 0; k < nbs; k++) {
-      HIPCHK(c0, hipEventRecord(c0->bend[k], bst[k]));
-      HIPCHK(c0, hipStreamWaitEvent(c0->stream, c0->bend[k], 0));
-    }
+    // Join: the context stream waits for every batch stream used, then records
+    // the end of the fused phase.
+    if ((rc = lease.join())) return rc;
     record(c0, 1);
     HIPCHK(c0, hipStreamSynchronize(c0->stream));   // `all` is the source of an async copy
-    c0->timing[0] = (flags & BEEP_BATCH_AUTOTUNE) ? -1 : elapsed(c0, 0, 1);
+    c0->timing[0] = autotune ? -1 : elapsed(c0, 0, 1);
     c0->timing[3] = nlaunch;
   }
   HIPCHK(c0, hipStreamSynchronize(c0->stream));   // also keeps `all` alive until its copy is done
