@@ -163,6 +163,13 @@ constexpr int kMaxDevices = 64;
 // joins on events of its own.  Twelve: a sweep over 1,120 unlike instances, whose
 // longest launch lasts 10.9 ms, takes 24.8 ms on 4 streams, 16.2 on 8, 12.7 on 12
 // and 12.3 on 16, and each costs 3.6 ms to make.
+//
+// A masked stream is made without flags, so it is a blocking one: work on the
+// null stream waits for what the batch streams hold and keeps back what they are
+// given later (a copy beside a 53 ms kernel: 53 ms on the null stream, 0.05 ms on
+// a non-blocking one).  The library itself queues nothing there: contexts use
+// their own stream, entry points without one side_stream.  A program's own
+// null-stream work does order with the batches under way.
 constexpr int kBatchStreams = 12;
 struct BatchStreams {
   std::vector<hipStream_t> st;
@@ -173,6 +180,30 @@ struct BatchStreams {
 };
 std::mutex g_bstream_mu;
 BatchStreams g_bstream[kMaxDevices];
+
+// The stream of entry points without a context: one per device, made when first
+// wanted, kept until the process ends.
+std::mutex g_side_mu;
+hipStream_t g_side[kMaxDevices] = {};
+
+// With `device` made current.
+bool side_stream(int device, hipStream_t* out) {
+  if (hipSetDevice(device) != hipSuccess || device < 0 || device >= kMaxDevices) return false;
+  std::lock_guard<std::mutex> lk(g_side_mu);
+  if (!g_side[device] && hipStreamCreateWithFlags(&g_side[device], hipStreamNonBlocking) != hipSuccess) {
+    g_side[device] = nullptr;
+    return false;
+  }
+  *out = g_side[device];
+  return true;
+}
+
+// A copy on st, finished on return.
+hipError_t copy_on(hipStream_t st, void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+  hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, st);
+  const hipError_t w = hipStreamSynchronize(st);
+  return e != hipSuccess ? e : w;
+}
 
 std::mutex g_noalloc_mu;
 void* g_noalloc_ptr[kMaxDevices] = {};
@@ -214,7 +245,7 @@ int upload(beep_ctx* c, T** d, const std::vector<T>& h) {
   size_t bytes = std::max<size_t>(1, h.size()) * sizeof(T);
   int rc = dalloc(c, (void**)d, bytes);
   if (rc) return rc;
-  if (!h.empty()) HIPCHK(c, hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+  if (!h.empty()) HIPCHK(c, copy_on(c->stream, *d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
   return BEEP_OK;
 }
 
@@ -714,19 +745,20 @@ int put_jobs(beep_ctx* c, const std::vector<Job>& jobs) {
 template <class F>
 int debug_run(int device, size_t in_bytes, const void* in, size_t in2_bytes, const void* in2, size_t out_bytes, void* out,
               F launch) {
-  if (hipSetDevice(device) != hipSuccess) return BEEP_EHIP;
+  hipStream_t st = nullptr;
+  if (!side_stream(device, &st)) return BEEP_EHIP;
   void *d_in = nullptr, *d_in2 = nullptr, *d_out = nullptr;
   int rc = BEEP_OK;
   if (hipMalloc(&d_in, in_bytes) != hipSuccess || hipMalloc(&d_out, out_bytes) != hipSuccess ||
       (in2_bytes && hipMalloc(&d_in2, in2_bytes) != hipSuccess))
     rc = BEEP_ENOMEM;
-  if (!rc && hipMemcpy(d_in, in, in_bytes, hipMemcpyHostToDevice) != hipSuccess) rc = BEEP_EHIP;
-  if (!rc && in2_bytes && hipMemcpy(d_in2, in2, in2_bytes, hipMemcpyHostToDevice) != hipSuccess) rc = BEEP_EHIP;
+  if (!rc && copy_on(st, d_in, in, in_bytes, hipMemcpyHostToDevice) != hipSuccess) rc = BEEP_EHIP;
+  if (!rc && in2_bytes && copy_on(st, d_in2, in2, in2_bytes, hipMemcpyHostToDevice) != hipSuccess) rc = BEEP_EHIP;
   if (!rc) {
-    launch(d_in, d_in2, d_out);
-    if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) rc = BEEP_EHIP;
+    launch(st, d_in, d_in2, d_out);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) rc = BEEP_EHIP;
   }
-  if (!rc && hipMemcpy(out, d_out, out_bytes, hipMemcpyDeviceToHost) != hipSuccess) rc = BEEP_EHIP;
+  if (!rc && copy_on(st, out, d_out, out_bytes, hipMemcpyDeviceToHost) != hipSuccess) rc = BEEP_EHIP;
   if (d_in) (void)hipFree(d_in);
   if (d_in2) (void)hipFree(d_in2);
   if (d_out) (void)hipFree(d_out);
@@ -934,7 +966,7 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
     return fail(c, BEEP_EINVAL, "R or external-force splines per area or strain run on the specialised kernels only "
                                 "(not BEEP_GENERIC_KERNEL)");
   if ((rc = dalloc(c, (void**)&c->d_topo, sizeof(TopoDev)))) return rc;
-  HIPCHK(c, hipMemcpy(c->d_topo, &tp, sizeof tp, hipMemcpyHostToDevice));
+  HIPCHK(c, copy_on(c->stream, c->d_topo, &tp, sizeof tp, hipMemcpyHostToDevice));
   c->Apad = (m.A + 63) / 64 * 64;
   if (c->dense) {
     // The GEMM's right operand: M transposed, in fragment order (Mt[j][a] = M[a][j]).
@@ -950,14 +982,14 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
     const size_t rows_pad = ((size_t)capacity * m.G + 63) / 64 * 64;
     size_t szD = rows_pad * c->Apad * sizeof(float), sz = (size_t)capacity * m.G * c->Apad * sizeof(float);
     if ((rc = dalloc(c, (void**)&c->d_D, szD)) || (rc = dalloc(c, (void**)&c->d_I, sz))) return rc;
-    HIPCHK(c, hipMemset(c->d_D, 0, szD));
-    HIPCHK(c, hipMemset(c->d_I, 0, sz));
+    HIPCHK(c, hipMemsetAsync(c->d_D, 0, szD, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->d_I, 0, sz, c->stream));
     if ((rc = dalloc(c, (void**)&c->d_rngp, 2 * sizeof(uint64_t)))) return rc;
   }
 
   // Slots and instances.
   if ((rc = dalloc(c, (void**)&c->d_tab, c->slot_stride * nslot * sizeof(float)))) return rc;
-  HIPCHK(c, hipMemset(c->d_tab, 0, c->slot_stride * nslot * sizeof(float)));
+  HIPCHK(c, hipMemsetAsync(c->d_tab, 0, c->slot_stride * nslot * sizeof(float), c->stream));
   c->slot_param.assign((size_t)nslot * m.nparam, 0.0);
   c->slot_set.assign(nslot, 0);
   c->inst_slot.assign(capacity, -1);
@@ -965,7 +997,7 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
   if (c->nospl) {
     size_t sz = (size_t)nslot * c->nospl * m.S * sizeof(double);
     if ((rc = dalloc(c, (void**)&c->d_ospl, sz))) return rc;
-    HIPCHK(c, hipMemset(c->d_ospl, 0, sz));
+    HIPCHK(c, hipMemsetAsync(c->d_ospl, 0, sz, c->stream));
     if ((rc = dalloc(c, (void**)&c->d_inst_slot, capacity * sizeof(int)))) return rc;
     c->inst_slot_dirty = true;
   }
@@ -977,23 +1009,23 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
   // simulation does not reach read as zero).
   if (keep & BEEP_KEEP_TRANSNUM) {
     if ((rc = dalloc(c, (void**)&c->d_tn, c->traj_sz * capacity * sizeof(int)))) return rc;
-    HIPCHK(c, hipMemset(c->d_tn, 0, c->traj_sz * capacity * sizeof(int)));
+    HIPCHK(c, hipMemsetAsync(c->d_tn, 0, c->traj_sz * capacity * sizeof(int), c->stream));
   }
   if (keep & BEEP_KEEP_TRANSMEAN) {
     if ((rc = dalloc(c, (void**)&c->d_tm, c->traj_sz * capacity * sizeof(float)))) return rc;
-    HIPCHK(c, hipMemset(c->d_tm, 0, c->traj_sz * capacity * sizeof(float)));
+    HIPCHK(c, hipMemsetAsync(c->d_tm, 0, c->traj_sz * capacity * sizeof(float), c->stream));
   }
   if (keep & BEEP_KEEP_POP) {
     if ((rc = dalloc(c, (void**)&c->d_pt, c->pop_traj_sz * capacity * sizeof(int)))) return rc;
-    HIPCHK(c, hipMemset(c->d_pt, 0, c->pop_traj_sz * capacity * sizeof(int)));
+    HIPCHK(c, hipMemsetAsync(c->d_pt, 0, c->pop_traj_sz * capacity * sizeof(int), c->stream));
   }
   if ((rc = dalloc(c, (void**)&c->d_EF, capacity * sizeof(double)))) return rc;
-  HIPCHK(c, hipMemset(c->d_EF, 0, capacity * sizeof(double)));
+  HIPCHK(c, hipMemsetAsync(c->d_EF, 0, capacity * sizeof(double), c->stream));
   if ((rc = dalloc(c, (void**)&c->d_err, sizeof(int)))) return rc;
-  HIPCHK(c, hipMemset(c->d_err, 0, sizeof(int)));
+  HIPCHK(c, hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream));
   for (int i = 0; i < capacity; i++)
-    HIPCHK(c, hipMemcpy(c->d_state + (size_t)i * c->state_sz, d_pop_init, c->state_sz * sizeof(int),
-                        hipMemcpyDeviceToDevice));
+    HIPCHK(c, hipMemcpyAsync(c->d_state + (size_t)i * c->state_sz, d_pop_init, c->state_sz * sizeof(int),
+                             hipMemcpyDeviceToDevice, c->stream));
 
   // Observations.  They are stored on the device in the order of their
   // first element, so that neighbouring lanes of the likelihood kernel read
@@ -1043,7 +1075,7 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
     od.nospl = c->nospl;
     od.S = m.S;
     if ((rc = dalloc(c, (void**)&c->d_obs, sizeof(beepdev::ObsDev)))) return rc;
-    HIPCHK(c, hipMemcpy(c->d_obs, &od, sizeof od, hipMemcpyHostToDevice));
+    HIPCHK(c, copy_on(c->stream, c->d_obs, &od, sizeof od, hipMemcpyHostToDevice));
     // Data tables and sections as lists of stored positions, ascending.
     std::vector<int> dt_obs;
     c->dt_ptr.assign(1, 0);
@@ -1066,6 +1098,7 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
         (rc = upload(c, &c->d_sec_ti, m.section_ti)) || (rc = upload(c, &c->d_sec_tf, m.section_tf)))
       return rc;
   }
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   return BEEP_OK;
 }
 
@@ -2077,7 +2110,8 @@ int beep_abcsmc_weights(int device, int nvar, int n_prev, const double* prev, co
       (n_new > 0 && (!theta || !logprior || !w_out)))
     return BEEP_EINVAL;
   if (n_new == 0) return BEEP_OK;
-  if (hipSetDevice(device) != hipSuccess) return BEEP_EHIP;
+  hipStream_t st = nullptr;
+  if (!side_stream(device, &st)) return BEEP_EHIP;
   // One upload: the previous particles and the proposals in rows of NV, the
   // weights, the triangle U of the quadratic form (k_abcsmc_partial), the
   // log priors.
@@ -2109,7 +2143,7 @@ int beep_abcsmc_weights(int device, int nvar, int n_prev, const double* prev, co
   double* d_part = d + n_in;
   double* d_out = d_part + (size_t)n_new * nsplit;
   int rc = BEEP_OK;
-  if (hipMemcpy(d, h.data(), n_in * 8, hipMemcpyHostToDevice) != hipSuccess) rc = BEEP_EHIP;
+  if (copy_on(st, d, h.data(), n_in * 8, hipMemcpyHostToDevice) != hipSuccess) rc = BEEP_EHIP;
   if (!rc) {
     using K = decltype(&beepdev::k_abcsmc_partial<2>);
     static const K ks[16] = {
@@ -2119,12 +2153,13 @@ int beep_abcsmc_weights(int device, int nvar, int n_prev, const double* prev, co
         beepdev::k_abcsmc_partial<20>, beepdev::k_abcsmc_partial<22>, beepdev::k_abcsmc_partial<24>,
         beepdev::k_abcsmc_partial<26>, beepdev::k_abcsmc_partial<28>, beepdev::k_abcsmc_partial<30>,
         beepdev::k_abcsmc_partial<32>};
-    hipLaunchKernelGGL(ks[NV / 2 - 1], dim3((unsigned)nb, (unsigned)nsplit), dim3(BEEP_ABC_BLOCK), 0, 0, n_prev, jper,
+    hipLaunchKernelGGL(ks[NV / 2 - 1], dim3((unsigned)nb, (unsigned)nsplit), dim3(BEEP_ABC_BLOCK), 0, st, n_prev, jper,
                        (const double*)d, (const double*)(d + o_w), n_new, (const double*)(d + o_th),
                        (const double*)(d + o_U), d_part);
-    hipLaunchKernelGGL(beepdev::k_abcsmc_finish, dim3((unsigned)nb), dim3(BEEP_ABC_BLOCK), 0, 0, n_new, nsplit,
+    hipLaunchKernelGGL(beepdev::k_abcsmc_finish, dim3((unsigned)nb), dim3(BEEP_ABC_BLOCK), 0, st, n_new, nsplit,
                        (const double*)d_part, (const double*)(d + o_lp), d_out);
-    if (hipGetLastError() != hipSuccess || hipMemcpy(w_out, d_out, (size_t)n_new * 8, hipMemcpyDeviceToHost) != hipSuccess)
+    if (hipGetLastError() != hipSuccess ||
+        copy_on(st, w_out, d_out, (size_t)n_new * 8, hipMemcpyDeviceToHost) != hipSuccess)
       rc = BEEP_EHIP;
   }
   (void)hipFree(d);
@@ -2165,7 +2200,8 @@ int beep_bootstrap(int device, int n, const double* L, double invT, uint64_t see
                    int32_t* bp_out, double* obprob_out) {
   if (n <= 0 || !L || !bp_out || !obprob_out || stream > 0xFFFF || sec < 0 || !(invT >= 0) || !std::isfinite(invT))
     return BEEP_EINVAL;
-  if (hipSetDevice(device) != hipSuccess) return BEEP_EHIP;
+  hipStream_t st = nullptr;
+  if (!side_stream(device, &st)) return BEEP_EHIP;
   const size_t bytes = 16 + (size_t)n * (8 + 8 + 4 * 4);     // estimate, error flag, L, wsum, 4 int arrays
   char* d = nullptr;
   if (hipMalloc((void**)&d, bytes) != hipSuccess) return BEEP_ENOMEM;
@@ -2178,15 +2214,16 @@ int beep_bootstrap(int device, int n, const double* L, double invT, uint64_t see
   int* d_draw = d_first + n;
   int* d_extra = d_draw + n;
   int rc = BEEP_OK, err = 0;
-  if (hipMemset(d, 0, 16) != hipSuccess || hipMemcpy(d_L, L, n * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
+  if (hipMemsetAsync(d, 0, 16, st) != hipSuccess ||
+      copy_on(st, d_L, L, n * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
     rc = BEEP_EHIP;
   if (!rc) {
-    launch_bootstrap(nullptr, n, d_L, 1, invT, seed, stream, sec, d_bp, d_w, d_first, d_draw, d_extra, d_ob, d_err);
-    if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) rc = BEEP_EHIP;
+    launch_bootstrap(st, n, d_L, 1, invT, seed, stream, sec, d_bp, d_w, d_first, d_draw, d_extra, d_ob, d_err);
+    if (hipGetLastError() != hipSuccess) rc = BEEP_EHIP;
   }
-  if (!rc && (hipMemcpy(bp_out, d_bp, n * sizeof(int), hipMemcpyDeviceToHost) != hipSuccess ||
-              hipMemcpy(obprob_out, d_ob, sizeof(double), hipMemcpyDeviceToHost) != hipSuccess ||
-              hipMemcpy(&err, d_err, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess))
+  if (!rc && (copy_on(st, bp_out, d_bp, n * sizeof(int), hipMemcpyDeviceToHost) != hipSuccess ||
+              copy_on(st, obprob_out, d_ob, sizeof(double), hipMemcpyDeviceToHost) != hipSuccess ||
+              copy_on(st, &err, d_err, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess))
     rc = BEEP_EHIP;
   (void)hipFree(d);
   if (!rc && err) rc = BEEP_ENAN;
@@ -2248,8 +2285,9 @@ int pow2_ceil(int x) {
 
 // A batch's use of its device's batch streams: every launch goes to the stream
 // with the least work queued by any thread's batch (two threads with one launch
-// of 5.1 ms each: 5.3 ms for both, 10.4 one after the other).  Destroyed, it gives back what it placed, and waits for it where the
-// batch did not reach join().
+// of 5.1 ms each: 5.3 ms for both, 10.4 one after the other).  Destroyed, it
+// gives back what it placed, and waits for it where the batch did not reach
+// join().
 class BatchLease {
  public:
   explicit BatchLease(beep_ctx* c0) : c0_(c0), b_(g_bstream[c0->device]) {}
@@ -2857,8 +2895,8 @@ int beep_synchronize(beep_ctx* c) {
 
 int beep_debug_philox(int device, int n, const uint32_t* ctr, uint32_t k0, uint32_t k1, uint32_t* out) {
   if (n <= 0 || !ctr || !out) return BEEP_EINVAL;
-  return debug_run(device, (size_t)n * 16, ctr, 0, nullptr, (size_t)n * 16, out, [&](void* a, void*, void* o) {
-    hipLaunchKernelGGL(beepdev::k_dbg_philox, dim3((n + 255) / 256), dim3(256), 0, 0, n, (const beepdev::u4*)a, k0, k1,
+  return debug_run(device, (size_t)n * 16, ctr, 0, nullptr, (size_t)n * 16, out, [&](hipStream_t st, void* a, void*, void* o) {
+    hipLaunchKernelGGL(beepdev::k_dbg_philox, dim3((n + 255) / 256), dim3(256), 0, st, n, (const beepdev::u4*)a, k0, k1,
                        (beepdev::u4*)o);
   });
 }
@@ -2867,8 +2905,8 @@ int beep_debug_poisson(int device, int n, const float* lam, uint64_t seed, uint3
   if (n <= 0 || !lam || !out) return BEEP_EINVAL;
   for (int i = 0; i < n; i++)
     if (!(lam[i] >= 0.f) || lam[i] > 1e9f) return BEEP_EINVAL;
-  return debug_run(device, (size_t)n * 4, lam, 0, nullptr, (size_t)n * 4, out, [&](void* a, void*, void* o) {
-    hipLaunchKernelGGL(beepdev::k_dbg_poisson, dim3((n + 255) / 256), dim3(256), 0, 0, n, (const float*)a, seed, key,
+  return debug_run(device, (size_t)n * 4, lam, 0, nullptr, (size_t)n * 4, out, [&](hipStream_t st, void* a, void*, void* o) {
+    hipLaunchKernelGGL(beepdev::k_dbg_poisson, dim3((n + 255) / 256), dim3(256), 0, st, n, (const float*)a, seed, key,
                        (int*)o);
   });
 }
@@ -2886,12 +2924,12 @@ int beep_debug_gemm(int device, int rows, int K, const float* A, const float* B,
   for (int k = 0; k < K; k++)
     for (int j = 0; j < K; j++) Btf[beepdev::frag_at(j, k, K)] = B[(size_t)k * K + j];
   return debug_run(device, Af.size() * 4, Af.data(), Btf.size() * 4, Btf.data(), (size_t)rows * K * 4, C,
-                   [&](void* a, void* b, void* o) {
+                   [&](hipStream_t st, void* a, void* b, void* o) {
                      if (beephost::narrow_tiles(tiles))
                        hipLaunchKernelGGL(beepdev::k_dbg_gemm<1>, dim3((unsigned)((2 * tiles + 7) / 8 * 8)), dim3(256), 0,
-                                          0, (const float*)a, (const float*)b, (float*)o, rows, K);
+                                          st, (const float*)a, (const float*)b, (float*)o, rows, K);
                      else
-                       hipLaunchKernelGGL(beepdev::k_dbg_gemm<2>, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, 0,
+                       hipLaunchKernelGGL(beepdev::k_dbg_gemm<2>, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, st,
                                           (const float*)a, (const float*)b, (float*)o, rows, K);
                    });
 }
@@ -2927,8 +2965,8 @@ int beep_debug_binomial(int device, int n, const int32_t* nn, const double* p, u
   if (n <= 0 || !nn || !p || !out) return BEEP_EINVAL;
   for (int i = 0; i < n; i++)
     if (nn[i] < 0 || !(p[i] > 0.0) || !(p[i] < 1.0)) return BEEP_EINVAL;
-  return debug_run(device, (size_t)n * 4, nn, (size_t)n * 8, p, (size_t)n * 4, out, [&](void* a, void* b, void* o) {
-    hipLaunchKernelGGL(beepdev::k_dbg_binomial, dim3((n + 255) / 256), dim3(256), 0, 0, n, (const int*)a,
+  return debug_run(device, (size_t)n * 4, nn, (size_t)n * 8, p, (size_t)n * 4, out, [&](hipStream_t st, void* a, void* b, void* o) {
+    hipLaunchKernelGGL(beepdev::k_dbg_binomial, dim3((n + 255) / 256), dim3(256), 0, st, n, (const int*)a,
                        (const double*)b, seed, key, (int*)o);
   });
 }
