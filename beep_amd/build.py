@@ -22,6 +22,7 @@ JIT_INC = os.path.join(CSRC, "jit_sources.inc")
 # time: SEIR (S->E, E->I, I->R, I infectious) with one strain, and the same
 # with two strains (which compiles the pooling of susceptibles).
 CHECK_PRELUDES = ["""#define BEEP_SPEC_FUSED
+#define BEEP_SPEC_REPLAY
 #define BEEP_SPEC_STEP
 namespace beepspec {
 constexpr int C = 4, T = 3, G = %d, CP = 4, INF_TR = 0, MIN_WAVES = 4, STEP_WAVES = 4, NSTRAIN = %d, DPM = 1;

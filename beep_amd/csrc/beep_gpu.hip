@@ -42,7 +42,7 @@ using beepdev::TopoDev;
 // of the process.
 struct SpecKernels {
   hipModule_t mod = nullptr;
-  hipFunction_t fn[3] = {};        // fused kernel, indexed by MODE_SIM / MBP / REPLAY
+  hipFunction_t fn[3] = {};        // fused kernel, indexed by MODE_SIM / MBP / REPLAY (null where nothing launches it)
   hipFunction_t step[3] = {};      // step-wise transition kernel, MODE_SIM / MBP / REPLAY
   int max_dyn_lds = 65536;         // dynamic LDS the fused kernels accept (the device's, less static use)
 };
@@ -455,7 +455,11 @@ std::string spec_prelude(const beep_ctx* c) {
 
 int spec_kernels(beep_ctx* c, SpecKernels** out) {
   // A context compiles the kernels of its own path only.
-  const std::string prelude = std::string(c->stepwise ? "#define BEEP_SPEC_STEP\n" : "#define BEEP_SPEC_FUSED\n") + spec_prelude(c);
+  // The fused replay kernel only where beep_put_transnum may come to it: with
+  // strains, or without kept populations (which then need scratch).
+  const bool replay = !c->stepwise && (c->m.nstrain > 1 || !(c->keep & BEEP_KEEP_POP));
+  const std::string prelude = std::string(c->stepwise ? "#define BEEP_SPEC_STEP\n" : "#define BEEP_SPEC_FUSED\n") +
+                              (replay ? "#define BEEP_SPEC_REPLAY\n" : "") + spec_prelude(c);
   const std::string key = std::to_string(c->device) + "\n" + prelude;
   std::lock_guard<std::mutex> lk(g_jit_mu);
   auto it = g_jit.find(key);
@@ -489,7 +493,8 @@ int spec_kernels(beep_ctx* c, SpecKernels** out) {
   auto* k = new SpecKernels();
   hipError_t e = hipModuleLoadData(&k->mod, code.data());
   const char* fn[3] = {"beep_fused_spec_sim", "beep_fused_spec_mbp", "beep_fused_spec_replay"};
-  for (int i = 0; e == hipSuccess && !c->stepwise && i < 3; i++) e = hipModuleGetFunction(&k->fn[i], k->mod, fn[i]);
+  const int nfn = c->stepwise ? 0 : replay ? 3 : 2;
+  for (int i = 0; e == hipSuccess && i < nfn; i++) e = hipModuleGetFunction(&k->fn[i], k->mod, fn[i]);
   const char* sn[3] = {"beep_step_spec_sim", "beep_step_spec_mbp", "beep_step_spec_replay"};
   for (int i = 0; e == hipSuccess && c->stepwise && i < 3; i++) e = hipModuleGetFunction(&k->step[i], k->mod, sn[i]);
   if (e != hipSuccess) {
@@ -497,7 +502,7 @@ int spec_kernels(beep_ctx* c, SpecKernels** out) {
     return fail(c, BEEP_EHIP, "loading the specialised kernel: %s", hipGetErrorString(e));
   }
   int lim = 0;
-  for (int i = 0; !c->stepwise && i < 3; i++) {
+  for (int i = 0; i < nfn; i++) {
     int v = 0;
     if (hipFuncGetAttribute(&v, HIP_FUNC_ATTRIBUTE_MAX_DYNAMIC_SHARED_SIZE_BYTES, k->fn[i]) == hipSuccess && v > 0)
       lim = i == 0 ? v : std::min(lim, v);

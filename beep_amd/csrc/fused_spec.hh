@@ -479,8 +479,10 @@ extern "C" __global__ void __launch_bounds__(BEEP_SPEC_MAX_BLOCK, beepspec::MIN_
     beep_fused_spec_mbp(const beepdev::Job* jobs, uint64_t seed, uint32_t stream) {
   beepdev::fused_spec_body<beepdev::MODE_MBP>(jobs, seed, stream);
 }
+#ifdef BEEP_SPEC_REPLAY
 extern "C" __global__ void __launch_bounds__(BEEP_SPEC_MAX_BLOCK, beepspec::MIN_WAVES)
     beep_fused_spec_replay(const beepdev::Job* jobs, uint64_t seed, uint32_t stream) {
   beepdev::fused_spec_body<beepdev::MODE_REPLAY>(jobs, seed, stream);
 }
+#endif
 #endif
