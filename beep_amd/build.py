@@ -2,6 +2,7 @@
 
 The library holds the device kernels, the C ABI of include/beep_gpu.h and the
 C++ host model (normalisation and parameter-derived tables)."""
+import hashlib
 import os
 import subprocess
 import sys
@@ -17,6 +18,8 @@ HEADERS = ["device_rng.hh", "fused_common.hh", "fused_spec.hh", "step_spec.hh", 
 # structure, embedded as string constants.
 JIT_HEADERS = [("kJitDeviceRng", "device_rng.hh"), ("kJitFusedCommon", "fused_common.hh"),
                ("kJitFusedSpec", "fused_spec.hh"), ("kJitStepSpec", "step_spec.hh")]
+# The fused kernels, generic and specialised: what tuned workgroup sizes hold for.
+TUNED_SOURCES = ["device_rng.hh", "fused_common.hh", "fused_spec.hh", "kernels.hh"]
 JIT_INC = os.path.join(CSRC, "jit_sources.inc")
 # Compartment structures the run-time compiled kernel is checked with at build
 # time: SEIR (S->E, E->I, I->R, I infectious) with one strain, and the same
@@ -45,13 +48,17 @@ def hipcc():
 
 
 def write_jit_sources():
-    """jit_sources.inc: the run-time compiled headers as raw string literals."""
+    """jit_sources.inc: the run-time compiled headers as raw string literals,
+    and a tag of the fused kernels' sources, under which tuned workgroup sizes
+    are saved."""
     out = ["// Generated by beep_amd/build.py from the headers named below; do not edit.\n"]
     for name, fn in JIT_HEADERS:
         text = open(os.path.join(CSRC, fn)).read()
         if ")BEEPJIT\"" in text:
             raise RuntimeError(f"{fn} contains the raw-string delimiter")
         out.append(f"static const char {name}[] = R\"BEEPJIT({text})BEEPJIT\";\n")
+    tag = hashlib.sha256("".join(open(os.path.join(CSRC, fn)).read() for fn in TUNED_SOURCES).encode()).hexdigest()[:16]
+    out.append(f"static const char kKernelTag[] = \"{tag}\";\n")
     tmp = JIT_INC + ".tmp"
     with open(tmp, "w") as f:
         f.write("".join(out))

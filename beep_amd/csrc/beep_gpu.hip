@@ -30,8 +30,8 @@
 #include "replay_kernels.hh"
 #include "step_kernels.hh"
 // kJitDeviceRng, kJitFusedCommon, kJitFusedSpec, kJitStepSpec: the texts of
-// device_rng.hh, fused_common.hh, fused_spec.hh and step_spec.hh (generated
-// by build.py).
+// device_rng.hh, fused_common.hh, fused_spec.hh and step_spec.hh; kKernelTag: a
+// hash of the fused kernels' sources (generated by build.py).
 #include "jit_sources.inc"
 
 using beepdev::Job;
@@ -45,6 +45,7 @@ struct SpecKernels {
   hipFunction_t fn[3] = {};        // fused kernel, indexed by MODE_SIM / MBP / REPLAY (null where nothing launches it)
   hipFunction_t step[3] = {};      // step-wise transition kernel, MODE_SIM / MBP / REPLAY
   int max_dyn_lds = 65536;         // dynamic LDS the fused kernels accept (the device's, less static use)
+  uint64_t id = 0;                 // hash of the prelude: names the kernels across processes, never 0
 };
 
 struct beep_ctx {
@@ -491,6 +492,9 @@ int spec_kernels(beep_ctx* c, SpecKernels** out) {
   hiprtcGetCode(prog, code.data());
   hiprtcDestroyProgram(&prog);
   auto* k = new SpecKernels();
+  k->id = 0xcbf29ce484222325ull;               // 64-bit FNV-1a
+  for (unsigned char ch : prelude) k->id = (k->id ^ ch) * 0x100000001b3ull;
+  k->id |= 1;
   hipError_t e = hipModuleLoadData(&k->mod, code.data());
   const char* fn[3] = {"beep_fused_spec_sim", "beep_fused_spec_mbp", "beep_fused_spec_replay"};
   const int nfn = c->stepwise ? 0 : replay ? 3 : 2;
@@ -2239,19 +2243,26 @@ int beep_bootstrap(int device, int n, const double* L, double invT, uint64_t see
 
 namespace {
 // A size class of a mixed batch: cells rounded up to a power of two, the
-// compartment structure, the kernel (specialised or generic) and the jobs'
+// compartment structure, the kernel (SpecKernels::id, 0 for the generic one: the
+// specialised kernels of one structure differ in registers and LDS with the
+// features compiled in, and with them in their best workgroup size) and the jobs'
 // mode (simulations and MBP proposals run as separate launches, each with the
 // kernel compiled for its mode alone, which needs fewer registers).
 struct TuneKey {
-  int ag2, C, T, spec, mode;
+  int ag2, C, T;
+  uint64_t kernel;
+  int mode;
   bool operator<(const TuneKey& o) const {
-    return std::tie(ag2, C, T, spec, mode) < std::tie(o.ag2, o.C, o.T, o.spec, o.mode);
+    return std::tie(ag2, C, T, kernel, mode) < std::tie(o.ag2, o.C, o.T, o.kernel, o.mode);
   }
 };
 std::shared_mutex g_tune_mu;       // the table: shared by batches under way, exclusive while one is tuned
 std::mutex g_tune_gate;
 std::map<TuneKey, int> g_tune;
 bool g_tune_loaded = false;
+
+// First line of the saved table: its format and the fused kernels' sources.
+constexpr char kTuneFormat[] = "beep-tune-4";
 
 const char* tune_path() {
   const char* p = std::getenv("BEEP_TUNE_CACHE");
@@ -2264,21 +2275,22 @@ void tune_load() {
   const char* p = tune_path();
   if (!p) return;
   std::ifstream f(p);
-  std::string ver;
-  if (!(f >> ver) || ver != "beep-tune-3") return;     // another format: ignored, rewritten on save
+  std::string ver, tag;
+  // Another format, or sizes tuned for other kernels: ignored, rewritten on save.
+  if (!(f >> ver >> tag) || ver != kTuneFormat || tag != kKernelTag) return;
   TuneKey k;
   int b;
-  while (f >> k.ag2 >> k.C >> k.T >> k.spec >> k.mode >> b)
-    if (b >= 64 && b <= (k.spec ? BEEP_SPEC_MAX_BLOCK : BEEP_FUSED_MAX_BLOCK) && b % 64 == 0) g_tune[k] = b;
+  while (f >> k.ag2 >> k.C >> k.T >> k.kernel >> k.mode >> b)
+    if (b >= 64 && b <= (k.kernel ? BEEP_SPEC_MAX_BLOCK : BEEP_FUSED_MAX_BLOCK) && b % 64 == 0) g_tune[k] = b;
 }
 
 void tune_save() {
   const char* p = tune_path();
   if (!p) return;
   std::ofstream f(p);
-  f << "beep-tune-3\n";
+  f << kTuneFormat << " " << kKernelTag << "\n";
   for (auto& kv : g_tune)
-    f << kv.first.ag2 << " " << kv.first.C << " " << kv.first.T << " " << kv.first.spec << " " << kv.first.mode << " "
+    f << kv.first.ag2 << " " << kv.first.C << " " << kv.first.T << " " << kv.first.kernel << " " << kv.first.mode << " "
       << kv.second << "\n";
 }
 
@@ -2656,7 +2668,7 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
     // structure; and mode), each sorted longest first.
     std::map<std::pair<TuneKey, SpecKernels*>, std::vector<Item>> groups;
     for (auto& it : fused)
-      groups[{{pow2_ceil(it.AG), it.ctx->m.C, it.ctx->m.T, it.spec ? 1 : 0, it.job.mode}, it.spec}].push_back(it);
+      groups[{{pow2_ceil(it.AG), it.ctx->m.C, it.ctx->m.T, it.spec ? it.spec->id : 0, it.job.mode}, it.spec}].push_back(it);
     std::vector<Job> all;
     // key, offset, count, lds, maxAG, kernel, every job starts from the initial state, the longest job's cost
     std::vector<std::tuple<TuneKey, size_t, size_t, size_t, int, SpecKernels*, bool, double>> launches;
