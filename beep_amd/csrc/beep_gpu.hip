@@ -77,7 +77,7 @@ struct beep_ctx {
   beepdev::ObsDev obs;
   beepdev::ObsDev* d_obs = nullptr;
   std::vector<int> dt_ptr;          // per data table: its stored observations d_dt_obs[dt_ptr[d] .. dt_ptr[d+1])
-  int* d_dt_obs = nullptr;
+  int* d_dt_obs = nullptr;          // null where the budget had no room for it
   std::vector<int> sec_ptr;
   int* d_sec_ptr = nullptr;
   int* d_sec_obs = nullptr;
@@ -1093,7 +1093,6 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
         if (dtab[k] == d) dt_obs.push_back(k);
       c->dt_ptr.push_back((int)dt_obs.size());
     }
-    if ((rc = upload(c, &c->d_dt_obs, dt_obs))) return rc;
     std::vector<int> sptr(1, 0), sobs;
     for (const auto& l : m.section_obs) {
       std::vector<int> v;
@@ -1106,6 +1105,13 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
     if ((rc = upload(c, &c->d_sec_ptr, sptr)) || (rc = upload(c, &c->d_sec_obs, sobs)) ||
         (rc = upload(c, &c->d_sec_ti, m.section_ti)) || (rc = upload(c, &c->d_sec_tf, m.section_tf)))
       return rc;
+    // The tables' lists last, where the budget has room for them: without them
+    // sums per table take every observation for each (k_obs_loglik).
+    if (!dt_obs.empty()) {
+      const std::string err = c->err;
+      if ((rc = upload(c, &c->d_dt_obs, dt_obs)) && rc != BEEP_ENOMEM) return rc;
+      c->err = err;
+    }
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return BEEP_OK;
@@ -2455,6 +2461,9 @@ int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const s
       return fail(c0, BEEP_EINVAL, "observation log-likelihood: too many chunks");
   }
   if (N == 0) return BEEP_OK;
+  if (out_dt)
+    for (const beep_ctx* c : ctxs)
+      if (c->dt_ptr.back() > 0 && !c->d_dt_obs) return fail(c0, BEEP_ENOMEM, "no room for the data tables' lists");
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t b_inst = al(N * sizeof(int32_t)), b_sets = al(nset * sizeof(ObsSet)), b_sums = al(nset * sizeof(ObsSum)),
                b_range = al(range.size() * sizeof(int2)), b_tab = al(tab.size() * sizeof(int));

@@ -130,3 +130,29 @@ def test_observations_within_held_scratch(gpu_lib, dt):
     assert len(set(np.round(acc[0], 12))) > 2
     free.close()
     tight.close()
+
+
+def test_context_without_room_for_table_lists(gpu_lib):
+    """The data tables' lists are 625 KB of a context that a budget without them
+    still serves."""
+    spec, truth = configs.seir_areas(400, 1, 400, seed=3, daily_obs=True)
+    spec = specmod.expand_obs(spec)
+    for k, o in enumerate(spec["obs"]):
+        o["datatable"] = k % 2
+    lists = 4 * len(spec["obs"])
+    assert lists == 640000
+    free = _lib.Context(spec, capacity=3, nslot=1)
+    tight = _lib.Context(spec, capacity=3, nslot=1, hbm_budget=free.device_bytes - lists + 500000)
+    assert tight.device_bytes == free.device_bytes - lists and _error(tight) == ""
+    out = []
+    for ctx in (free, tight):
+        ctx.set_param([0], truth[None, :])
+        ctx.simulate(range(3), [0] * 3, range(5, 8), seed=4)
+        out.append(ctx.obs_loglik([2, 0, 1], with_dt=True))
+    assert _error(tight) == ""
+    for a, b in zip(*out):
+        # 160,000 terms in another order: to 160,000 x 2^-53 of their magnitudes, at most some five times the sum.
+        assert np.all(np.abs(a - b) <= 1e-10 * np.abs(a))
+    assert np.array_equal(free.obs_loglik([1]), tight.obs_loglik([1]))
+    free.close()
+    tight.close()
