@@ -49,12 +49,19 @@ inline std::string fused_geometry(long long njobs, int block, size_t lds, size_t
 }
 
 // Whether a product of `tiles` tiles of 64x64 is done in tiles of 32 columns:
-// twice the workgroups of half the length, where those of 64 columns leave some
-// of the 256 CUs with one and others with two.  Contraction and transitions of a
-// step, 64 columns against 32: 45 tiles 21.9 and 18.5 us, 288 tiles 58.6 and
-// 56.5, 360 tiles 93.0 and 90.7, 510 tiles 125.1 and 126.3, 720 tiles 183.7 and
-// 182.9, 1440 tiles 370.4 and 368.
-inline bool narrow_tiles(long long tiles) { return tiles < 432; }
+// twice the workgroups of half the length, so where the tiles of 64 columns do
+// not deal out evenly over the 256 CUs the last round of workgroups is half as
+// long.  Where both need as many rounds, which is from one and a half to two
+// tiles a CU and from there on in ever narrower bands, those of 64 columns load
+// less.  Contraction and transitions of a step, 64 columns against 32, 320 areas:
+// 45 tiles 21.3 and 17.8 us, 270 tiles 56.8 and 54.5, 360 tiles 76.8 and 74.5,
+// 395 tiles 82.5 and 83.4, 430 tiles 89.2 and 90.5, 490 tiles 96.5 and 97.9, 510
+// tiles 99.7 and 101.2, 540 tiles 110.9 and 106.8, 720 tiles 138.7 and 137.8, 1080
+// tiles 211.5 and 208.0, 1440 tiles 280 and 278; 640 areas: 360 tiles 77.4 and
+// 72.4, 430 tiles 87.9 and 88.6, 480 tiles 95.9 and 96.6, 720 tiles 135.7 and 134.8.
+// (Beyond a million tiles there is nothing to choose, and twice the grid may pass
+// the dispatch's limit.)
+inline bool narrow_tiles(long long tiles) { return tiles <= 384 || (tiles > 512 && tiles <= (1 << 20)); }
 
 // The step-wise path's launches for n jobs of one context (A areas, G age
 // groups, Apad the padded area count of its D / I buffers, which hold

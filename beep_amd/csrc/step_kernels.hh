@@ -180,8 +180,7 @@ __device__ inline bool xcd_tile(int ntm, int ntn, int cols, int* tm, int* tn) {
 // interleaved with them would wait out one latency per row.  With NB = 1 they
 // are issued before the product too, whose loop hides their latency (three
 // dependent loads to a row's m(t)); with NB = 2 there are no registers for them:
-// they are capped for three wavefronts per SIMD, so that three workgroups per CU
-// hold the grid of 720 workgroups of a 9216-row product at once.
+// they are capped for three wavefronts per SIMD, three workgroups per CU.
 template <int NB>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) k_dense_contract(DenseMix p) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
