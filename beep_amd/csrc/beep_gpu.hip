@@ -152,7 +152,7 @@ namespace {
 constexpr int kMaxDevices = 64;
 
 // Streams over which mixed batches spread their size classes, one set per
-// device, made by the first batch and destroyed with the device's last
+// device, made as batches want them and destroyed with the device's last
 // context.  A launch of a batch is rarely wide enough to fill the device and
 // lasts as long as its longest instance, so what counts is how many launches
 // run at once: ordinary streams share a handful of hardware queues, whose
@@ -163,7 +163,15 @@ constexpr int kMaxDevices = 64;
 // each places its launches by what all of them have queued (BatchLease) and
 // joins on events of its own.  Twelve: a sweep over 1,120 unlike instances, whose
 // longest launch lasts 10.9 ms, takes 24.8 ms on 4 streams, 16.2 on 8, 12.7 on 12
-// and 12.3 on 16, and each costs 3.6 ms to make.
+// and 12.3 on 16.
+//
+// A masked stream takes 3.6 ms to make and 3.1 to destroy, and a program of a few
+// short batches would pay that for nothing (its first batch of 12 launches of 20
+// steps: 45-53 ms with them, 1.1 on four ordinary streams, which take 0.1 ms each;
+// closing its contexts: 48 and 9 ms).  So batches begin on ordinary streams, and
+// a masked one is made whenever batches that lacked it have lasted as long as it
+// costs (the sweep above: 30, 35, 34, 29 and 17 ms, then 12.7; 27 ms a pass on
+// ordinary streams).
 //
 // A masked stream is made without flags, so it is a blocking one: work on the
 // null stream waits for what the batch streams hold and keeps back what they are
@@ -171,13 +179,24 @@ constexpr int kMaxDevices = 64;
 // a non-blocking one).  The library itself queues nothing there: contexts use
 // their own stream, entry points without one side_stream.  A program's own
 // null-stream work does order with the batches under way.
-constexpr int kBatchStreams = 12;
+constexpr int kBatchStreams = 12;        // masked ones, at most
+constexpr int kPlainStreams = 4;         // ordinary ones: as many as hardware queues they share
+constexpr double kMaskedStreamMs = 6.7;
 struct BatchStreams {
-  std::vector<hipStream_t> st;
-  std::vector<double> load;        // cost of the launches placed and not yet joined
-  std::vector<int> queued;         // and their number
-  size_t wanted = 0;               // launches of the batches under way
-  int users = 0;                   // contexts of the device
+  struct Lane {
+    hipStream_t st;
+    double load = 0;                 // cost of the launches placed and not yet joined
+    int queued = 0;                  // and their number
+  };
+  std::vector<Lane> lane[2];         // ordinary, masked
+  size_t wanted = 0;                 // launches of the batches under way
+  double lacked = 0;                 // milliseconds of the batches that lacked masked streams
+  int users = 0;                     // contexts of the device
+  // Masked streams that the batches under way would use and do not have.
+  size_t missing() const {
+    const size_t use = std::min<size_t>(wanted, kBatchStreams);
+    return use - std::min(use, lane[1].size());
+  }
 };
 std::mutex g_bstream_mu;
 BatchStreams g_bstream[kMaxDevices];
@@ -1128,13 +1147,14 @@ int beep_destroy(beep_ctx* c) {
     std::lock_guard<std::mutex> lk(g_bstream_mu);
     BatchStreams& b = g_bstream[c->device];
     if (--b.users == 0) {
-      for (auto& st : b.st) {
-        (void)hipStreamSynchronize(st);
-        (void)hipStreamDestroy(st);
+      for (auto& v : b.lane) {
+        for (auto& l : v) {
+          (void)hipStreamSynchronize(l.st);
+          (void)hipStreamDestroy(l.st);
+        }
+        v.clear();
       }
-      b.st.clear();
-      b.load.clear();
-      b.queued.clear();
+      b.lacked = 0;
     }
   }
   if (c->bstart) (void)hipEventDestroy(c->bstart);
@@ -2321,34 +2341,45 @@ class BatchLease {
       for (int k : used_) (void)hipStreamSynchronize(stream(k));
     std::lock_guard<std::mutex> lk(g_bstream_mu);
     b_.wanted -= want_;
-    for (const auto& p : placed_) b_.load[p.first] = --b_.queued[p.first] == 0 ? 0.0 : b_.load[p.first] - p.second;
+    for (const auto& p : placed_) {
+      auto& l = b_.lane[masked_][p.first];
+      l.load = --l.queued == 0 ? 0.0 : l.load - p.second;
+    }
   }
 
-  // The batch's launches, `want` of them: streams for the launches of every
-  // batch under way, up to kBatchStreams (made as batches first want them: 3.6 ms
-  // each, and 3.1 to destroy).  The launches start after what c0's stream holds
-  // now, from where its timing event 0 is taken.
+  // The batch's launches, `want` of them.  Masked streams for the launches of
+  // every batch under way are made as far as earlier batches have lacked them for
+  // long enough; the batch takes the masked ones where they are enough or no fewer
+  // than the ordinary ones.
+  // The launches start after what c0's stream holds now, from where its timing
+  // event 0 is taken.
   int start(size_t want) {
     HIPCHK(c0_, hipSetDevice(c0_->device));
     {
       std::lock_guard<std::mutex> lk(g_bstream_mu);
       b_.wanted += want_ = want;
-      std::vector<uint32_t> mask;
-      while (b_.st.size() < std::min<size_t>(b_.wanted, kBatchStreams)) {
-        if (mask.empty()) {
-          hipDeviceProp_t prop;
-          HIPCHK(c0_, hipGetDeviceProperties(&prop, c0_->device));
-          mask.assign((prop.multiProcessorCount + 31) / 32, 0u);
-          for (int i = 0; i < prop.multiProcessorCount; i++) mask[i / 32] |= 1u << (i % 32);
+      const size_t n = std::min(b_.missing(), (size_t)(b_.lacked / kMaskedStreamMs));
+      if (n) {
+        b_.lacked -= kMaskedStreamMs * n;
+        hipDeviceProp_t prop;
+        HIPCHK(c0_, hipGetDeviceProperties(&prop, c0_->device));
+        std::vector<uint32_t> mask((prop.multiProcessorCount + 31) / 32, 0u);
+        for (int i = 0; i < prop.multiProcessorCount; i++) mask[i / 32] |= 1u << (i % 32);
+        for (size_t i = 0; i < n; i++) {
+          hipStream_t st = nullptr;
+          if (hipExtStreamCreateWithCUMask(&st, (uint32_t)mask.size(), mask.data()) != hipSuccess) {
+            (void)hipGetLastError();
+            HIPCHK(c0_, hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+          }
+          b_.lane[1].push_back({st});
         }
+      }
+      lacks_ = b_.missing() > 0;
+      masked_ = b_.lane[1].size() >= std::min<size_t>(b_.wanted, kPlainStreams);
+      while (!masked_ && b_.lane[0].size() < kPlainStreams) {
         hipStream_t st = nullptr;
-        if (hipExtStreamCreateWithCUMask(&st, (uint32_t)mask.size(), mask.data()) != hipSuccess) {
-          (void)hipGetLastError();
-          HIPCHK(c0_, hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-        }
-        b_.st.push_back(st);
-        b_.load.push_back(0.0);
-        b_.queued.push_back(0);
+        HIPCHK(c0_, hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+        b_.lane[0].push_back({st});
       }
     }
     if (!c0_->bstart) HIPCHK(c0_, hipEventCreateWithFlags(&c0_->bstart, hipEventDisableTiming));
@@ -2362,12 +2393,13 @@ class BatchLease {
     int k;
     {
       std::lock_guard<std::mutex> lk(g_bstream_mu);
-      k = (int)(std::min_element(b_.load.begin(), b_.load.end()) - b_.load.begin());
-      b_.load[k] += cost;
-      b_.queued[k]++;
+      auto& v = b_.lane[masked_];
+      k = (int)(std::min_element(v.begin(), v.end(), [](const auto& a, const auto& b) { return a.load < b.load; }) - v.begin());
+      v[k].load += cost;
+      v[k].queued++;
       placed_.emplace_back(k, cost);
+      *out = v[k].st;
     }
-    *out = stream(k);
     if (std::find(used_.begin(), used_.end(), k) != used_.end()) return BEEP_OK;
     HIPCHK(c0_, hipStreamWaitEvent(*out, c0_->bstart, 0));
     used_.push_back(k);
@@ -2389,14 +2421,22 @@ class BatchLease {
     return BEEP_OK;
   }
 
+  // The joined launches lasted `ms`.
+  void took(double ms) {
+    if (!lacks_ || !(ms > 0)) return;
+    std::lock_guard<std::mutex> lk(g_bstream_mu);
+    b_.lacked = std::min(b_.lacked + ms, kMaskedStreamMs * kBatchStreams);
+  }
+
  private:
   hipStream_t stream(int k) {
     std::lock_guard<std::mutex> lk(g_bstream_mu);      // another thread may be adding streams
-    return b_.st[k];
+    return b_.lane[masked_][k].st;
   }
   beep_ctx* c0_;
   BatchStreams& b_;
   size_t want_ = 0;
+  bool masked_ = false, lacks_ = false;
   std::vector<std::pair<int, double>> placed_;
   std::vector<int> used_;
   bool joined_ = false;
@@ -2801,6 +2841,7 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
     record(c0, 1);
     HIPCHK(c0, hipStreamSynchronize(c0->stream));   // `all` is the source of an async copy
     c0->timing[0] = autotune ? -1 : elapsed(c0, 0, 1);
+    lease.took(c0->timing[0]);
     c0->timing[3] = nlaunch;
   }
   HIPCHK(c0, hipStreamSynchronize(c0->stream));   // also keeps `all` alive until its copy is done
