@@ -2349,18 +2349,19 @@ class BatchLease {
 
   // The batch's launches, `want` of them.  Masked streams for the launches of
   // every batch under way are made as far as earlier batches have lacked them for
-  // long enough; the batch takes the masked ones where they are enough or no fewer
+  // long enough, all of them for an autotuning call, whose program has come to
+  // stay; the batch takes the masked ones where they are enough or no fewer
   // than the ordinary ones.
   // The launches start after what c0's stream holds now, from where its timing
   // event 0 is taken.
-  int start(size_t want) {
+  int start(size_t want, bool autotune) {
     HIPCHK(c0_, hipSetDevice(c0_->device));
     {
       std::lock_guard<std::mutex> lk(g_bstream_mu);
       b_.wanted += want_ = want;
-      const size_t n = std::min(b_.missing(), (size_t)(b_.lacked / kMaskedStreamMs));
+      const size_t n = autotune ? b_.missing() : std::min(b_.missing(), (size_t)(b_.lacked / kMaskedStreamMs));
       if (n) {
-        b_.lacked -= kMaskedStreamMs * n;
+        b_.lacked = std::max(0.0, b_.lacked - kMaskedStreamMs * n);
         hipDeviceProp_t prop;
         HIPCHK(c0_, hipGetDeviceProperties(&prop, c0_->device));
         std::vector<uint32_t> mask((prop.multiProcessorCount + 31) / 32, 0u);
@@ -2764,7 +2765,7 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
     // streams start to after they have all ended (timing[0]).
     const bool autotune = (flags & BEEP_BATCH_AUTOTUNE) != 0;
     BatchLease lease(c0);
-    if ((rc = lease.start(autotune ? 0 : launches.size()))) return rc;
+    if ((rc = lease.start(launches.size(), autotune))) return rc;
     // An autotuning call has the batch kernels to itself, so that the timed
     // candidates run alone; other batches run side by side.  The gate lets no
     // batch past a waiting autotuning call.
