@@ -2443,11 +2443,6 @@ class BatchLease {
   bool joined_ = false;
 };
 
-// ObservationModel::calculate (src/obsmodel.cc:22-109) of every item's
-// instance after a batch: per context one observation-kernel launch over its
-// items' instances, the launches spread over the batch streams, one upload of
-// the instance lists and one download of the sums.  Each instance's EF is
-// kept for the acceptance steps.
 // Observation log-likelihoods (ObservationModel::calculate, src/obsmodel.cc:
 // 22-35) of the instances inst[k][0..ninst[k]) of contexts ctxs[k], into out
 // (the contexts' results one after the other, in that order): each context's
@@ -2588,6 +2583,8 @@ int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const s
   return BEEP_OK;
 }
 
+// ObservationModel::calculate (src/obsmodel.cc:22-109) of every item's instance
+// after a batch, kept as its EF for the acceptance steps.
 int batch_loglik(beep_ctx* c0, int n, const beep_work* w, double* L_out) {
   std::vector<beep_ctx*> ctxs;
   std::map<beep_ctx*, std::vector<int>> items;
