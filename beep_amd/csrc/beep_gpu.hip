@@ -76,7 +76,8 @@ struct beep_ctx {
   // observations
   beepdev::ObsDev obs;
   beepdev::ObsDev* d_obs = nullptr;
-  std::vector<int> dt_ptr;          // per data table: its stored observations d_dt_obs[dt_ptr[d] .. dt_ptr[d+1])
+  std::vector<std::pair<int, int>> dt_first;   // data tables with observations, ascending, and the place of each one's
+                                    // first in d_dt_obs (stored observations, table by table)
   int* d_dt_obs = nullptr;          // null where the budget had no room for it
   std::vector<int> sec_ptr;
   int* d_sec_ptr = nullptr;
@@ -1105,13 +1106,11 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
     if ((rc = dalloc(c, (void**)&c->d_obs, sizeof(beepdev::ObsDev)))) return rc;
     HIPCHK(c, copy_on(c->stream, c->d_obs, &od, sizeof od, hipMemcpyHostToDevice));
     // Data tables and sections as lists of stored positions, ascending.
-    std::vector<int> dt_obs;
-    c->dt_ptr.assign(1, 0);
-    for (int d = 0; d < m.ndatatable; d++) {
-      for (int k = 0; k < nobs; k++)
-        if (dtab[k] == d) dt_obs.push_back(k);
-      c->dt_ptr.push_back((int)dt_obs.size());
-    }
+    std::vector<int> dt_obs(nobs);
+    for (int k = 0; k < nobs; k++) dt_obs[k] = k;
+    std::stable_sort(dt_obs.begin(), dt_obs.end(), [&](int a, int b) { return dtab[a] < dtab[b]; });
+    for (int k = 0; k < nobs; k++)
+      if (k == 0 || dtab[dt_obs[k]] != dtab[dt_obs[k - 1]]) c->dt_first.emplace_back(dtab[dt_obs[k]], k);
     std::vector<int> sptr(1, 0), sobs;
     for (const auto& l : m.section_obs) {
       std::vector<int> v;
@@ -2478,10 +2477,16 @@ int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const s
     range0[k] = range.size();
     tab0[k] = tab.size();
     su.ndt = out_dt ? c->m.ndatatable : 0;
+    size_t e = 0;
     for (int t = 0; t < (out_dt ? su.ndt : 1); t++) {
       tab.push_back((int)(range.size() - range0[k]));
-      const int k1 = out_dt ? c->dt_ptr[t + 1] : c->obs.nobs;
-      for (int x = out_dt ? c->dt_ptr[t] : 0; x < k1; x += BEEP_OBS_CHUNK)
+      int x = 0, k1 = c->obs.nobs;
+      if (out_dt) {
+        if (e == c->dt_first.size() || c->dt_first[e].first != t) continue;
+        x = c->dt_first[e++].second;
+        if (e < c->dt_first.size()) k1 = c->dt_first[e].second;
+      }
+      for (; x < k1; x += BEEP_OBS_CHUNK)
         range.push_back(make_int2(x, std::min(k1, x + BEEP_OBS_CHUNK)));
     }
     su.nchunk = (int)(range.size() - range0[k]);
@@ -2499,7 +2504,7 @@ int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const s
   if (N == 0) return BEEP_OK;
   if (out_dt)
     for (const beep_ctx* c : ctxs)
-      if (c->dt_ptr.back() > 0 && !c->d_dt_obs) return fail(c0, BEEP_ENOMEM, "no room for the data tables' lists");
+      if (!c->dt_first.empty() && !c->d_dt_obs) return fail(c0, BEEP_ENOMEM, "no room for the data tables' lists");
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t b_inst = al(N * sizeof(int32_t)), b_sets = al(nset * sizeof(ObsSet)), b_sums = al(nset * sizeof(ObsSum)),
                b_range = al(range.size() * sizeof(int2)), b_tab = al(tab.size() * sizeof(int));
