@@ -2582,9 +2582,14 @@ int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const s
                      (const ObsSum*)d_sums, (int)nset, (int)N, (const double*)d_part, d_out, d_out + N);
   HIPCHK(c0, hipGetLastError());
   if (ev0 >= 0) record(c0, ev0 + 1);
-  HIPCHK(c0, hipMemcpyAsync(out, d_out, N * sizeof(double), hipMemcpyDeviceToHost, st));
-  if (ND) HIPCHK(c0, hipMemcpyAsync(out_dt, d_out + N, ND * sizeof(double), hipMemcpyDeviceToHost, st));
+  // The tables' sums lie behind the totals: one download for both.
+  std::vector<double> both(ND ? N + ND : 0);
+  HIPCHK(c0, hipMemcpyAsync(ND ? both.data() : out, d_out, (N + ND) * sizeof(double), hipMemcpyDeviceToHost, st));
   HIPCHK(c0, hipStreamSynchronize(st));
+  if (ND) {
+    std::copy(both.begin(), both.begin() + N, out);
+    std::copy(both.begin() + N, both.end(), out_dt);
+  }
   return BEEP_OK;
 }
 
