@@ -1738,13 +1738,17 @@ namespace {
 // device trajectory `dev` ([s][x][area * group]) and host memory `host`
 // ([s][area][x][group]): slabs of steps are reordered by a kernel next to their
 // copy.  A slab is at most 16 MiB of staging, or whole steps of what the context
-// already holds; without room for one step, and for up to 4096 values (8 us of
-// host loop, about a kernel launch), the host does the reordering.
+// already holds; without room for one step, and where the values come in up to
+// 8,192 runs of one area's groups (and to 65,536 values), the host does the
+// reordering: its loop costs by the run, the kernel 13 us a call.  Read back by the
+// host and by the device: 12,000 values of one group 32 and 26 us, 7,200 of one 34
+// and 36, 12,000 of four 17 and 26, 33,000 of four 30 and 30, 48,000 of four 39 and
+// 33, 48,600 of nine 30 and 33, 64,800 of nine 36 and 36.
 int move_trajectory(beep_ctx* c, int* dev, int* host, int S, int X, bool to_host) {
   const auto& m = c->m;
   const size_t row = (size_t)X * m.AG, total = (size_t)S * row;
   size_t steps = std::min<size_t>((size_t)S, std::max<size_t>(1, ((size_t)16 << 20) / (row * sizeof(int))));
-  if (total <= 4096) steps = 0;
+  if (total / m.G <= 8192 && total <= 65536) steps = 0;
   else if (!try_scratch(c, steps * row * sizeof(int))) steps = c->scratch_cap / (row * sizeof(int));
   if (steps == 0) {
     std::vector<int> h(total);
@@ -1752,15 +1756,19 @@ int move_trajectory(beep_ctx* c, int* dev, int* host, int S, int X, bool to_host
       HIPCHK(c, hipMemcpyAsync(h.data(), dev, total * sizeof(int), hipMemcpyDeviceToHost, c->stream));
       HIPCHK(c, hipStreamSynchronize(c->stream));
     }
-    for (int s = 0; s < S; s++)
-      for (int a = 0; a < m.A; a++)
-        for (int x = 0; x < X; x++)
-          for (int g = 0; g < m.G; g++) {
-            int& o = host[(((size_t)s * m.A + a) * X + x) * m.G + g];
-            int& i = h[((size_t)s * X + x) * m.AG + a * m.G + g];
-            if (to_host) o = i;
-            else i = o;
+    const int A = m.A, G = m.G;
+    int* hd = h.data();
+    auto runs = [&](auto move) {       // (device order, host order)
+      for (int s = 0; s < S; s++)
+        for (int a = 0; a < A; a++)
+          for (int x = 0; x < X; x++) {
+            int* d = hd + ((size_t)s * X + x) * A * G + (size_t)a * G;
+            int* o = host + (((size_t)s * A + a) * X + x) * G;
+            for (int g = 0; g < G; g++) move(d[g], o[g]);
           }
+    };
+    if (to_host) runs([](int& d, int& o) { o = d; });
+    else runs([](int& d, int& o) { d = o; });
     if (!to_host) {
       HIPCHK(c, hipMemcpyAsync(dev, h.data(), total * sizeof(int), hipMemcpyHostToDevice, c->stream));
       HIPCHK(c, hipStreamSynchronize(c->stream));
