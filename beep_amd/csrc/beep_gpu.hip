@@ -1659,13 +1659,14 @@ int beep_pois_loglik(beep_ctx* c, int n, const int32_t* inst, double* L_out) {
   if (n == 0) return BEEP_OK;
   int rc;
   // Instances on the grid's y: at most 65535 of them a launch, fewer where the
-  // chunk sums of so many do not fit, and without room for those of one instance
-  // one workgroup goes over all its chunks and writes the result.
+  // chunk sums of so many do not fit, and without room for those of one instance,
+  // or where there is only one chunk, one workgroup goes over all its chunks and
+  // writes the result.
   size_t nchunk = (c->traj_sz + BEEP_POIS_CHUNK - 1) / BEEP_POIS_CHUNK;
   size_t nb = (size_t)std::min(n, 65535);
   auto bytes = [&] { return (size_t)n * (sizeof(double) + sizeof(int)) + nb * nchunk * sizeof(double); };
-  while (nb > 1 && !try_scratch(c, bytes())) nb /= 2;
-  const bool direct = !try_scratch(c, bytes());
+  while (nchunk > 1 && nb > 1 && !try_scratch(c, bytes())) nb /= 2;
+  const bool direct = nchunk == 1 || !try_scratch(c, bytes());
   if (direct) {
     nchunk = 1;
     nb = 0;
