@@ -78,7 +78,7 @@ struct beep_ctx {
   beepdev::ObsDev* d_obs = nullptr;
   std::vector<std::pair<int, int>> dt_first;   // data tables with observations, ascending, and the place of each one's
                                     // first in d_dt_obs (stored observations, table by table)
-  int* d_dt_obs = nullptr;          // null where the budget had no room for it
+  int* d_dt_obs = nullptr;          // null for one table, or where the budget had no room for it
   std::vector<int> sec_ptr;
   int* d_sec_ptr = nullptr;
   int* d_sec_obs = nullptr;
@@ -1109,7 +1109,8 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
     // Data tables and sections as lists of stored positions, ascending.
     std::vector<int> dt_obs(nobs);
     for (int k = 0; k < nobs; k++) dt_obs[k] = k;
-    std::stable_sort(dt_obs.begin(), dt_obs.end(), [&](int a, int b) { return dtab[a] < dtab[b]; });
+    auto before = [&](int a, int b) { return dtab[a] < dtab[b]; };
+    if (!std::is_sorted(dt_obs.begin(), dt_obs.end(), before)) std::stable_sort(dt_obs.begin(), dt_obs.end(), before);
     for (int k = 0; k < nobs; k++)
       if (k == 0 || dtab[dt_obs[k]] != dtab[dt_obs[k - 1]]) c->dt_first.emplace_back(dtab[dt_obs[k]], k);
     std::vector<int> sptr(1, 0), sobs;
@@ -1125,8 +1126,9 @@ int beep_create(const beep_spec* spec, int device, size_t hbm_budget, int capaci
         (rc = upload(c, &c->d_sec_ti, m.section_ti)) || (rc = upload(c, &c->d_sec_tf, m.section_tf)))
       return rc;
     // The tables' lists last, where the budget has room for them: without them
-    // sums per table take every observation for each (k_obs_loglik).
-    if (!dt_obs.empty()) {
+    // sums per table take every observation for each (k_obs_loglik).  One table
+    // holds all observations in stored order.
+    if (c->dt_first.size() > 1) {
       const std::string err = c->err;
       if ((rc = upload(c, &c->d_dt_obs, dt_obs)) && rc != BEEP_ENOMEM) return rc;
       c->err = err;
@@ -2514,7 +2516,7 @@ int obs_loglik_chunked(beep_ctx* c0, const std::vector<beep_ctx*>& ctxs, const s
   if (N == 0) return BEEP_OK;
   if (out_dt)
     for (const beep_ctx* c : ctxs)
-      if (!c->dt_first.empty() && !c->d_dt_obs) return fail(c0, BEEP_ENOMEM, "no room for the data tables' lists");
+      if (c->dt_first.size() > 1 && !c->d_dt_obs) return fail(c0, BEEP_ENOMEM, "no room for the data tables' lists");
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t b_inst = al(N * sizeof(int32_t)), b_sets = al(nset * sizeof(ObsSet)), b_sums = al(nset * sizeof(ObsSum)),
                b_range = al(range.size() * sizeof(int2)), b_tab = al(tab.size() * sizeof(int));
