@@ -1,6 +1,7 @@
 """A batch's streams: the first batch of a device's first context is no slower
 than later ones by streams that it does not pay for, and batches give the same
 on ordinary streams, on masked ones and while those are being made."""
+import threading
 import time
 
 import numpy as np
@@ -47,5 +48,35 @@ def test_batches_give_the_same_as_streams_are_made(gpu_lib):
         _batch(ctxs)
         for c, w in zip(ctxs, want):
             assert np.array_equal(c.get_transnum(0), w)
+    for c in ctxs:
+        c.close()
+
+
+def test_threads_while_streams_are_made(gpu_lib):
+    """Three threads' batches of four launches, some 3 ms each, from no streams
+    to masked ones, with contexts made and closed beside them."""
+    ctxs = _contexts(400)
+    want = [c.get_transnum(2) for c in ctxs]
+    small, truth = configs.seir_areas(3, 1, 10, seed=2)
+    wrong = []
+
+    def work(k):
+        mine = ctxs[4 * k: 4 * k + 4]
+        items = [(c, _lib.WORK_SIMULATE, 0, 0, 0, 5 + 4 * k + i, 0, c.S) for i, c in enumerate(mine)]
+        for _ in range(15):
+            _lib.run_batch(items, seed=3)
+            extra = _lib.Context(small, capacity=1, nslot=1)
+            for c, w in zip(mine, want[4 * k:]):
+                if not np.array_equal(c.get_transnum(0), w):
+                    wrong.append(k)
+            extra.close()
+
+    th = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join(timeout=90)
+        assert not t.is_alive()
+    assert not wrong
     for c in ctxs:
         c.close()
