@@ -119,7 +119,7 @@ struct beep_ctx {
   SpecKernels* spec = nullptr;
   size_t spec_lds = 0;
   // The events a mixed batch launched from this context starts the device's
-  // batch streams from and joins them with (created on first use).
+  // batch streams from and waits for them with (created on first use).
   hipEvent_t bstart = nullptr;
   std::vector<hipEvent_t> bend;    // end of each batch stream's work
   bool counted = false;            // holds a share of the device's batch streams
@@ -162,7 +162,7 @@ constexpr int kMaxDevices = 64;
 // workgroups each: 22.8 ms on 16 ordinary streams, 5.7 ms on 16 masked ones,
 // 6.1 ms for one launch).  Batches of several host threads share the streams:
 // each places its launches by what all of them have queued (BatchLease) and
-// joins on events of its own.  Twelve: a sweep over 1,120 unlike instances, whose
+// waits on events of its own.  Twelve: a sweep over 1,120 unlike instances, whose
 // longest launch lasts 10.9 ms, takes 24.8 ms on 4 streams, 16.2 on 8, 12.7 on 12
 // and 12.3 on 16.
 //
@@ -2418,26 +2418,29 @@ class BatchLease {
     return BEEP_OK;
   }
 
-  // c0's stream goes on after everything placed.
-  int join() {
+  // Waits for everything placed; ms: from c0's timing event 0 to its end.  The
+  // host waits, not c0's stream: a wait queued there would hold up every stream
+  // that shares its hardware queue, other contexts' among them, for as long as
+  // the batch runs (one in eight contexts' calls beside a batch of 27 ms took 21).
+  int join(double* ms) {
     while (c0_->bend.size() < used_.size()) {
       hipEvent_t e = nullptr;
-      HIPCHK(c0_, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      HIPCHK(c0_, hipEventCreate(&e));
       c0_->bend.push_back(e);
     }
+    for (size_t i = 0; i < used_.size(); i++) HIPCHK(c0_, hipEventRecord(c0_->bend[i], stream(used_[i])));
+    *ms = 0;
     for (size_t i = 0; i < used_.size(); i++) {
-      HIPCHK(c0_, hipEventRecord(c0_->bend[i], stream(used_[i])));
-      HIPCHK(c0_, hipStreamWaitEvent(c0_->stream, c0_->bend[i], 0));
+      HIPCHK(c0_, hipEventSynchronize(c0_->bend[i]));
+      float t = 0;
+      HIPCHK(c0_, hipEventElapsedTime(&t, c0_->ev[0], c0_->bend[i]));
+      *ms = std::max(*ms, (double)t);
     }
     joined_ = true;
-    return BEEP_OK;
-  }
-
-  // The joined launches lasted `ms`.
-  void took(double ms) {
-    if (!lacks_ || !(ms > 0)) return;
+    if (!lacks_) return BEEP_OK;
     std::lock_guard<std::mutex> lk(g_bstream_mu);
-    b_.lacked = std::min(b_.lacked + ms, kMaskedStreamMs * kBatchStreams);
+    b_.lacked = std::min(b_.lacked + *ms, kMaskedStreamMs * kBatchStreams);
+    return BEEP_OK;
   }
 
  private:
@@ -2780,8 +2783,8 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
     // instances of one launch overlap the next launch instead of leaving the
     // device idle; each stream starts after the job upload.  (Autotuning
     // launches run alone on the context stream to be timed.)
-    // The fused phase is timed on the context stream from before the batch
-    // streams start to after they have all ended (timing[0]).
+    // The fused phase is timed from before the batch streams start, on the
+    // context stream, to the end of the last of them (timing[0]).
     const bool autotune = (flags & BEEP_BATCH_AUTOTUNE) != 0;
     BatchLease lease(c0);
     if ((rc = lease.start(launches.size(), autotune))) return rc;
@@ -2855,13 +2858,10 @@ int beep_run_batch(int n, const beep_work* w, uint64_t seed, uint32_t stream, in
       nlaunch++;
     }
     if (tuned_any) tune_save();
-    // Join: the context stream waits for every batch stream used, then records
-    // the end of the fused phase.
-    if ((rc = lease.join())) return rc;
-    record(c0, 1);
+    double ms = 0;
+    if ((rc = lease.join(&ms))) return rc;
     HIPCHK(c0, hipStreamSynchronize(c0->stream));   // `all` is the source of an async copy
-    c0->timing[0] = autotune ? -1 : elapsed(c0, 0, 1);
-    lease.took(c0->timing[0]);
+    c0->timing[0] = autotune ? -1 : ms;
     c0->timing[3] = nlaunch;
   }
   HIPCHK(c0, hipStreamSynchronize(c0->stream));   // also keeps `all` alive until its copy is done

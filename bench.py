@@ -282,8 +282,8 @@ def bench_uneven(args):
         "roofline": {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": None,
                      "algorithmic_bytes_per_sweep": algo_bytes,
-                     "note": "fused phase of the batch (size-class launches over the batch streams) timed with HIP events on "
-                             "the context stream from the streams' start to their join; traffic counters in profiles/"},
+                     "note": "fused phase of the batch (size-class launches over the batch streams) timed with HIP events "
+                             "from the streams' start to the end of the last; traffic counters in profiles/"},
         "mc3": {"accepted_per_sweep": float(np.mean([r["accepted"] for r in sweeps])),
                 "swaps_per_sweep": float(np.mean([r["swaps"] for r in sweeps]))},
     }
